@@ -157,25 +157,37 @@ __device__ __forceinline__ void gather(const LevelArgs<T> &L, const T *__restric
 __device__ __forceinline__ double sor_div(double a, double d) { return a / d; }
 __device__ __forceinline__ float sor_div(float a, float d) { return a * __builtin_amdgcn_rcpf(d); }
 
+// the divisor in the form sor_quot_inv takes (FP32: its reciprocal), for a
+// loop that divides by it again and again: sor_quot_inv(a, sor_inv(d)) is
+// sor_div(a, d)
+__device__ __forceinline__ double sor_inv(double d) { return d; }
+__device__ __forceinline__ float sor_inv(float d) { return __builtin_amdgcn_rcpf(d); }
+__device__ __forceinline__ double sor_quot_inv(double a, double d) { return a / d; }
+__device__ __forceinline__ float sor_quot_inv(float a, float r) { return a * r; }
+
 // RB-SOR point update (poisson_d3.cc:109-116, poisson_d2.cc:103-108):
-// (1 - w) x + sor_quot, the quotient from the neighbours alone
+// (1 - w) x + sor_quot, the quotient sor_num / sor_den from the neighbours alone
 template <typename T, int DIM>
-__device__ __forceinline__ T sor_quot(const Stencil<T, DIM> &s, T c2x, T c1x, T c2y, T c1y, T c2z, T c1z, T b,
-                                      T w) {
+__device__ __forceinline__ T sor_num(const Stencil<T, DIM> &s, T c2x, T c1x, T c2y, T c1y, T c2z, T c1z, T b, T w) {
     T sum = c2x * (s.xE + s.xW) + c1x * (s.xE - s.xW);
-    T den;
     if (DIM == 3) {
         sum = sum + c2y * (s.yN + s.yS);
         sum = sum + c1y * (s.yN - s.yS);
-        sum = sum + c2z * (s.zT + s.zB);
-        sum = sum + c1z * (s.zT - s.zB);
-        den = T(2.0) * ((c2x + c2y) + c2z);
-    } else {
-        sum = sum + c2z * (s.zT + s.zB);
-        sum = sum + c1z * (s.zT - s.zB);
-        den = T(2.0) * (c2x + c2z);
     }
-    return sor_div((sum - b) * w, den);
+    sum = sum + c2z * (s.zT + s.zB);
+    sum = sum + c1z * (s.zT - s.zB);
+    return (sum - b) * w;
+}
+
+template <typename T, int DIM>
+__device__ __forceinline__ T sor_den(T c2x, T c2y, T c2z) {
+    return DIM == 3 ? T(2.0) * ((c2x + c2y) + c2z) : T(2.0) * (c2x + c2z);
+}
+
+template <typename T, int DIM>
+__device__ __forceinline__ T sor_quot(const Stencil<T, DIM> &s, T c2x, T c1x, T c2y, T c1y, T c2z, T c1z, T b,
+                                      T w) {
+    return sor_div(sor_num<T, DIM>(s, c2x, c1x, c2y, c1y, c2z, c1z, b, w), sor_den<T, DIM>(c2x, c2y, c2z));
 }
 
 template <typename T, int DIM>

@@ -45,12 +45,11 @@ void set_error(const std::string &s) { g_last_error = s; }
     } while (0)
 
 constexpr int kThreads = 256;
-// default dynamic LDS budget of the single-workgroup tail (SARAS_TAIL_LDS_KB
-// overrides it, up to 150 KB of the 160 KB a workgroup may hold: the tail's
-// static LDS is under 2 KB); the tail also takes only levels its threads
-// cover with a cell each or with colour lists (see tail_first_level)
-constexpr size_t kTailLdsDefault = 128 * 1024;
-constexpr int kTailThreads = 512;
+// default dynamic LDS budget of the single-workgroup tail, of the 160 KB a
+// workgroup may hold (SARAS_TAIL_LDS_KB lowers it; the tail's static LDS is
+// under 1 KB); above the coarsest level the tail also takes only levels whose
+// cells its threads keep in registers (see tail_layout)
+constexpr size_t kTailLdsDefault = 150 * 1024;
 
 inline unsigned blocks_for(long n) { return (unsigned)std::max<long>(1, (n + kThreads - 1) / kThreads); }
 
@@ -93,11 +92,13 @@ struct Hierarchy {
     // host copies of the metric coefficients (c2, c1) and restriction
     // factors (lo, hi, wd) per level and axis, for the tail's packed image
     std::vector<std::array<std::vector<double>, 3>> hc2, hc1, hlo, hhi, hwd;
-    // the tail kernel's coefficient region of LDS for tail levels
-    // tail_first..D, packed in its order (see k_tail)
-    T *tail_coef = nullptr;
+    // the tail kernel's levels tail_first..D (D + 1: no tail), its arguments
+    // and LDS size, and the packed images of its coefficients and cell tables
     int tail_first = -1;
-    size_t tail_coef_n = 0;
+    saras::TailArgs<T> tail_args{};
+    size_t tail_bytes = 0;
+    T *tail_coef = nullptr;
+    unsigned *tail_cells = nullptr;
 
     // a level takes split rows when each half-row is a whole number of 16-byte vectors
     static bool splittable(int nz) {
@@ -117,34 +118,7 @@ struct Hierarchy {
         for (int a = 0; a < 3; ++a) (void)hipFree(wall[a]);
         (void)hipFree(coarse_scratch);
         (void)hipFree(tail_coef);
-    }
-
-    // The tail's coefficient image for levels S..D: per level and axis c2
-    // then c1 (one zero each for the planar y axis), then for levels S+1..D
-    // of a 3-D hierarchy per axis the restriction factors lo, hi, wd.
-    saras_status pack_tail(int S) {
-        const int D = (int)lv.size() - 1;
-        if (S > D) return SARAS_OK;
-        std::vector<double> flat;
-        for (int l = S; l <= D; ++l)
-            for (int a = 0; a < 3; ++a) {
-                flat.insert(flat.end(), hc2[l][a].begin(), hc2[l][a].end());
-                flat.insert(flat.end(), hc1[l][a].begin(), hc1[l][a].end());
-            }
-        if (dim == 3)
-            for (int l = S + 1; l <= D; ++l)
-                for (int a = 0; a < 3; ++a) {
-                    flat.insert(flat.end(), hlo[l][a].begin(), hlo[l][a].end());
-                    flat.insert(flat.end(), hhi[l][a].begin(), hhi[l][a].end());
-                    flat.insert(flat.end(), hwd[l][a].begin(), hwd[l][a].end());
-                }
-        (void)hipFree(tail_coef);
-        tail_coef = nullptr;
-        saras_status st = upload(&tail_coef, flat);
-        if (st) return st;
-        tail_first = S;
-        tail_coef_n = flat.size();
-        return SARAS_OK;
+        (void)hipFree(tail_cells);
     }
 
     saras_status build(const saras::GridLevels &G, const std::vector<std::vector<double>> &walls) {
@@ -345,33 +319,158 @@ saras::LevelArgs<T> level_args(const saras_mg *m, const Hierarchy<T> &H, int l, 
     return a;
 }
 
-// first level of the single-workgroup tail: the smallest S whose levels S..D
-// fit in the tail's LDS budget (D + 1, i.e. no tail, when even the coarsest
-// level does not fit)
+// The tail's LDS layout for levels S..D (the offsets of A.L) and its bytes;
+// 0 where the levels do not fit or the tail does not take them.
 template <typename T>
-int tail_first_level(const saras_mg *m, const Hierarchy<T> &H) {
+size_t tail_layout(const saras_mg *m, const Hierarchy<T> &H, int S, saras::TailArgs<T> &A) {
     const int D = (int)H.lv.size() - 1;
-    size_t bytes = 0;
-    int S = D + 1;
-    for (int l = D; l >= 0; --l) {
+    if (D - S + 1 > saras::kTailMaxLevels) return 0;
+    auto up4 = [](size_t n) { return (n + 3) / 4 * 4; };
+    A = saras::TailArgs<T>{};
+    A.first = S;
+    A.last = D;
+    size_t off = 0, ncoef = 0, ncell = 0;
+    for (int l = S; l <= D; ++l) {
         const DevLevel<T> &L = H.lv[l];
-        const size_t core = (size_t)L.n[0] * L.n[1] * L.n[2];
-        const size_t pad = H.dim == 3 ? (size_t)(L.n[0] + 2) * (L.n[1] + 2) * (L.n[2] + 2)
-                                      : (size_t)(L.n[0] + 2) * (L.n[2] + 2);
-        // metric coefficients (2 per index) and restriction factors (3)
-        const size_t coef = 5 * ((size_t)L.n[0] + L.n[1] + L.n[2]);
-        bytes += ((pad + 3) / 4 * 4 + (core + 3) / 4 * 4 + coef) * sizeof(T);
-        if (bytes > m->tail_lds || D - l + 1 > saras::kTailMaxLevels) break;
-        // a cell per thread, or colour lists (even z extent, at most
-        // kTailColourCells cells of a colour per thread); larger levels
-        // would walk every cell in each colour pass and run faster as
-        // multi-workgroup passes
-        const bool one = core <= (size_t)kTailThreads;
-        const bool lists = L.n[2] % 2 == 0 && core / 2 <= (size_t)saras::kTailColourCells * kTailThreads;
-        if (l < D && !one && !lists) break;
-        S = l;
+        saras::TailLevel &V = A.L[l - S];
+        for (int a = 0; a < 3; ++a) V.n[a] = L.n[a];
+        const int ny = H.dim == 3 ? L.n[1] : 1;
+        V.hz = (L.n[2] + 1) / 2;
+        const size_t half = (size_t)L.n[0] * ny * V.hz;
+        if (2 * half > 65535) return 0;   // a cell's LDS offset takes 16 bits
+        V.half = (int)half;
+        for (int a = 0; a < 3; ++a) {
+            if (H.dim == 2 && a == 1) continue;
+            const int lo = bc_code(m->p, m->g, a, l, false, false), hi = bc_code(m->p, m->g, a, l, false, true);
+            V.neg |= lo == saras::BC_DIR || hi == saras::BC_DIR;
+            V.odd |= lo == saras::BC_PER && (L.n[a] & 1);
+        }
+        const size_t reg = (size_t)saras::kTailColourCells * saras::kTailThreads;
+        // levels above the coarsest: the cells that the threads keep in
+        // registers; larger ones run faster as multi-workgroup passes
+        if (l < D && (half > reg || V.odd)) return 0;
+        // inhomogeneous walls (the finest level of the reference's test
+        // problem) are left to the multi-workgroup kernels
+        if (l == 0 && m->p.bc == SARAS_BC_DIRICHLET_TEST) return 0;
+        V.x = (int)off;
+        off += up4(2 * half);
+        V.b = (int)off;
+        off += up4(2 * half);
+        V.old = (int)off;
+        if (l == D && (m->p.solve_flag || (V.odd && half > reg))) off += up4(2 * half);
+        ncoef += 2 * ((size_t)L.n[0] + ny + L.n[2]);
+        if (H.dim == 3 && l > S) ncoef += 3 * ((size_t)L.n[0] + ny + L.n[2]);
+        // cell tables of levels with at most one cell of a colour per thread
+        V.cell1 = half <= (size_t)saras::kTailThreads ? 0 : -1;
+        if (V.cell1 >= 0) ncell += 2 * up4(2 * half) * 5 / 2;
     }
-    return S;
+    A.res = (int)off;
+    if (S < D) off += up4(2 * (size_t)A.L[0].half);
+    A.coff = (int)off;
+    A.ncoef = (int)ncoef;
+    off += up4(ncoef);
+    const size_t words = sizeof(T) / 4;
+    size_t w = off * words;
+    A.cellw = (int)w;
+    A.ncellw = (int)ncell;
+    for (int l = S; l <= D; ++l) {
+        saras::TailLevel &V = A.L[l - S];
+        if (V.cell1 < 0) continue;
+        const size_t n = up4(2 * (size_t)V.half);
+        V.cell4 = (int)w;
+        V.cell1 = (int)(w + 4 * n);
+        w += 5 * n;
+    }
+    const size_t bytes = w * 4;
+    return bytes <= m->tail_lds && w / words < 65536 ? bytes : 0;
+}
+
+// The tail of a hierarchy: the levels from the finest one that fits its LDS
+// budget to the coarsest (none when even that does not fit), with the images
+// the kernel copies to LDS -- the coefficients as pairs (c2, c1) per level and
+// axis (a pair of zeros for the planar y axis), the restriction factors lo,
+// hi, wd of levels S+1..D of a 3-D hierarchy, and the cell tables.
+template <typename T>
+saras_status pack_tail(const saras_mg *m, Hierarchy<T> &H) {
+    const int D = (int)H.lv.size() - 1;
+    H.tail_first = D + 1;
+    for (int S = D; S >= 0; --S) {
+        saras::TailArgs<T> A;
+        const size_t bytes = tail_layout(m, H, S, A);
+        if (!bytes) break;
+        H.tail_first = S;
+        H.tail_args = A;
+        H.tail_bytes = bytes;
+    }
+    const int S = H.tail_first;
+    if (S > D) return SARAS_OK;
+    saras::TailArgs<T> &A = H.tail_args;
+    std::vector<double> flat;
+    int coff[saras::kTailMaxLevels][3];
+    for (int l = S; l <= D; ++l)
+        for (int a = 0; a < 3; ++a) {
+            coff[l - S][a] = A.coff + (int)flat.size();
+            for (size_t q = 0; q < H.hc2[l][a].size(); ++q) {
+                flat.push_back(H.hc2[l][a][q]);
+                flat.push_back(H.hc1[l][a][q]);
+            }
+        }
+    if (H.dim == 3)
+        for (int l = S + 1; l <= D; ++l)
+            for (int a = 0; a < 3; ++a) {
+                saras::TailLevel &V = A.L[l - S];
+                V.lo[a] = A.coff + (int)flat.size();
+                flat.insert(flat.end(), H.hlo[l][a].begin(), H.hlo[l][a].end());
+                V.hi[a] = A.coff + (int)flat.size();
+                flat.insert(flat.end(), H.hhi[l][a].begin(), H.hhi[l][a].end());
+                V.wd[a] = A.coff + (int)flat.size();
+                flat.insert(flat.end(), H.hwd[l][a].begin(), H.hwd[l][a].end());
+            }
+    // host-side guard: the kernel copies ncoef elements
+    if ((int)flat.size() != A.ncoef) {
+        set_error("internal error: tail coefficients do not match their layout");
+        return SARAS_HIP_ERROR;
+    }
+    saras_status st = upload(&H.tail_coef, flat);
+    if (st) return st;
+    // the LDS image of the cell tables, then the tables of larger levels
+    std::vector<unsigned> img((size_t)A.ncellw, 0u);
+    size_t gn = 0;   // entries of the tables in global memory
+    for (int l = S; l <= D; ++l) {
+        saras::TailLevel &V = A.L[l - S];
+        if (V.cell1 >= 0) continue;
+        V.cell4 = (int)gn;
+        gn += (2 * (size_t)V.half + 3) / 4 * 4;
+    }
+    const size_t nimg = img.size();
+    img.resize(nimg + 5 * gn, 0u);
+    for (int l = S; l <= D; ++l) {
+        const saras::TailLevel &V = A.L[l - S];
+        int lo[3], hi[3];
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = bc_code(m->p, m->g, a, l, false, false);
+            hi[a] = bc_code(m->p, m->g, a, l, false, true);
+        }
+        std::vector<saras::TailCell> t(2 * (size_t)V.half);
+        if (H.dim == 3) saras::tail_cells<3>(V, coff[l - S], lo, hi, t.data());
+        else saras::tail_cells<2>(V, coff[l - S], lo, hi, t.data());
+        unsigned *w4 = V.cell1 >= 0 ? img.data() + (V.cell4 - A.cellw) : img.data() + nimg + 4 * V.cell4;
+        unsigned *w1 = V.cell1 >= 0 ? img.data() + (V.cell1 - A.cellw) : img.data() + nimg + 4 * gn + V.cell4;
+        for (size_t q = 0; q < t.size(); ++q) {
+            w4[4 * q] = t[q].a[0];
+            w4[4 * q + 1] = t[q].a[1];
+            w4[4 * q + 2] = t[q].a[2];
+            w4[4 * q + 3] = t[q].cxy;
+            w1[q] = t[q].czf;
+        }
+    }
+    HIP_TRY(hipMalloc((void **)&H.tail_cells, std::max<size_t>(4, img.size()) * sizeof(unsigned)));
+    HIP_TRY(hipMemcpy(H.tail_cells, img.data(), img.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+    A.coef = H.tail_coef;
+    A.cellimg = H.tail_cells;
+    A.cells4 = reinterpret_cast<const uint4 *>(H.tail_cells + nimg);
+    A.cells1 = H.tail_cells + nimg + 4 * gn;
+    return SARAS_OK;
 }
 
 // Level operations for one precision.  `inhom0` selects the inhomogeneous
@@ -673,38 +772,21 @@ struct Ops {
                            F.n[2], F.sx, F.sy, F.hz, F.x, C.x, C.sx, C.sy, C.hz);
     }
 
-    int tail_start() const { return tail_first_level(m, H); }
+    int tail_start() const { return H.tail_first; }
 
     void tail(int S) {
         const int D = (int)H.lv.size() - 1;
-        saras::TailArgs<T> A{};
-        A.first = S;
-        A.last = D;
-        size_t off = 0;
-        for (int l = S; l <= D; ++l) {
-            const DevLevel<T> &L = H.lv[l];
-            A.L[l - S] = level_args(m, H, l, inhom(l, false));
-            for (int q = 0; q < 3; ++q) {
-                A.R[l - S].lo[q] = L.rlo[q];
-                A.R[l - S].hi[q] = L.rhi[q];
-                A.R[l - S].wd[q] = L.rwd[q];
-            }
-            const size_t core = (size_t)L.n[0] * L.n[1] * L.n[2];
-            const size_t pad = H.dim == 3 ? (size_t)(L.n[0] + 2) * (L.n[1] + 2) * (L.n[2] + 2)
-                                          : (size_t)(L.n[0] + 2) * (L.n[2] + 2);
-            A.xoff[l - S] = (int)off;
-            off += (pad + 3) / 4 * 4;
-            A.boff[l - S] = (int)off;
-            off += (core + 3) / 4 * 4;
+        // host-side guard: the tail packed for this hierarchy
+        if (S != H.tail_first || S > D || H.tail_bytes > m->tail_lds) {
+            refuse("tail levels not packed");
+            return;
         }
-        A.coff = (int)off;
-        for (int l = S; l <= D; ++l) {
-            const DevLevel<T> &L = H.lv[l];
-            off += 2 * ((size_t)L.n[0] + (H.dim == 3 ? L.n[1] : 1) + L.n[2]);
-            if (H.dim == 3 && l > S) off += 3 * ((size_t)L.n[0] + L.n[1] + L.n[2]);   // restriction factors
-        }
+        saras::TailArgs<T> A = H.tail_args;
         A.x = H.lv[S].x;
         A.b = H.lv[S].b;
+        A.sx = H.lv[S].sx;
+        A.sy = H.lv[S].sy;
+        A.hz = H.lv[S].hz;
         A.pre = m->p.pre_smooth;
         A.post = m->p.post_smooth;
         A.solve_flag = m->p.solve_flag;
@@ -712,28 +794,11 @@ struct Ops {
         A.w = w;
         A.tol = m->p.mg_tol;
         A.rel_floor = coarse_rel_floor();
-        A.zero_bc_first = S != 0;
         A.iters_out = m->iters_host;
-        size_t ncoef = 0;
-        for (int l = S; l <= D; ++l)
-            for (int q = 0; q < 3; ++q) {
-                ncoef += 2 * (size_t)(H.dim == 2 && q == 1 ? 1 : H.lv[l].n[q]);
-                if (H.dim == 3 && l > S) ncoef += 3 * (size_t)H.lv[l].n[q];
-            }
-        if (H.tail_first != S || !H.tail_coef || H.tail_coef_n != ncoef) {
-            refuse("tail coefficients not packed for this tail");
-            return;
-        }
-        A.coef = H.tail_coef;
-        // host-side guard: tail_start() keeps the levels within tail_lds
-        if (off * sizeof(T) > m->tail_lds) {
-            refuse("tail levels exceed the LDS budget");
-            return;
-        }
         if (H.dim == 3)
-            hipLaunchKernelGGL((saras::k_tail<T, 3>), dim3(1), dim3(kTailThreads), off * sizeof(T), s, A);
+            hipLaunchKernelGGL((saras::k_tail<T, 3>), dim3(1), dim3(saras::kTailThreads), H.tail_bytes, s, A);
         else
-            hipLaunchKernelGGL((saras::k_tail<T, 2>), dim3(1), dim3(kTailThreads), off * sizeof(T), s, A);
+            hipLaunchKernelGGL((saras::k_tail<T, 2>), dim3(1), dim3(saras::kTailThreads), H.tail_bytes, s, A);
     }
 
     // poisson::vCycle (poisson.cc:203-279); levels S..D run in the tail kernel
@@ -1089,10 +1154,10 @@ saras_status saras_mg_create(const saras_grid_desc *grid, const saras_mg_params 
         st = m->h32->build(m->G, nowall);
         if (st) return st;
         HIP_TRY(hipMalloc((void **)&m->x64b, m->h64.lv[0].elems * sizeof(double)));
-        st = m->h32->pack_tail(tail_first_level(m.get(), *m->h32));
+        st = pack_tail(m.get(), *m->h32);
         if (st) return st;
     }
-    st = m->h64.pack_tail(tail_first_level(m.get(), m->h64));
+    st = pack_tail(m.get(), m->h64);
     if (st) return st;
     HIP_TRY(hipMalloc((void **)&m->partial, 2 * saras::kNormBlocks * sizeof(double)));
     HIP_TRY(hipHostMalloc((void **)&m->norm_host, 2 * sizeof(double), hipHostMallocCoherent));

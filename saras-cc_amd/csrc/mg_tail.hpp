@@ -2,60 +2,93 @@
 //
 // Below a few thousand cells per level a V-cycle is all launch latency: the
 // levels S..D of the reference V-cycle (poisson.cc:227-277 restricted to
-// those levels) run here inside one workgroup, every level held in LDS with
-// a real ghost layer and the reference's literal ghost timing (imposeBC at
-// the start of each sweep, periodic refresh between colours, final imposeBC;
-// poisson_d3.cc:96-246, the coarsest solve :249-432).  Arithmetic follows the
-// same expressions as the multi-block kernels, so the FP64 path stays
-// bit-identical to the reference ordering.
+// those levels) run here inside one workgroup, every level held in LDS.
+// Arithmetic follows the same expressions as the multi-block kernels, so the
+// FP64 path stays bit-identical to the reference ordering.
 //
-// Each phase of a level is a chain of LDS round trips, so the kernel keeps
-// that chain short: a level is described by LDS offsets (every access is a
-// plain LDS read, never a pointer fetched from memory), and when a level has
-// no more cells than threads each thread loads its cell's indices,
-// coefficients and right-hand side once per smoothing call, leaving a colour
-// pass with the seven neighbour reads and one write.
+// One compute unit runs the kernel, and most of its levels have fewer cells
+// than the workgroup has threads: what bounds it is the number of
+// instructions a wave issues from one barrier to the next.  So
+//  * a level is stored by colour (all red cells, then all black, each in
+//    (i, j, k / 2) order): the lanes of a pass read and write consecutive
+//    words;
+//  * there are no ghost cells to refresh: a wall neighbour is a function of
+//    the cell's own value (its address is the cell's own, its sign flipped
+//    for Dirichlet), a periodic one is the opposite core cell (as in the
+//    multi-block kernels; see mg_kernels.hpp), so a sweep is two phases;
+//  * the neighbour addresses of every cell are tabulated on the host (TailCell)
+//    and kept in registers through a smoothing call, with the coefficients,
+//    the divisor's reciprocal (FP32), the right-hand side and the value;
+//  * the residual before a restriction is taken by all fine cells at once;
+//  * the coarsest solve tests max|r| < tol by a ballot instead of a
+//    reduction, and a level of at most 64 cells of a colour runs on one wave
+//    without barriers.
+// Measured against literal ghost layers with colour lists, per V(2,2) cycle:
+// 16^3..2^3 FP32 47 -> 35 us, FP64 55 -> 43 us; 64^2..4^2 FP64 53 -> 38 us; V(3,6)
+// 16^3..2^3 FP32 70 -> 47 us; three sweeps of an 18 x 14 x 25 coarsest level FP64
+// 49 -> 24 us.  A pass of 16^3 takes about 0.7 us, the vector issue of its 32
+// wave iterations; a pass of 8^3 and below 0.2-0.3 us.
 #pragma once
+#include <type_traits>
+
 #include "mg_kernels.hpp"
 
 namespace saras {
 
 constexpr int kTailMaxLevels = 8;
+constexpr int kTailThreads = 512;
+// cells of one colour a thread keeps in registers
+constexpr int kTailColourCells = 4;
+
+// One cell of a level stored by colour.  Directions: x+, x-, y+, y-, z+, z-.
+struct TailCell {
+    unsigned a[3];   // LDS offsets of the neighbours, two per word (a wall: the cell itself)
+    unsigned cxy;    // LDS offsets of the x and y coefficient pairs (c2, c1)
+    unsigned czf;    // of the z pair, | flags << 16
+};
+// flags: bit d, direction d is a Dirichlet wall; bit 6 + d, the coarsest
+// residual sees an old value there (see tail_smooth); kNoCell: a row of odd
+// length has no such cell
+constexpr unsigned kTailNoCell = 1u << 15;
+
+// One tail level; every array is an LDS offset in elements.
+struct TailLevel {
+    int n[3];
+    int hz, half;              // cells of one colour per row (rounded up) and per level
+    int x, b, old;             // iterate, right-hand side, old values of a coarsest solve
+    int lo[3], hi[3], wd[3];   // restriction factors of this (coarse) level, 3-D
+    int neg;                   // some wall is Dirichlet
+    int odd;                   // an odd periodic extent (the coarsest level alone can have one)
+    int cell4;                 // the level's TailCell table, by words: LDS offset of the first four
+    int cell1;                 // ... and of the fifth; -1: the table is in global memory, from entry cell4
+};
 
 template <typename T>
 struct TailArgs {
     int first, last;                     // levels S and D
-    LevelArgs<T> L[kTailMaxLevels];      // level args of S..D (index l - S)
-    RestrictArgs<T> R[kTailMaxLevels];   // restriction factors of level l (l > S)
-    int xoff[kTailMaxLevels], boff[kTailMaxLevels];  // LDS offsets (elements)
-    int coff;                            // LDS offset of the staged coefficients and restriction factors
+    TailLevel L[kTailMaxLevels];         // levels S..D (index l - S)
+    long sx, sy, hz;                     // level S's layout in global memory
+    int res;                             // LDS offset of the residual of a level (by colour, as its iterate)
+    int coff, ncoef;                     // the coefficients' place in LDS and their number
+    int cellw, ncellw;                   // the cell tables' place in LDS and size, in 32-bit words
     const T *coef;                       // their packed image in global memory (the LDS region's order)
+    const unsigned *cellimg;             // the same of the cell tables
+    const uint4 *cells4;                 // the tables that are not in LDS
+    const unsigned *cells1;
     T *x;                                // global core array of level S (in/out)
     const T *b;                          // global core array of level S
     int pre, post, solve_flag, max_count;
     T w;
     double tol;
     double rel_floor;                    // as CoarseCtl::rel_floor
-    int zero_bc_first;                   // 0 only when S is the finest level
     int *iters_out;
 };
 
-
-// One tail level, every array an LDS element offset.
-template <typename T>
-struct TailLevel {
-    int n[3];
-    int PY, PZ;                // padded extents of y (1 in 2-D) and z
-    int x, b;                  // padded iterate, core right-hand side
-    int c2[3], c1[3];          // metric coefficients per axis
-    int lo[3], hi[3], wd[3];   // restriction factors of this (coarse) level, 3-D
-    int bc_lo[3], bc_hi[3];
-    const T *wall[3];
-};
-
+// position of core cell (i, j, k) in a level stored by colour
 template <int DIM>
-__device__ __forceinline__ int tidx(int PY, int PZ, int i, int j, int k) {
-    return DIM == 3 ? ((i + 1) * PY + (j + 1)) * PZ + (k + 1) : (i + 1) * PZ + (k + 1);
+__host__ __device__ __forceinline__ int tail_at(const TailLevel &V, int i, int j, int k) {
+    const int row = DIM == 3 ? i * V.n[1] + j : i;
+    return ((i + j + k) & 1) * V.half + row * V.hz + (k >> 1);
 }
 
 // (i, j, k) of core index t of a small level (32-bit unsigned arithmetic)
@@ -67,452 +100,417 @@ __device__ __forceinline__ void tcoords(int t, int ny, int nz, int &i, int &j, i
     i = (int)q;
 }
 
-// one core cell with everything but its neighbours
+// the TailCell of every cell of a level: col * half + u
+template <int DIM>
+inline void tail_cells(const TailLevel &V, const int (&c)[3], const int (&bc_lo)[3], const int (&bc_hi)[3],
+                       TailCell *out) {
+    for (int q = 0; q < 2 * V.half; ++q) out[q].czf = kTailNoCell << 16;
+    const int ny = DIM == 3 ? V.n[1] : 1;
+    for (int i = 0; i < V.n[0]; ++i)
+        for (int j = 0; j < ny; ++j)
+            for (int k = 0; k < V.n[2]; ++k) {
+                const int own = tail_at<DIM>(V, i, j, k);
+                TailCell &t = out[own];
+                unsigned flags = 0, a[6] = {0, 0, 0, 0, 0, 0};
+                for (int d = 0; d < 6; ++d) {
+                    const int ax = d / 2;
+                    if (DIM == 2 && ax == 1) continue;
+                    int p[3] = {i, j, k};
+                    const int n = V.n[ax], bc = d & 1 ? bc_lo[ax] : bc_hi[ax];
+                    p[ax] += d & 1 ? -1 : 1;
+                    if (p[ax] < 0 || p[ax] >= n) {
+                        if (bc != BC_PER) {
+                            a[d] = (unsigned)(V.x + own);
+                            flags |= 64u << d;
+                            if (bc == BC_DIR) flags |= 1u << d;
+                            continue;
+                        }
+                        p[ax] = p[ax] < 0 ? n - 1 : 0;
+                        if ((p[0] + p[1] + p[2]) & 1) flags |= 64u << d;   // a black cell
+                    }
+                    a[d] = (unsigned)(V.x + tail_at<DIM>(V, p[0], p[1], p[2]));
+                }
+                for (int ax = 0; ax < 3; ++ax) t.a[ax] = a[2 * ax] | a[2 * ax + 1] << 16;
+                t.cxy = (unsigned)(c[0] + 2 * i) | (unsigned)(c[1] + 2 * j) << 16;
+                t.czf = (unsigned)(c[2] + 2 * k) | flags << 16;
+            }
+}
+
+// the coefficient pair (c2, c1) at an LDS offset
 template <typename T>
-struct TCell {
-    int c;     // padded offset (relative to the iterate)
-    int par;   // (i + j + k) & 1
-    T c2x, c1x, c2y, c1y, c2z, c1z, b;
+__device__ __forceinline__ void tail_coef(const T *lds, unsigned at, T &c2, T &c1) {
+    using P = std::conditional_t<sizeof(T) == 4, float2, double2>;
+    const P p = *reinterpret_cast<const P *>(lds + at);
+    c2 = p.x;
+    c1 = p.y;
+}
+
+template <typename T>
+struct TailCoef {
+    T c2x, c1x, c2y, c1y, c2z, c1z;
+};
+template <typename T, int DIM>
+__device__ __forceinline__ TailCoef<T> tail_coefs(const T *lds, const TailCell &t) {
+    TailCoef<T> m;
+    m.c2y = m.c1y = T(0);
+    tail_coef(lds, t.cxy & 0xffffu, m.c2x, m.c1x);
+    if (DIM == 3) tail_coef(lds, t.cxy >> 16, m.c2y, m.c1y);
+    tail_coef(lds, t.czf & 0xffffu, m.c2z, m.c1z);
+    return m;
+}
+
+// A thread's cell: right-hand side, sor_inv of the divisor, value; KEEP: the
+// coefficients too.
+template <typename T, bool KEEP>
+struct TailOwn {
+    TailCell t;
+    T b, d, x;
+};
+template <typename T>
+struct TailOwn<T, true> {
+    TailCell t;
+    T b, d, x;
+    TailCoef<T> m;
 };
 
-template <typename T, int DIM>
-__device__ __forceinline__ void tcell_load(const T *lds, const TailLevel<T> &V, int t, TCell<T> &q) {
-    int i, j, k;
-    tcoords(t, V.n[1], V.n[2], i, j, k);
-    q.c = tidx<DIM>(V.PY, V.PZ, i, j, k);
-    q.par = (i + j + k) & 1;
-    q.c2x = lds[V.c2[0] + i];
-    q.c1x = lds[V.c1[0] + i];
-    q.c2y = DIM == 3 ? lds[V.c2[1] + j] : T(0);
-    q.c1y = DIM == 3 ? lds[V.c1[1] + j] : T(0);
-    q.c2z = lds[V.c2[2] + k];
-    q.c1z = lds[V.c1[2] + k];
-    q.b = lds[V.b + t];
-}
-
-template <typename T, int DIM>
-__device__ __forceinline__ void tgather(const T *X, int c, int sx, int sy, Stencil<T, DIM> &s) {
-    s.c = X[c];
-    s.xE = X[c + sx];
-    s.xW = X[c - sx];
-    if (DIM == 3) {
-        s.yN = X[c + sy];
-        s.yS = X[c - sy];
+// The six neighbour values of a cell; STALE: as the coarsest residual sees
+// them, `delta` from the iterate to its old values.
+template <typename T, int DIM, bool STALE>
+__device__ __forceinline__ Stencil<T, DIM> tail_gather(const T *lds, const TailCell &t, T c, bool neg, int delta) {
+    T v[6];
+#pragma unroll
+    for (int d = 0; d < 6; ++d) {
+        if (DIM == 2 && (d == 2 || d == 3)) continue;
+        int a = (int)(d & 1 ? t.a[d >> 1] >> 16 : t.a[d >> 1] & 0xffffu);
+        if (STALE && (t.czf & (64u << 16 << d))) a += delta;
+        v[d] = lds[a];
     }
-    s.zT = X[c + 1];
-    s.zB = X[c - 1];
-}
-
-template <typename T, int DIM>
-__device__ __forceinline__ T tresidual(const T *X, const TCell<T> &q, int sx, int sy) {
+    if (neg) {
+#pragma unroll
+        for (int d = 0; d < 6; ++d) {
+            if (DIM == 2 && (d == 2 || d == 3)) continue;
+            if (t.czf & (1u << 16 << d)) v[d] = -v[d];
+        }
+    }
     Stencil<T, DIM> s;
-    tgather<T, DIM>(X, q.c, sx, sy, s);
-    return residual<T, DIM>(s, q.c2x, q.c1x, q.c2y, q.c1y, q.c2z, q.c1z, q.b);
-}
-
-// One face-ghost pair: the ghosts at both ends of a line of cells along an
-// axis (lo beside cell 0, hi beside cell n-1).
-template <typename T>
-struct TGhost {
-    int glo, ghi, s0, s1;
-    int bclo, bchi;
-    bool per;
-    T wv;
-};
-
-// item q of the face lines: x faces (j, k), then y faces (i, k), then z faces (i, j)
-template <typename T, int DIM>
-__device__ __forceinline__ void tghost_load(const TailLevel<T> &V, int q, TGhost<T> &g) {
-    const int nx = V.n[0], ny = DIM == 3 ? V.n[1] : 1, nz = V.n[2];
-    const int fx = ny * nz, fy = DIM == 3 ? nx * nz : 0;
-    if (q < fx) {
-        const unsigned j = (unsigned)q / (unsigned)nz;
-        const int k = q - (int)(j * (unsigned)nz), jj = (int)j;
-        g.glo = tidx<DIM>(V.PY, V.PZ, -1, jj, k);
-        g.ghi = tidx<DIM>(V.PY, V.PZ, nx, jj, k);
-        g.s0 = tidx<DIM>(V.PY, V.PZ, 0, jj, k);
-        g.s1 = tidx<DIM>(V.PY, V.PZ, nx - 1, jj, k);
-        g.bclo = V.bc_lo[0];
-        g.bchi = V.bc_hi[0];
-        g.wv = V.bc_lo[0] == BC_DIRV ? (DIM == 3 ? V.wall[0][(jj + 1) * (nz + 2) + k + 1] : V.wall[0][k + 1]) : T(0);
-    } else if (q < fx + fy) {
-        const unsigned uq = (unsigned)(q - fx), i = uq / (unsigned)nz;
-        const int k = (int)(uq - i * (unsigned)nz), ii = (int)i;
-        g.glo = tidx<DIM>(V.PY, V.PZ, ii, -1, k);
-        g.ghi = tidx<DIM>(V.PY, V.PZ, ii, ny, k);
-        g.s0 = tidx<DIM>(V.PY, V.PZ, ii, 0, k);
-        g.s1 = tidx<DIM>(V.PY, V.PZ, ii, ny - 1, k);
-        g.bclo = V.bc_lo[1];
-        g.bchi = V.bc_hi[1];
-        g.wv = V.bc_lo[1] == BC_DIRV ? V.wall[1][(ii + 1) * (nz + 2) + k + 1] : T(0);
-    } else {
-        const unsigned uq = (unsigned)(q - fx - fy), i = uq / (unsigned)ny;
-        const int j = (int)(uq - i * (unsigned)ny), ii = (int)i;
-        g.glo = tidx<DIM>(V.PY, V.PZ, ii, j, -1);
-        g.ghi = tidx<DIM>(V.PY, V.PZ, ii, j, nz);
-        g.s0 = tidx<DIM>(V.PY, V.PZ, ii, j, 0);
-        g.s1 = tidx<DIM>(V.PY, V.PZ, ii, j, nz - 1);
-        g.bclo = V.bc_lo[2];
-        g.bchi = V.bc_hi[2];
-        g.wv = V.bc_lo[2] == BC_DIRV ? (DIM == 3 ? V.wall[2][(ii + 1) * (ny + 2) + j + 1] : V.wall[2][ii + 1]) : T(0);
+    s.c = c;
+    s.xE = v[0];
+    s.xW = v[1];
+    if (DIM == 3) {
+        s.yN = v[2];
+        s.yS = v[3];
     }
-    g.per = g.bclo == BC_PER;
+    s.zT = v[4];
+    s.zB = v[5];
+    return s;
 }
 
-// periodic lines copy the opposite core cell; with `walls` the others take
-// the wall rule of their own core cell (updateFace / imposeBC,
-// poisson_d3.cc:876-993).  Only ghosts beside core cells are written: edges
-// and corners of the shell are never read by the 7-point stencil.
-template <typename T>
-__device__ __forceinline__ void tghost_apply(T *X, const TGhost<T> &g, bool walls) {
-    if (g.per) {
-        X[g.ghi] = X[g.s0];
-        X[g.glo] = X[g.s1];
-    } else if (walls) {
-        X[g.glo] = wall_rule(g.bclo, X[g.s0], g.wv);
-        X[g.ghi] = wall_rule(g.bchi, X[g.s1], g.wv);
-    }
-}
-
-// cells of one colour per thread held in a colour list (see tail_level)
-constexpr int kTailColourCells = 4;
-// face-ghost items per thread held in registers
-constexpr int kTailGhostItems = 2;
-
-// The smoothing sweeps (or the coarsest solve) of one level: `count` RB-SOR
-// sweeps, then the final imposeBC; with SOLVE, sweeps until max|r| < tol or
-// the iteration cap (poisson_d3.cc:249-432), returning the iteration count.
-// A level with no more cells than threads keeps each thread's cell in
-// registers; a larger level with an even z extent and at most
-// kTailColourCells cells of a colour per thread keeps colour lists: the
-// packed (i, j, k) of the thread's cells of each colour, so a colour pass
-// visits only its own cells with every lane busy and loads all of a
-// thread's stencils before the first write (the cells of a colour never
-// read each other).  Other levels walk all cells.
-template <typename T, int DIM, bool WAVE, bool SOLVE>
-__device__ int tail_level(T *lds, const TailLevel<T> &V, int count, T w, double tol, double rel_floor, int max_count,
-                          double *red) {
-    constexpr int CPT = kTailColourCells, GPT = kTailGhostItems;
-    const int tid = threadIdx.x, nthr = lthreads<WAVE>();
-    const int total = V.n[0] * V.n[1] * V.n[2];
-    const int nface = DIM == 3 ? V.n[1] * V.n[2] + V.n[0] * V.n[2] + V.n[0] * V.n[1] : V.n[2] + V.n[0];
-    const int sx = DIM == 3 ? V.PY * V.PZ : V.PZ, sy = V.PZ;
-    T *X = lds + V.x;
-    const bool cached = total <= nthr, gcached = nface <= GPT * nthr;
-    const int half = total >> 1, hz2 = V.n[2] >> 1;
-    const bool lists = !cached && (V.n[2] & 1) == 0 && half <= CPT * nthr;
-    TCell<T> q{};
-    TGhost<T> g[GPT]{};
-    const bool act = cached && tid < total;
-    if (act) tcell_load<T, DIM>(lds, V, tid, q);
-    if (gcached)
-#pragma unroll
-        for (int e = 0; e < GPT; ++e)
-            if (tid + e * nthr < nface) tghost_load<T, DIM>(V, tid + e * nthr, g[e]);
-    int cell[2][CPT];   // packed i << 20 | j << 10 | k, or -1
-#pragma unroll
-    for (int col = 0; col < 2; ++col)
-#pragma unroll
-        for (int e = 0; e < CPT; ++e) {
-            cell[col][e] = -1;
-            const int u = tid + e * nthr;
-            if (lists && u < half) {
-                const unsigned row = (unsigned)u / (unsigned)hz2;
-                const int m = u - (int)(row * (unsigned)hz2);
-                const unsigned i = row / (unsigned)V.n[1];
-                const int j = (int)(row - i * (unsigned)V.n[1]);
-                const int k = 2 * m + (((int)i + j + col) & 1);
-                cell[col][e] = ((int)i << 20) | (j << 10) | k;
-            }
-        }
-
-    auto ghosts = [&](bool walls) {
-        if (gcached) {
-#pragma unroll
-            for (int e = 0; e < GPT; ++e)
-                if (tid + e * nthr < nface) tghost_apply(X, g[e], walls);
+// The smoothing sweeps of a level, or its coarsest solve: with `pro`, first
+// the correction of coarse level C is added (injection plus the saved
+// iterate, poisson_d3.cc:548-558, poisson.cc:266); then `count` RB-SOR
+// sweeps, or with `solve` sweeps until max|r| < tol or the iteration cap
+// (poisson_d3.cc:249-432), returning the iteration count; with `emit`, last
+// the residual of every cell into A.res.
+//
+// The reference takes the coarsest residual with its ghosts as they stand
+// after a sweep (poisson_d3.cc:398-415): a wall ghost is the rule applied to
+// the cell's value before the sweep, and a periodic ghost was refreshed
+// between the colours, so it holds a wrapped black cell's value from before
+// the black pass.  A pass of the solve leaves each cell's old value at
+// V.old, and the residual reads those neighbours there.
+//
+// Where a periodic extent is odd, a wrapped neighbour has the cell's own
+// colour, and its ghost its value from before the pass: all cells are read
+// before the first is written.
+//
+// CPT cells of a colour per thread are kept in registers; the cells of a
+// larger level beyond them (a coarsest one: the others are limited to
+// kTailColourCells) are loaded anew in each pass (and with an odd periodic
+// extent wait at V.old for the others' reads).
+template <typename T, int DIM, int CPT>
+__device__ __forceinline__ int tail_smooth(T *lds, const TailArgs<T> &A, const TailLevel &V, const TailLevel &C,
+                                           bool pro, bool solve, int count, bool emit, double *red, int *wflag) {
+    // FP64 with several cells per thread: the coefficients do not fit beside them
+    constexpr bool KEEP = CPT == 1 || sizeof(T) == 4;
+    using Own = TailOwn<T, KEEP>;
+    const int tid = threadIdx.x;
+    constexpr int nthr = kTailThreads, nwave = kTailThreads / 64;
+    constexpr int PAIR = CPT > 1 ? 2 : 1;   // cells whose neighbours are read together
+    const int lane = tid & 63, wv = tid >> 6;
+    const int half = V.half;
+    // at most one cell of a colour per lane of wave 0: the other waves wait
+    // at the closing barrier and the phases need none
+    const bool wave = CPT == 1 && half <= 64;
+    const bool neg = V.neg != 0, odd = V.odd != 0;
+    const bool rest = CPT > 1 && half > CPT * nthr;
+    const int delta = V.old - V.x;
+    const T w = A.w;
+    auto sync = [&]() __attribute__((always_inline)) {
+        if (wave) wave_lds_sync();
+        else __syncthreads();
+    };
+    auto cell = [&](int q) __attribute__((always_inline)) {
+        TailCell t;
+        uint4 v;
+        if (CPT == 1) {
+            const unsigned *lw = reinterpret_cast<const unsigned *>(lds);
+            v = *reinterpret_cast<const uint4 *>(lw + V.cell4 + 4 * q);
+            t.czf = lw[V.cell1 + q];
         } else {
-            for (int t = tid; t < nface; t += nthr) {
-                TGhost<T> h;
-                tghost_load<T, DIM>(V, t, h);
-                tghost_apply(X, h, walls);
-            }
+            v = A.cells4[V.cell4 + q];
+            t.czf = A.cells1[V.cell4 + q];
         }
-        lsync<WAVE>();
+        t.a[0] = v.x;
+        t.a[1] = v.y;
+        t.a[2] = v.z;
+        t.cxy = v.w;
+        return t;
     };
-    auto update = [&](const TCell<T> &r) {
-        Stencil<T, DIM> s;
-        tgather<T, DIM>(X, r.c, sx, sy, s);
-        X[r.c] = sor_update<T, DIM>(s, r.c2x, r.c1x, r.c2y, r.c1y, r.c2z, r.c1z, r.b, w);
+    // cell q of the level (col * half + u) with its value; false: none there
+    // (the addresses are valid all the same, so a caller may go on with it)
+    auto load = [&](int q, Own &o) __attribute__((always_inline)) {
+        o.t = cell(q);
+        o.b = lds[V.b + q];
+        o.x = lds[V.x + q];
+        const TailCoef<T> m = tail_coefs<T, DIM>(lds, o.t);
+        if constexpr (KEEP) o.m = m;
+        o.d = sor_inv(sor_den<T, DIM>(m.c2x, m.c2y, m.c2z));
+        return !(o.t.czf & (kTailNoCell << 16));
     };
-    auto colour = [&](int col) {
-        if (cached) {
-            if (act && q.par == col) update(q);
-        } else if (lists) {
-            T r[CPT];
-            int c[CPT];
+    auto coefs = [&](const Own &o) __attribute__((always_inline)) {
+        if constexpr (KEEP) return o.m;
+        else return tail_coefs<T, DIM>(lds, o.t);
+    };
+    auto update = [&](const Own &o) __attribute__((always_inline)) {
+        const Stencil<T, DIM> s = tail_gather<T, DIM, false>(lds, o.t, o.x, neg, 0);
+        const TailCoef<T> m = coefs(o);
+        const T num = sor_num<T, DIM>(s, m.c2x, m.c1x, m.c2y, m.c1y, m.c2z, m.c1z, o.b, w);
+        return (T(1.0) - w) * o.x + sor_quot_inv(num, o.d);
+    };
+    auto resid = [&](const Own &o, auto stale) __attribute__((always_inline)) {
+        constexpr bool STALE = decltype(stale)::value;
+        const Stencil<T, DIM> s = tail_gather<T, DIM, STALE>(lds, o.t, o.x, neg, delta);
+        const TailCoef<T> m = coefs(o);
+        return residual<T, DIM>(s, m.c2x, m.c1x, m.c2y, m.c1y, m.c2z, m.c1z, o.b);
+    };
+    int iter = 0;
+    if (!wave || wv == 0) {
+        Own o[2][CPT];
+        bool act[2][CPT];
+        if (pro) {
+            for (int q = tid; q < 2 * half; q += wave ? 64 : nthr) {
+                const int col = q >= half, u = q - col * half;
+                const unsigned row = (unsigned)u / (unsigned)V.hz;
+                const int m = u - (int)(row * (unsigned)V.hz);
+                // rows (i, j) -> coarse (i / 2, j / 2); both cells m of a row have K = m
+                const int i = DIM == 3 ? (int)(row / (unsigned)V.n[1]) : (int)row;
+                const int j = DIM == 3 ? (int)(row - (unsigned)i * (unsigned)V.n[1]) : 0;
+                lds[V.x + q] = lds[C.x + tail_at<DIM>(C, i >> 1, j >> 1, m)] + lds[V.x + q];
+            }
+            sync();
+        }
+        // a thread beyond the level's last cell takes that cell too, without
+        // writing it: no load waits behind a branch
+#pragma unroll
+        for (int col = 0; col < 2; ++col)
 #pragma unroll
             for (int e = 0; e < CPT; ++e) {
-                const int p = col ? cell[1][e] : cell[0][e];
-                c[e] = -1;
-                if (p < 0) continue;
-                const int i = p >> 20, j = (p >> 10) & 1023, k = p & 1023;
-                TCell<T> t;
-                t.c = tidx<DIM>(V.PY, V.PZ, i, j, k);
-                t.c2x = lds[V.c2[0] + i];
-                t.c1x = lds[V.c1[0] + i];
-                t.c2y = DIM == 3 ? lds[V.c2[1] + j] : T(0);
-                t.c1y = DIM == 3 ? lds[V.c1[1] + j] : T(0);
-                t.c2z = lds[V.c2[2] + k];
-                t.c1z = lds[V.c1[2] + k];
-                t.b = lds[V.b + (i * V.n[1] + j) * V.n[2] + k];
-                Stencil<T, DIM> s;
-                tgather<T, DIM>(X, t.c, sx, sy, s);
-                r[e] = sor_update<T, DIM>(s, t.c2x, t.c1x, t.c2y, t.c1y, t.c2z, t.c1z, t.b, w);
-                c[e] = t.c;
+                const int u = tid + e * nthr;
+                act[col][e] = load(col * half + min(u, half - 1), o[col][e]) && u < half;
             }
+        auto pass = [&](auto colc) __attribute__((always_inline)) {
+            constexpr int col = decltype(colc)::value;
+            const int base = V.x + col * half;
 #pragma unroll
-            for (int e = 0; e < CPT; ++e)
-                if (c[e] >= 0) X[c[e]] = r[e];
-        } else {
-            for (int t = tid; t < total; t += nthr) {
-                int i, j, k;
-                tcoords(t, V.n[1], V.n[2], i, j, k);
-                if (((i + j + k) & 1) != col) continue;
-                TCell<T> r;
-                tcell_load<T, DIM>(lds, V, t, r);
-                update(r);
+            for (int p = 0; p < CPT; p += PAIR) {
+                if (p > 0 && p * nthr >= half) continue;
+                T v[PAIR];
+#pragma unroll
+                for (int e = 0; e < PAIR; ++e) v[e] = update(o[col][p + e]);
+#pragma unroll
+                for (int e = 0; e < PAIR; ++e) {
+                    const int at = base + tid + (p + e) * nthr;
+                    if (act[col][p + e]) {
+                        if (solve) lds[at + delta] = o[col][p + e].x;
+                        if (!odd) lds[at] = v[e];
+                    }
+                    o[col][p + e].x = v[e];
+                }
             }
-        }
-        lsync<WAVE>();
-    };
-    // imposeBC, red, the periodic refresh, black: one loop so that the
-    // colour pass's code appears once
-    auto sweep = [&]() {
-        for (int col = 0; col < 2; ++col) {
-            ghosts(col == 0);
-            colour(col);
-        }
-    };
-
-    int iter = 0;
-    if (SOLVE) {
-        if (rel_floor > 0.0) {
+            if (rest)
+                for (int u = tid + CPT * nthr; u < half; u += nthr) {
+                    Own q;
+                    if (!load(col * half + u, q)) continue;
+                    const T v = update(q);
+                    lds[base + u] = odd ? q.x : v;
+                    if (solve || odd) lds[base + u + delta] = odd ? v : q.x;
+                }
+            if (odd) {
+                sync();
+#pragma unroll
+                for (int e = 0; e < CPT; ++e)
+                    if (act[col][e]) lds[base + tid + e * nthr] = o[col][e].x;
+                if (rest)
+                    for (int u = tid + CPT * nthr; u < half; u += nthr) {
+                        const T v = lds[base + u + delta];
+                        lds[base + u + delta] = lds[base + u];
+                        lds[base + u] = v;
+                    }
+            }
+            sync();
+        };
+        double tol = A.tol;
+        if (solve && A.rel_floor > 0.0) {
             // the FP32 floor of the correction equation (CoarseCtl::rel_floor)
             double bm = 0.0;
-            for (int t = tid; t < total; t += nthr) bm = fmax(bm, fabs((double)lds[V.b + t]));
-            tol = fmax(tol, rel_floor * group_max<WAVE>(bm, red));
-        }
-        for (;;) {
-            sweep();
-            // max |r| with the ghosts as they stand (poisson_d3.cc:398-415)
-            double lm = -1.0e-10;
-            if (cached) {
-                if (act) {
-                    const double a = fabs((double)tresidual<T, DIM>(X, q, sx, sy));
-                    if (a > lm) lm = a;
-                }
-            } else {
-                for (int t = tid; t < total; t += nthr) {
-                    TCell<T> r;
-                    tcell_load<T, DIM>(lds, V, t, r);
-                    const double a = fabs((double)tresidual<T, DIM>(X, r, sx, sy));
-                    if (a > lm) lm = a;
-                }
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+#pragma unroll
+                for (int e = 0; e < CPT; ++e)
+                    if (act[col][e]) bm = fmax(bm, fabs((double)o[col][e].b));
+                if (rest)
+                    for (int u = tid + CPT * nthr; u < half; u += nthr) {
+                        Own q;
+                        if (load(col * half + u, q)) bm = fmax(bm, fabs((double)q.b));
+                    }
             }
-            const double mx = group_max<WAVE>(lm, red);
-            if (mx < tol) break;
-            iter += 1;
-            if (iter > max_count) break;
+            tol = fmax(tol, A.rel_floor * (wave ? group_max<true>(bm, red) : group_max<false>(bm, red)));
         }
-    } else {
-        for (int n = 0; n < count; ++n) sweep();
+        for (int n = 0; solve || n < count; ++n) {
+            pass(std::integral_constant<int, 0>{});
+            pass(std::integral_constant<int, 1>{});
+            if (!solve) continue;
+            bool any = false;
+            // |r| >= tol of some cell; the reference's maximum starts at
+            // -1e-10 and passes over NaN
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+#pragma unroll
+                for (int e = 0; e < CPT; ++e) {
+                    if (e > 0 && e * nthr >= half) continue;
+                    any = (fabs((double)resid(o[col][e], std::true_type{})) >= tol && act[col][e]) || any;
+                }
+                if (rest)
+                    for (int u = tid + CPT * nthr; u < half; u += nthr) {
+                        Own q;
+                        if (load(col * half + u, q)) any = fabs((double)resid(q, std::true_type{})) >= tol || any;
+                    }
+            }
+            any = __ballot(any) != 0;
+            if (!wave) {
+                if (lane == 0) wflag[wv] = any ? 1 : 0;
+                __syncthreads();
+                any = __ballot(lane < nwave && wflag[lane < nwave ? lane : 0] != 0) != 0;
+            }
+            if (!any && -1.0e-10 < tol) break;
+            iter += 1;
+            if (iter > A.max_count) break;
+        }
+        if (emit) {
+#pragma unroll
+            for (int col = 0; col < 2; ++col)
+#pragma unroll
+                for (int e = 0; e < CPT; ++e) {
+                    if (e > 0 && e * nthr >= half) continue;
+                    const T r = resid(o[col][e], std::false_type{});
+                    if (act[col][e]) lds[A.res + col * half + tid + e * nthr] = r;
+                }
+        }
     }
-    ghosts(true);
+    // a one-wave level is read by the whole workgroup next
+    __syncthreads();
     return iter;
 }
 
 template <typename T, int DIM>
-__global__ void __launch_bounds__(512) k_tail(TailArgs<T> A) {
+__global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A) {
     extern __shared__ __align__(16) unsigned char tail_raw[];
     T *lds = reinterpret_cast<T *>(tail_raw);
     __shared__ double red[16];
-    __shared__ TailLevel<T> TL[kTailMaxLevels];
-    const int S = A.first, D = A.last, nl = D - S + 1;
-    auto ext = [&](int q, int a) { return (DIM == 2 && a == 1) ? 1 : A.L[q].n[a]; };
+    __shared__ int wflag[kTailThreads / 64];
+    const int S = A.first, D = A.last;
 
     // Staging, with every global load issued before the first barrier: the
-    // metric coefficients of each tail level and (3-D) the restriction
-    // factors of levels S+1..D, which every phase reads, are copied to LDS
-    // from their packed image (one flat coalesced copy) and described by LDS
-    // offsets; level S's iterate and right-hand side come in beside them.
-    // Level S's ghost shell is not cleared: every face ghost is written
-    // before it is read.
+    // metric coefficients and restriction factors and the cell tables as flat
+    // coalesced copies of their packed images, level S's iterate and
+    // right-hand side beside them.
     {
-        if (threadIdx.x == 0) {
-            int off = A.coff;
-            for (int q = 0; q < nl; ++q) {
-                TailLevel<T> &V = TL[q];
-                const LevelArgs<T> &L = A.L[q];
-                for (int a = 0; a < 3; ++a) {
-                    V.n[a] = L.n[a];
-                    V.bc_lo[a] = L.bc_lo[a];
-                    V.bc_hi[a] = L.bc_hi[a];
-                    V.wall[a] = L.wall[a];
-                    V.c2[a] = off;
-                    V.c1[a] = off + ext(q, a);
-                    off += 2 * ext(q, a);
-                }
-                V.PY = DIM == 3 ? L.n[1] + 2 : 1;
-                V.PZ = L.n[2] + 2;
-                V.x = A.xoff[q];
-                V.b = A.boff[q];
-            }
-            if (DIM == 3)
-                for (int q = 1; q < nl; ++q)
-                    for (int a = 0; a < 3; ++a) {
-                        const int n = A.L[q].n[a];
-                        TL[q].lo[a] = off;
-                        TL[q].hi[a] = off + n;
-                        TL[q].wd[a] = off + 2 * n;
-                        off += 3 * n;
-                    }
-        }
-        int ncoef = 0, nres = 0;
-        for (int q = 0; q < nl; ++q)
-            for (int a = 0; a < 3; ++a) {
-                ncoef += 2 * ext(q, a);
-                if (DIM == 3 && q > 0) nres += 3 * A.L[q].n[a];
-            }
-        for (int e = threadIdx.x; e < ncoef + nres; e += blockDim.x) lds[A.coff + e] = A.coef[e];
-        const LevelArgs<T> &L = A.L[0];
-        const int PZ = L.n[2] + 2, PY = DIM == 3 ? L.n[1] + 2 : 1;
-        T *XS = lds + A.xoff[0];
-        T *BS = lds + A.boff[0];
-        const int total = L.n[0] * L.n[1] * L.n[2];
-        for (int t = threadIdx.x; t < total; t += blockDim.x) {
+        unsigned *lw = reinterpret_cast<unsigned *>(lds);
+        for (int e = threadIdx.x; e < A.ncoef; e += kTailThreads) lds[A.coff + e] = A.coef[e];
+        for (int e = threadIdx.x; e < A.ncellw / 4; e += kTailThreads)
+            *reinterpret_cast<uint4 *>(lw + A.cellw + 4 * e) = reinterpret_cast<const uint4 *>(A.cellimg)[e];
+        const TailLevel &V = A.L[0];
+        const int total = V.n[0] * V.n[1] * V.n[2];
+        for (int t = threadIdx.x; t < total; t += kTailThreads) {
             int i, j, k;
-            tcoords(t, L.n[1], L.n[2], i, j, k);
-            const long g = (long)i * L.sx + (long)j * L.sy + kof(L, k);
-            XS[tidx<DIM>(PY, PZ, i, j, k)] = A.x[g];
-            BS[t] = A.b[g];
+            tcoords(t, V.n[1], V.n[2], i, j, k);
+            const long g = (long)i * A.sx + (long)j * A.sy + (A.hz ? (long)(k & 1) * A.hz + (k >> 1) : (long)k);
+            const int at = tail_at<DIM>(V, i, j, k);
+            lds[V.x + at] = A.x[g];
+            lds[V.b + at] = A.b[g];
         }
         __syncthreads();
     }
-    auto padded = [&](const TailLevel<T> &V) { return DIM == 3 ? (V.n[0] + 2) * V.PY * V.PZ : (V.n[0] + 2) * V.PZ; };
-    // one level's smoothing or coarsest solve by the whole workgroup (a
-    // wave-only variant for the smallest levels measured no faster and
-    // doubled the kernel's code)
-    auto level = [&](int l, bool solve, int count) {
-        const TailLevel<T> V = TL[l - S];
-        if (solve) return tail_level<T, DIM, false, true>(lds, V, 0, A.w, A.tol, A.rel_floor, A.max_count, red);
-        tail_level<T, DIM, false, false>(lds, V, count, A.w, A.tol, A.rel_floor, A.max_count, red);
-        return 0;
-    };
 
     // The V-cycle over levels S..D as one loop of steps, so that each phase's
     // code appears once in the kernel (a single CU runs this kernel, and its
     // instruction cache holds far less than one copy per call site):
-    //   step 0: level S -- the coarsest treatment when S == D > 0 (the host
-    //     restricted into it), otherwise pre-smoothing, which is also the
-    //     whole V-cycle of a single-level hierarchy (poisson.cc:228);
-    //   down-leg, per l = S..D-1: the residual of l restricted into the
-    //     right-hand side of l + 1 (whose iterate starts at zero), then
-    //     pre-smoothing of l + 1 or the coarsest solve;
-    //   up-leg, per l = D-1..S: injection plus the saved iterate, then
+    //   down-leg, l = S..D: pre-smoothing (the coarsest treatment at D > 0;
+    //     l = S = D = 0 is the whole V-cycle of a single-level hierarchy,
+    //     poisson.cc:228), then the residual of l restricted into the
+    //     right-hand side of l + 1, whose iterate starts at zero;
+    //   up-leg, l = D-1..S: injection plus the saved iterate, then
     //     post-smoothing of l.
     int iters = 0;  // meaningful in thread 0
-    const int nsteps = 1 + 4 * (D - S);
+    const int nsteps = 2 * (D - S) + 1;
     for (int st = 0; st < nsteps; ++st) {
-        int kind = 0, l = S, count = A.pre;   // kind 0: smooth/solve l, 1: restrict l, 2: prolong into l
-        bool solve = false;
-        if (st == 0) {
-            solve = S == D && S > 0 && A.solve_flag;
-        } else if (st <= 2 * (D - S)) {
-            const int d = st - 1;
-            l = S + d / 2;
-            if ((d & 1) == 0) {
-                kind = 1;
+        const bool up = st > D - S;
+        const int l = up ? D - (st - (D - S)) : S + st;
+        const bool solve = l == D && D > 0 && A.solve_flag;
+        const bool emit = !up && l < D;
+        const int count = up ? A.post : A.pre;
+        const TailLevel &V = A.L[l - S], &C = A.L[l < D ? l + 1 - S : l - S];
+        int it;
+        if (V.cell1 >= 0) it = tail_smooth<T, DIM, 1>(lds, A, V, C, up, solve, count, emit, red, wflag);
+        else it = tail_smooth<T, DIM, kTailColourCells>(lds, A, V, C, up, solve, count, emit, red, wflag);
+        if (solve) iters = it;
+        if (!emit) continue;
+        // computeResidual + coarsen (poisson_d3.cc:71-93, 484-511; poisson_d2.cc:288-297)
+        const int ctotal = C.n[0] * C.n[1] * C.n[2];
+        const T *R = lds + A.res;
+        for (int q = threadIdx.x; q < 2 * C.half; q += kTailThreads) lds[C.x + q] = T(0);
+        for (int t = threadIdx.x; t < ctotal; t += kTailThreads) {
+            int I, J, K;
+            tcoords(t, C.n[1], C.n[2], I, J, K);
+            // child (di, dj, dk): row (2I + di, 2J + dj), position K of the colour of its k parity
+            auto r = [&](int di, int dj, int dk) {
+                return R[((di + dj + dk) & 1) * V.half + (DIM == 3 ? (2 * I + di) * V.n[1] + 2 * J + dj : 2 * I + di) * V.hz + K];
+            };
+            T out;
+            if (DIM == 3) {
+                const T lx = lds[C.lo[0] + I], hx = lds[C.hi[0] + I], ly = lds[C.lo[1] + J], hy = lds[C.hi[1] + J],
+                        lz = lds[C.lo[2] + K], hz = lds[C.hi[2] + K];
+                const T v000 = lx * ly * lz, v100 = hx * ly * lz, v010 = lx * hy * lz, v001 = lx * ly * hz;
+                const T v011 = lx * hy * hz, v101 = hx * ly * hz, v110 = hx * hy * lz, v111 = hx * hy * hz;
+                const T vtot = lds[C.wd[0] + I] * lds[C.wd[1] + J] * lds[C.wd[2] + K];
+                out = (v111 * r(1, 1, 1) + v000 * r(0, 0, 0) + v110 * r(1, 1, 0) + v001 * r(0, 0, 1) +
+                       v101 * r(1, 0, 1) + v010 * r(0, 1, 0) + v011 * r(0, 1, 1) + v100 * r(1, 0, 0)) / vtot;
             } else {
-                l += 1;
-                solve = l == D && A.solve_flag;
+                out = (r(1, 0, 1) + r(0, 0, 0) + r(1, 0, 0) + r(0, 0, 1)) / T(4);
             }
-        } else {
-            const int u = st - 1 - 2 * (D - S);
-            l = D - 1 - u / 2;
-            kind = (u & 1) == 0 ? 2 : 0;
-            count = A.post;
+            lds[C.b + tail_at<DIM>(C, I, J, K)] = out;
         }
-        if (kind == 1) {
-            const TailLevel<T> F = TL[l - S];
-            const TailLevel<T> C = TL[l + 1 - S];
-            const int fsx = DIM == 3 ? F.PY * F.PZ : F.PZ, fsy = F.PZ;
-            const T *XF = lds + F.x;
-            T *XC = lds + C.x;
-            for (int q = threadIdx.x; q < padded(C); q += blockDim.x) XC[q] = T(0);
-            const int ctotal = C.n[0] * C.n[1] * C.n[2];
-            for (int t = threadIdx.x; t < ctotal; t += blockDim.x) {
-                int I, J, K;
-                tcoords(t, C.n[1], C.n[2], I, J, K);
-                T res[2][2][2];
-                for (int di = 0; di < 2; ++di)
-                    for (int dj = 0; dj < (DIM == 3 ? 2 : 1); ++dj)
-                        for (int dk = 0; dk < 2; ++dk) {
-                            const int i = 2 * I + di, j = DIM == 3 ? 2 * J + dj : 0, k = 2 * K + dk;
-                            TCell<T> r;
-                            r.c = tidx<DIM>(F.PY, F.PZ, i, j, k);
-                            r.c2x = lds[F.c2[0] + i];
-                            r.c1x = lds[F.c1[0] + i];
-                            r.c2y = DIM == 3 ? lds[F.c2[1] + j] : T(0);
-                            r.c1y = DIM == 3 ? lds[F.c1[1] + j] : T(0);
-                            r.c2z = lds[F.c2[2] + k];
-                            r.c1z = lds[F.c1[2] + k];
-                            r.b = lds[F.b + (i * F.n[1] + j) * F.n[2] + k];
-                            res[di][dj][dk] = tresidual<T, DIM>(XF, r, fsx, fsy);
-                        }
-                T out;
-                if (DIM == 3) {
-                    const T lx = lds[C.lo[0] + I], hx = lds[C.hi[0] + I], ly = lds[C.lo[1] + J],
-                            hy = lds[C.hi[1] + J], lz = lds[C.lo[2] + K], hz = lds[C.hi[2] + K];
-                    const T v000 = lx * ly * lz, v100 = hx * ly * lz, v010 = lx * hy * lz, v001 = lx * ly * hz;
-                    const T v011 = lx * hy * hz, v101 = hx * ly * hz, v110 = hx * hy * lz, v111 = hx * hy * hz;
-                    const T vtot = lds[C.wd[0] + I] * lds[C.wd[1] + J] * lds[C.wd[2] + K];
-                    out = (v111 * res[1][1][1] + v000 * res[0][0][0] + v110 * res[1][1][0] + v001 * res[0][0][1] +
-                           v101 * res[1][0][1] + v010 * res[0][1][0] + v011 * res[0][1][1] + v100 * res[1][0][0]) /
-                          vtot;
-                } else {
-                    out = (res[1][0][1] + res[0][0][0] + res[1][0][0] + res[0][0][1]) / T(4);
-                }
-                lds[C.b + t] = out;
-            }
-            __syncthreads();
-        } else if (kind == 2) {
-            const TailLevel<T> F = TL[l - S];
-            const TailLevel<T> C = TL[l + 1 - S];
-            const int total = F.n[0] * F.n[1] * F.n[2];
-            T *XF = lds + F.x;
-            const T *XC = lds + C.x;
-            for (int t = threadIdx.x; t < total; t += blockDim.x) {
-                int i, j, k;
-                tcoords(t, F.n[1], F.n[2], i, j, k);
-                const int c = tidx<DIM>(F.PY, F.PZ, i, j, k);
-                XF[c] = XC[tidx<DIM>(C.PY, C.PZ, i >> 1, j >> 1, k >> 1)] + XF[c];
-            }
-            __syncthreads();
-        } else {
-            const int it = level(l, solve, count);
-            if (solve) iters = it;
-        }
+        __syncthreads();
     }
     // level S back to global memory
     {
-        const LevelArgs<T> &L = A.L[0];
-        const TailLevel<T> V = TL[0];
-        const int total = L.n[0] * L.n[1] * L.n[2];
-        for (int t = threadIdx.x; t < total; t += blockDim.x) {
+        const TailLevel &V = A.L[0];
+        const int total = V.n[0] * V.n[1] * V.n[2];
+        for (int t = threadIdx.x; t < total; t += kTailThreads) {
             int i, j, k;
-            tcoords(t, L.n[1], L.n[2], i, j, k);
-            A.x[(long)i * L.sx + (long)j * L.sy + kof(L, k)] = lds[V.x + tidx<DIM>(V.PY, V.PZ, i, j, k)];
+            tcoords(t, V.n[1], V.n[2], i, j, k);
+            A.x[(long)i * A.sx + (long)j * A.sy + (A.hz ? (long)(k & 1) * A.hz + (k >> 1) : (long)k)] =
+                lds[V.x + tail_at<DIM>(V, i, j, k)];
         }
     }
     if (threadIdx.x == 0 && A.iters_out && A.solve_flag) *A.iters_out = iters;
