@@ -27,6 +27,7 @@
 #include "mg_kernels.hpp"
 #include "mg_split.hpp"
 #include "mg_tail.hpp"
+#include "mg_tile.hpp"
 #include "saras_hip.h"
 
 namespace {
@@ -65,7 +66,13 @@ struct DevLevel {
     long sx = 0, sy = 0;
     size_t elems = 0;  // allocation size in elements
     T *x = nullptr, *b = nullptr;
-    T *xalt = nullptr;  // second iterate buffer: fused sweeps run out of place
+    T *xalt = nullptr;  // second iterate buffer: fused sweeps and tiles run out of place
+    // the visits of a V-cycle by tiles (k_tile): pre-smoothing from a zero
+    // iterate (and, level 0, from any) with the restriction, post-smoothing
+    // with the prolongation; no launches: by separate passes
+    struct Tile {
+        int ti = 0, tj = 0, sweeps = 0;   // tile rows, sweeps of a launch
+    } pre, pre0, post;
     long hz = 0;        // colour-split rows when > 0 (offset of the odd half)
     T *c2zs = nullptr, *c1zs = nullptr;  // z coefficients in split order
     T *c2[3] = {nullptr, nullptr, nullptr}, *c1[3] = {nullptr, nullptr, nullptr};
@@ -258,6 +265,7 @@ struct saras_mg {
     bool split_off = false;            // SARAS_NO_SPLIT=1 keeps every level z-contiguous
     size_t tail_lds = kTailLdsDefault;  // dynamic LDS budget of the tail kernel
     bool red_fold = true;              // SARAS_NO_RED_FOLD=1: the restriction leaves the first red pass to the sweep
+    bool tile_off = false;             // SARAS_NO_TILE=1 runs every pass as a launch of its own
     bool rr_lane = false;              // SARAS_RR_LANE=1: 3-D split restriction with all eight children in one lane
     // V-cycles replayed from captured hipGraphs (saras_mg_set_graphs).  A
     // graph bakes in the level buffers, and out-of-place sweeps swap them, so
@@ -383,6 +391,80 @@ size_t tail_layout(const saras_mg *m, const Hierarchy<T> &H, int S, saras::TailA
     }
     const size_t bytes = w * 4;
     return bytes <= m->tail_lds && w / words < 65536 ? bytes : 0;
+}
+
+// LDS of a tile (k_tile has no static LDS), of the 160 KB a workgroup may hold
+constexpr size_t kTileLds = 156 * 1024;
+
+// The plan of one visit of level l by tiles, or none where separate passes are
+// faster by this estimate (us).  A kernel takes about 4 us however little it
+// does; a pass beyond that is bound by its 1.5 words per cell at about 7 TB/s
+// (levels of this size sit in the Infinity Cache).  A tile launch adds, per
+// workgroup of a compute unit, its rows' vectors: about kVec cycles of vector
+// issue for 64 of them, and about 350 cycles a pass for the barrier and the LDS
+// latency.  Measured over tiles of 2 to 16 by 1 to 8 rows, 1 to 6 sweeps a
+// launch, 32^3..128^3 and 128^2..2048^2 in both precisions: the estimate's choice
+// is within 3 % of the fastest V-cycle, and turns to separate passes where
+// those are (64^3 with six sweeps FP64, 128^3, 2048^2).
+template <typename T>
+typename DevLevel<T>::Tile plan_tile(const saras_mg *m, const Hierarchy<T> &H, int l, int count, bool zero, bool pro,
+                                     bool restr) {
+    typename DevLevel<T>::Tile best;
+    const DevLevel<T> &L = H.lv[l];
+    const int nv = saras::tile_vecs<T>(L.n[2]);
+    if (m->tile_off || count < 1 || l + 1 >= (int)H.lv.size() || (L.n[2] & 1) || nv > saras::kTileThreads) return best;
+    for (int a = 0; a < 3; ++a)
+        if (m->g.periodic[a] && !(H.dim == 2 && a == 1) && (L.n[a] & 1)) return best;
+    if (l == 0 && m->p.bc == SARAS_BC_DIRICHLET_TEST) return best;
+    constexpr double kLaunch = 4.0, kVec = 125.0, kClock = 2400.0, kCus = 256.0;
+    const double cells = (double)L.n[0] * L.n[1] * L.n[2];
+    const double pass = std::max(kLaunch + 0.2, 2.8 + 1.5 * cells * sizeof(T) / 7e6);
+    double cost = 2 * count * pass + (restr ? 1.4 * pass : 0.0) + (pro ? 0.4 * pass : 0.0);
+    if (!L.hz && pro) cost += pass;   // a prolongation pass of its own
+    cost *= 0.95;
+    const int jmax = H.dim == 3 ? 8 : 1;
+    for (int ti = 2; ti <= 32; ti *= 2)
+        for (int tj = H.dim == 3 ? 2 : 1; tj <= jmax; tj *= 2)
+            for (int s = 1; s <= count; ++s) {
+                double c = 0.0;
+                bool ok = true;
+                for (int done = 0; done < count && ok; done += s) {
+                    const bool z = zero && done == 0, r = restr && done + s >= count;
+                    const int sw = std::min(s, count - done), halo = saras::tile_halo(sw, z, r);
+                    ok = saras::tile_bytes<T>(H.dim, L.n[2], ti, tj, halo) <= kTileLds && halo <= L.n[0] &&
+                         (H.dim == 2 || halo <= L.n[1]);
+                    auto rows = [&](int q) { return (double)(ti + 2 * q) * (H.dim == 3 ? tj + 2 * q : 1); };
+                    double vecs = (z ? 1.0 : 1.5) * rows(halo) + (r ? 3.0 * rows(0) : 0.0);
+                    for (int p = 0; p < 2 * sw; ++p) vecs += rows(2 * sw - 1 - p + (r ? 1 : 0));
+                    const double tiles = std::ceil((double)L.n[0] / ti) * (H.dim == 3 ? std::ceil((double)L.n[1] / tj) : 1.0);
+                    const double per_cu = std::max(1.0, tiles / kCus);
+                    c += kLaunch + 1.0 + (std::ceil(per_cu) * vecs * nv / 64.0 * kVec + 350.0 * 2 * sw) / kClock;
+                }
+                if (ok && c < cost) {
+                    cost = c;
+                    best.ti = ti;
+                    best.tj = tj;
+                    best.sweeps = s;
+                }
+            }
+    return best;
+}
+
+// plans of every level, and the second iterate buffer of those that tile
+template <typename T>
+saras_status plan_tiles(const saras_mg *m, Hierarchy<T> &H) {
+    const int D = (int)H.lv.size() - 1;
+    for (int l = 0; l < std::min(H.tail_first, D); ++l) {
+        DevLevel<T> &L = H.lv[l];
+        L.pre = plan_tile(m, H, l, m->p.pre_smooth, true, false, true);
+        if (l == 0) L.pre0 = plan_tile(m, H, l, m->p.pre_smooth, false, false, true);
+        L.post = plan_tile(m, H, l, m->p.post_smooth, false, true, false);
+        if ((L.pre.sweeps || L.pre0.sweeps || L.post.sweeps) && !L.xalt) {
+            HIP_TRY(hipMalloc((void **)&L.xalt, L.elems * sizeof(T)));
+            HIP_TRY(hipMemset(L.xalt, 0, L.elems * sizeof(T)));
+        }
+    }
+    return SARAS_OK;
 }
 
 // The tail of a hierarchy: the levels from the finest one that fits its LDS
@@ -774,6 +856,88 @@ struct Ops {
 
     int tail_start() const { return H.tail_first; }
 
+    template <int DIM, bool HZ, int MODE>
+    void tile_launch(int grid, size_t bytes, const saras::TileArgs<T> &A) {
+        hipLaunchKernelGGL((saras::k_tile<T, DIM, HZ, MODE>), dim3(grid), dim3(saras::kTileThreads), bytes, s, A);
+    }
+    template <int DIM>
+    void tile_launch(int grid, size_t bytes, const saras::TileArgs<T> &A) {
+        using namespace saras;
+        if (A.L.hz) {
+            if (A.zero) tile_launch<DIM, true, TILE_ZERO>(grid, bytes, A);
+            else if (A.pro) tile_launch<DIM, true, TILE_PRO>(grid, bytes, A);
+            else tile_launch<DIM, true, TILE_PLAIN>(grid, bytes, A);
+        } else {
+            if (A.zero) tile_launch<DIM, false, TILE_ZERO>(grid, bytes, A);
+            else if (A.pro) tile_launch<DIM, false, TILE_PRO>(grid, bytes, A);
+            else tile_launch<DIM, false, TILE_PLAIN>(grid, bytes, A);
+        }
+    }
+
+    // `count` sweeps of level l by tiles of plan t, at most t.sweeps of them a
+    // launch: the first launch takes `zero` or `pro`, the last one `restr`
+    void tile(int l, const typename DevLevel<T>::Tile &t, int count, bool zero, bool pro, bool restr) {
+        DevLevel<T> &L = H.lv[l];
+        const int ntj = H.dim == 3 ? (L.n[1] + t.tj - 1) / t.tj : 1;
+        for (int done = 0; done < count; done += t.sweeps) {
+            const bool first = done == 0, last = done + t.sweeps >= count;
+            saras::TileArgs<T> A{};
+            A.L = level_args(m, H, l, false);
+            A.x = L.x;
+            A.y = L.xalt;
+            A.b = L.b;
+            A.ti = t.ti;
+            A.tj = t.tj;
+            A.nti = (L.n[0] + t.ti - 1) / t.ti;
+            A.ntj = ntj;
+            A.sweeps = std::min(t.sweeps, count - done);
+            A.zero = zero && first;
+            A.pro = pro && first;
+            A.restr = restr && last;
+            A.halo = saras::tile_halo(A.sweeps, A.zero, A.restr);
+            A.w = w;
+            if (A.pro) {
+                const DevLevel<T> &C = H.lv[l + 1];
+                A.e = C.x;
+                A.esx = C.sx;
+                A.esy = C.sy;
+                A.ehz = C.hz;
+            }
+            if (A.restr) {
+                DevLevel<T> &C = H.lv[l + 1];
+                A.C = level_args(m, H, l + 1, false);
+                A.cb = C.b;
+                A.cx = C.x;
+                for (int q = 0; q < 3; ++q) {
+                    A.R.lo[q] = C.rlo[q];
+                    A.R.hi[q] = C.rhi[q];
+                    A.R.wd[q] = C.rwd[q];
+                }
+            }
+            const size_t bytes = saras::tile_bytes<T>(H.dim, L.n[2], t.ti, t.tj, A.halo);
+            // host-side guards of what the kernel assumes
+            if (!L.xalt || bytes > kTileLds || (L.n[2] & 1) || saras::tile_vecs<T>(L.n[2]) > saras::kTileThreads) {
+                refuse("a level that does not tile");
+                return;
+            }
+            const int ntile = A.nti * A.ntj, grid = (ntile + saras::kXcds - 1) / saras::kXcds * saras::kXcds;
+            if (H.dim == 3) tile_launch<3>(grid, bytes, A);
+            else tile_launch<2>(grid, bytes, A);
+            std::swap(L.x, L.xalt);
+        }
+    }
+
+    // pre-smoothing of level l < D and the residual's restriction; `zero`: the iterate is zero
+    void descend(int l, bool zero, bool red_next) {
+        const auto &t = zero ? H.lv[l].pre : H.lv[l].pre0;
+        if (t.sweeps) {
+            tile(l, t, m->p.pre_smooth, zero, false, true);
+            return;
+        }
+        smooth(l, m->p.pre_smooth, l != 0);
+        resid_restrict(l, red_next);
+    }
+
     void tail(int S) {
         const int D = (int)H.lv.size() - 1;
         // host-side guard: the tail packed for this hierarchy
@@ -809,19 +973,25 @@ struct Ops {
             tail(0);
             return;
         }
-        smooth(0, m->p.pre_smooth, false);
+        if (D == 0) smooth(0, m->p.pre_smooth, false);
         for (int l = 0; l < D; ++l) {
-            resid_restrict(l, m->red_fold && l + 1 < S && l + 1 < D && m->p.pre_smooth > 0);
+            // the restriction also takes the coarse level's first red pass where that level runs by passes
+            const bool red = m->red_fold && l + 1 < S && l + 1 < D && m->p.pre_smooth > 0 && !H.lv[l + 1].pre.sweeps;
+            const bool zero = l > 0 || zero0;
+            if (l == 0 && H.lv[0].pre.sweeps) zero0 = false;
+            descend(l, zero, red);
             if (l + 1 == S) break;
             if (l + 1 == D) {
                 if (m->p.solve_flag) coarse(D, true, 0, 0);
                 else smooth(D, m->p.pre_smooth, true);
-            } else {
-                smooth(l + 1, m->p.pre_smooth, true);
             }
         }
         if (S <= D) tail(S);
         for (int l = std::min(S, D) - 1; l >= 0; --l) {
+            if (H.lv[l].post.sweeps) {
+                tile(l, H.lv[l].post, m->p.post_smooth, false, true, false);
+                continue;
+            }
             if (m->p.post_smooth > 0 && (march_ok(l) || H.lv[l].hz)) pend_level = l;
             else prolong_correct(l);
             smooth(l, m->p.post_smooth, l != 0);
@@ -1124,6 +1294,8 @@ saras_status saras_mg_create(const saras_grid_desc *grid, const saras_mg_params 
         m->march_tj8 = env4 && env4[0] == '1';
         const char *env5 = std::getenv("SARAS_NO_SPLIT");
         m->split_off = env5 && env5[0] == '1';
+        const char *env10 = std::getenv("SARAS_NO_TILE");
+        m->tile_off = env10 && env10[0] == '1';
         const char *env9 = std::getenv("SARAS_RR_LANE");
         m->rr_lane = env9 && env9[0] == '1';
         const char *env8 = std::getenv("SARAS_NO_RED_FOLD");
@@ -1155,9 +1327,12 @@ saras_status saras_mg_create(const saras_grid_desc *grid, const saras_mg_params 
         if (st) return st;
         HIP_TRY(hipMalloc((void **)&m->x64b, m->h64.lv[0].elems * sizeof(double)));
         st = pack_tail(m.get(), *m->h32);
+        if (!st) st = plan_tiles(m.get(), *m->h32);
         if (st) return st;
     }
     st = pack_tail(m.get(), m->h64);
+    // (the mixed solver's cycles run on the FP32 hierarchy alone)
+    if (!st && p.precision == SARAS_PREC_FP64) st = plan_tiles(m.get(), m->h64);
     if (st) return st;
     HIP_TRY(hipMalloc((void **)&m->partial, 2 * saras::kNormBlocks * sizeof(double)));
     HIP_TRY(hipHostMalloc((void **)&m->norm_host, 2 * sizeof(double), hipHostMallocCoherent));
@@ -1534,7 +1709,7 @@ size_t saras_mg_footprint(const saras_grid_desc *grid, const saras_mg_params *pa
             const long a128 = 128 / (long)word;
             const size_t sy = (size_t)((n[2] + a128 - 1) / a128 * a128);
             const size_t elems = sy * n[1] * n[0];
-            tot += elems * word * ((l < D && grid->dim == 3) ? 3 : 2);
+            tot += elems * word * (l < D ? 3 : 2);
             tot += 5 * 3 * (size_t)(n[0] + n[1] + n[2]) * word;
         }
         return tot;
