@@ -70,7 +70,7 @@ import saras_amd as S  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
 N = 256
-DOMINANT = "k_rb_split_zp<float,3,true,false,true,false>"
+DOMINANT = "k_rb_split<float,3,0,true,true,false>"
 # HBM bytes per launch of the dominant kernel (one FP32 colour pass of the
 # finest level of the z-periodic 256^3 grid, SOR parameter 1) from rocprofv3
 # --pmc FETCH_SIZE / WRITE_SIZE (KiB per dispatch), calibrated against the

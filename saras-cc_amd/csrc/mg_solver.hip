@@ -75,6 +75,7 @@ struct DevLevel {
     } pre, pre0, post;
     long hz = 0;        // colour-split rows when > 0 (offset of the odd half)
     T *c2zs = nullptr, *c1zs = nullptr;  // z coefficients in split order
+    bool uniform = false;                // every axis has one value of c2 and one of c1
     T *c2[3] = {nullptr, nullptr, nullptr}, *c1[3] = {nullptr, nullptr, nullptr};
     T *rlo[3] = {nullptr, nullptr, nullptr}, *rhi[3] = {nullptr, nullptr, nullptr}, *rwd[3] = {nullptr, nullptr, nullptr};
 };
@@ -153,6 +154,7 @@ struct Hierarchy {
                 HIP_TRY(hipMemset(L.xalt, 0, L.elems * sizeof(T)));
             }
             HIP_TRY(hipMemset(L.b, 0, L.elems * sizeof(T)));
+            L.uniform = true;
             for (int a = 0; a < 3; ++a) {
                 if (dim == 2 && a == 1) {
                     std::vector<double> z(1, 0.0);
@@ -173,6 +175,7 @@ struct Hierarchy {
                     c2[i] = A.xix2[i + 1] * ih2;
                     c1[i] = A.xixx[i + 1] * i2h;
                 }
+                for (int i = 1; i < A.n; ++i) L.uniform = L.uniform && c2[i] == c2[0] && c1[i] == c1[0];
                 if (upload(&L.c2[a], c2) || upload(&L.c1[a], c1)) return SARAS_HIP_ERROR;
                 hc2[l][a] = c2;
                 hc1[l][a] = c1;
@@ -265,6 +268,7 @@ struct saras_mg {
     bool split_off = false;            // SARAS_NO_SPLIT=1 keeps every level z-contiguous
     size_t tail_lds = kTailLdsDefault;  // dynamic LDS budget of the tail kernel
     bool red_fold = true;              // SARAS_NO_RED_FOLD=1: the restriction leaves the first red pass to the sweep
+    bool rb_general = false;           // SARAS_RB_GENERAL=1 runs every split colour pass in the general form
     bool tile_off = false;             // SARAS_NO_TILE=1 runs every pass as a launch of its own
     bool rr_lane = false;              // SARAS_RR_LANE=1: 3-D split restriction with all eight children in one lane
     // V-cycles replayed from captured hipGraphs (saras_mg_set_graphs).  A
@@ -632,68 +636,64 @@ struct Ops {
         return L.n[1] % 16 == 0 && L.n[2] % 64 == 0 && (long)L.n[0] * L.n[1] * L.n[2] >= (8L << 20);
     }
 
-    template <int DIM, bool ZP, bool FINE, bool PRO>
-    void split_launch(const dim3 &g, const saras::LevelArgs<T> &a, DevLevel<T> &L, int colour, int nb, const T *e,
-                      long esx, long esy, long ehz, bool z = false) {
-        const dim3 bl(saras::kSplitThreads);
-        // z: the finest level's first red pass on an iterate known to be zero
-        if constexpr (FINE && !PRO) {
-            if (z) {
-                if (w == T(1)) {
-                    if (ZP) hipLaunchKernelGGL((saras::k_rb_split_zp<T, DIM, FINE, PRO, true, true>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-                    else hipLaunchKernelGGL((saras::k_rb_split<T, DIM, FINE, PRO, true, true>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-                } else {
-                    if (ZP) hipLaunchKernelGGL((saras::k_rb_split_zp<T, DIM, FINE, PRO, false, true>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-                    else hipLaunchKernelGGL((saras::k_rb_split<T, DIM, FINE, PRO, false, true>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-                }
-                return;
-            }
+    // One colour pass of a split level.  The paired form (k_rb_split with R = 2)
+    // takes levels whose rows pair up along y (x in a planar level), whose
+    // arrays 32-bit byte offsets reach and whose walls are homogeneous -- every
+    // level but a DIRICHLET_TEST level 0, odd row counts (a coarsest level's
+    // parent has even ones) and FP64 arrays of 4 GB and more, which the
+    // general form takes.
+    // Time of a pass, one row per lane with branches around each load / now:
+    // FP32 256^3 19.6 / 16.8 us (after the prolongation: red 33 / 20, black
+    // 20 / 16.4), 512^3 180 / 150 us (279 / 197, 183 / 147), tanh z 256^3 20.1 /
+    // 17.7 us; FP64 256^3 38.9 / 32.0 us (red 58 / 47.8).  512^3 FP32 moves its
+    // 1.5 words per cell at 5.4 TB/s.
+    template <int DIM, int MODE>
+    void rb_pass(int l, const saras::LevelArgs<T> &a, int colour, const T *e, long esx, long esy, long ehz) {
+        using namespace saras;
+        DevLevel<T> &L = H.lv[l];
+        const int np = DIM == 3 ? L.n[1] : L.n[0];
+        const bool dirv = a.bc_lo[0] == BC_DIRV || a.bc_lo[2] == BC_DIRV;
+        const bool gen = (np & 1) || L.elems * sizeof(T) > 0xffffffffull || dirv || m->rb_general;
+        const int R = gen ? 1 : 2;
+        RowMap M;
+        const unsigned q = (unsigned)(L.n[2] / 2 / Vec16<T>::W);
+        const unsigned wj = DIM == 3 ? (unsigned)((a.rtile ? a.rtile : L.n[1]) / R) : 1u;
+        M.q = FastDiv::of(q);
+        M.tile = FastDiv::of((unsigned)L.n[0] * wj);
+        M.wj = FastDiv::of(wj);
+        const size_t total = (size_t)L.n[0] * L.n[1] / R * q;
+        // host-side guard: vector numbers stay below 2^31
+        if (total + kSplitThreads * kXcds > 0x7fffffffull || (a.rtile && a.rtile % R)) {
+            refuse("a level too large for one pass");
+            return;
         }
-        // w == 1 (every reference deck): the pass that skips the cells' own values
-        if (w == T(1)) {
-            if (ZP) hipLaunchKernelGGL((saras::k_rb_split_zp<T, DIM, FINE, PRO, true>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-            else hipLaunchKernelGGL((saras::k_rb_split<T, DIM, FINE, PRO, true>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-        } else {
-            if (ZP) hipLaunchKernelGGL((saras::k_rb_split_zp<T, DIM, FINE, PRO, false>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-            else hipLaunchKernelGGL((saras::k_rb_split<T, DIM, FINE, PRO, false>), g, bl, 0, s, a, L.x, L.b, colour, w, nb, e, esx, esy, ehz);
-        }
+        M.total = (unsigned)total;
+        const unsigned nb = (unsigned)((total + kSplitThreads - 1) / kSplitThreads);
+        const dim3 g((nb + kXcds - 1) / kXcds * kXcds), bl(kSplitThreads);
+        if (gen)
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, true>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+        else if (w != T(1))
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, false>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+        else if (L.uniform)
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, true, false>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+        else
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, false, false>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
     }
 
     template <int DIM>
-    void split_pass(bool fine, bool pro, int grid, const saras::LevelArgs<T> &a, DevLevel<T> &L, int colour, int nb,
-                    const T *e, long esx, long esy, long ehz, bool z = false) {
-        const dim3 g(grid);
-        // rows that wrap in z, or rows split between waves, need the
-        // z-prefetching variant (see rb_split_body)
-        const int q = L.n[2] / 2 / saras::Vec16<T>::W;
-        const bool zp = a.bc_lo[2] == saras::BC_PER || !(q % 64 == 0 || 64 % q == 0);
-        if (zp) {
-            if (fine) {
-                if (pro) split_launch<DIM, true, true, true>(g, a, L, colour, nb, e, esx, esy, ehz);
-                else split_launch<DIM, true, true, false>(g, a, L, colour, nb, e, esx, esy, ehz, z);
-            } else {
-                if (pro) split_launch<DIM, true, false, true>(g, a, L, colour, nb, e, esx, esy, ehz);
-                else split_launch<DIM, true, false, false>(g, a, L, colour, nb, e, esx, esy, ehz);
-            }
-            return;
-        }
-        if (fine) {
-            if (pro) split_launch<DIM, false, true, true>(g, a, L, colour, nb, e, esx, esy, ehz);
-            else split_launch<DIM, false, true, false>(g, a, L, colour, nb, e, esx, esy, ehz, z);
-        } else {
-            if (pro) split_launch<DIM, false, false, true>(g, a, L, colour, nb, e, esx, esy, ehz);
-            else split_launch<DIM, false, false, false>(g, a, L, colour, nb, e, esx, esy, ehz);
-        }
+    void rb_pass(int l, const saras::LevelArgs<T> &a, int colour, bool pro, bool zero, const T *e, long esx, long esy,
+                 long ehz) {
+        using namespace saras;
+        if (zero) rb_pass<DIM, RB_ZERO>(l, a, colour, e, esx, esy, ehz);
+        else if (!pro) rb_pass<DIM, RB_PLAIN>(l, a, colour, e, esx, esy, ehz);
+        else if (colour == 0) rb_pass<DIM, RB_RED>(l, a, colour, e, esx, esy, ehz);
+        else rb_pass<DIM, RB_BLACK>(l, a, colour, e, esx, esy, ehz);
     }
 
     void rb_sweep(int l, bool zero_bc) {
         DevLevel<T> &L = H.lv[l];
         auto a = level_args(m, H, l, inhom(l, zero_bc));
         if (L.hz) {
-            constexpr int W = saras::Vec16<T>::W;
-            const long total = (long)L.n[0] * L.n[1] * (L.n[2] / 2 / W);
-            const int nb = (int)((total + saras::kSplitThreads - 1) / saras::kSplitThreads);
-            const int grid = (nb + saras::kXcds - 1) / saras::kXcds * saras::kXcds;
             // the first sweep after the prolongation applies it (see k_rb_split)
             const bool pro = pend_level == l;
             const T *e = nullptr;
@@ -714,8 +714,8 @@ struct Ops {
             if (l == 0) zero0 = false;
             for (int colour = first; colour < 2; ++colour) {
                 const bool zc = z && colour == 0;
-                if (H.dim == 3) split_pass<3>(l == 0, pro, grid, a, L, colour, nb, e, esx, esy, ehz, zc);
-                else split_pass<2>(l == 0, pro, grid, a, L, colour, nb, e, esx, esy, ehz, zc);
+                if (H.dim == 3) rb_pass<3>(l, a, colour, pro, zc, e, esx, esy, ehz);
+                else rb_pass<2>(l, a, colour, pro, zc, e, esx, esy, ehz);
             }
             return;
         }
@@ -1294,6 +1294,8 @@ saras_status saras_mg_create(const saras_grid_desc *grid, const saras_mg_params 
         m->march_tj8 = env4 && env4[0] == '1';
         const char *env5 = std::getenv("SARAS_NO_SPLIT");
         m->split_off = env5 && env5[0] == '1';
+        const char *env11 = std::getenv("SARAS_RB_GENERAL");
+        m->rb_general = env11 && env11[0] == '1';
         const char *env10 = std::getenv("SARAS_NO_TILE");
         m->tile_off = env10 && env10[0] == '1';
         const char *env9 = std::getenv("SARAS_RR_LANE");

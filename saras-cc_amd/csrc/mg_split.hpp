@@ -15,6 +15,8 @@
 // rows: the neighbour rows of a row were fetched by the same XCD a moment
 // earlier and are read from its L2.
 #pragma once
+#include <type_traits>
+
 #include "mg_kernels.hpp"
 
 namespace saras {
@@ -115,258 +117,350 @@ __device__ __forceinline__ T coarse_at(const T *__restrict__ e, long base, long 
     return e[base + (chz ? (long)(K & 1) * chz + (K >> 1) : (long)K)];
 }
 
-// One colour pass over a split level; the grid is a multiple of kXcds
-// blocks, `nblocks` of them carry work.  PRO: the pass belongs to the first
-// sweep after the prolongation, whose input is x + P e with P the injection
-// from the coarse iterate e (poisson_d3.cc:548-558, poisson.cc:266): the red
-// pass reads every cell as e(coarse) + x, the black pass its own cells (its
-// neighbours are the red values just written), so the separate
-// prolongation pass is not needed.
-// ZPRE: the z neighbour that no adjacent lane holds (periodic wrap, or a row
-// split between waves) is loaded together with the row vectors; without it
-// that load is issued only where needed, which is cheaper when it never is.
+// n / d for n < 2^31 by a multiplication (Granlund and Montgomery, "Division
+// by invariant integers using multiplication", 1994): m = ceil(2^(31 + l) / d),
+// l = ceil(log2 d), and the quotient is the high word of m n shifted by l - 1.
+struct FastDiv {
+    unsigned m = 0, s = 0, d = 1;   // m = 0: d = 1
+    __host__ static FastDiv of(unsigned d) {
+        FastDiv f;
+        f.d = d;
+        if (d <= 1) return f;
+        unsigned l = 0;
+        while ((1ull << l) < d) ++l;
+        f.m = (unsigned)(((1ull << (31 + l)) + d - 1) / d);
+        f.s = l - 1;
+        return f;
+    }
+    __device__ __forceinline__ unsigned div(unsigned n) const { return m ? __umulhi(n, m) >> s : n; }
+};
+
+// How the vectors of a colour pass are numbered: vector v of row group g, the
+// R rows (i, R jp ..) of a 3-D level or (R g ..) of a planar one.  Groups run
+// over the rows of a tile of wj groups, i by i, then the next tile (wj covers
+// the whole y axis where rows need no tiles, see LevelArgs::rtile).
+struct RowMap {
+    FastDiv q, tile, wj;   // vectors of a half-row; groups of a tile; groups of a tile's i-row
+    unsigned total;        // vectors of the level
+};
+
+// What the iterate is when a colour pass reads it.
+//   RB_PLAIN  the level's iterate.
+//   RB_ZERO   zero (a red pass): x is not read, +0 stands wherever a cell would
+//             have been, and the black half is written as +0, the same values
+//             as clearing x and running the ordinary pass.
+//   RB_RED, RB_BLACK  the first sweep after the prolongation, whose input is
+//             x + P e with P the injection from the coarse iterate e
+//             (poisson_d3.cc:548-558, poisson.cc:266): the red pass reads every
+//             cell as e(coarse) + x, the black pass its own cells (its
+//             neighbours are the red values just written), so the separate
+//             prolongation pass is not needed.
+enum RbMode { RB_PLAIN, RB_ZERO, RB_RED, RB_BLACK };
+
+// One colour pass over a split level; the grid is a multiple of kXcds blocks.
+// A lane updates one vector of each of R rows that follow one another along y
+// (x in a planar level).  With R = 2 each row's vector of the other colour is
+// also the neighbour row of the other, so the pair loads 10 vectors of the
+// iterate and right-hand side where two single rows load 14.
+//
 // W1: w == 1 (the "SOR Parameter" of every reference deck).  The update
 // (1 - w) x + q then equals q whenever q != 0 and x is finite (0 x is a
 // signed zero), so the cells' own values are read only where q is a zero
-// (to give the sign the reference's sum has) or where a wall rule needs them:
-// a pass reads 1.5 words per updated cell pair instead of 2.
-// Z: the level's iterate is known to be zero (the FP32 correction at the
-// start of a refinement); the red pass reads no x at all, uses +0 wherever
-// it would have read a cell, and writes +0 to the black half of its vectors,
-// which the iterate would otherwise have been cleared to beforehand: the
-// same values as clearing x and running the ordinary pass.
-template <typename T, int DIM, bool PRO, bool ZPRE, bool W1, bool Z = false>
-__device__ __forceinline__ void rb_split_body(const LevelArgs<T> &L, T *__restrict__ x, const T *__restrict__ b,
-                                              int colour, T w, int nblocks, const T *__restrict__ e, long esx,
-                                              long esy, long ehz) {
-    static_assert(!(Z && PRO), "a zero iterate has no prolongation to apply");
+// (to give the sign the reference's sum has).
+// UNI: every axis is uniform, so the coefficients are one value per axis and
+// the divisor (FP32: its reciprocal) is formed once.
+// GEN: the general form (R = 1, any w, 64-bit offsets, inhomogeneous walls).
+//
+// No load waits behind a lane-dependent branch: a neighbour beyond a wall is
+// read at the cell's own place (which is the Neumann rule) and its sign
+// flipped for a Dirichlet wall, and a row's parity selects between loaded
+// values; byte offsets are 32 bits wide on scalar bases, divisions by the row
+// length are multiplications.  Issuing that arithmetic and waiting for one
+// load after another took as long as the traffic before: see the measured
+// times at Ops::rb_pass (mg_solver.hip).
+template <typename T, int DIM, int MODE, bool W1, bool UNI, bool GEN>
+__global__ void __launch_bounds__(kSplitThreads) k_rb_split(LevelArgs<T> L, RowMap M, T *__restrict__ x,
+                                                            const T *__restrict__ b, int colour, T w,
+                                                            const T *__restrict__ e, long esx, long esy, long ehz) {
+    static_assert(!GEN || (!W1 && !UNI), "the general form takes any w and any metric");
     using VT = Vec16<T>;
     using V = typename VT::V;
-    constexpr int W = VT::W;
-    const int per = gridDim.x / kXcds;
-    const int logical = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-    if (logical >= nblocks) return;
-    const int nx = L.n[0], ny = L.n[1], nz = L.n[2];
-    const int half = nz >> 1, q = half / W;
-    const long total = (long)nx * ny * q;
-    const long t = (long)logical * kSplitThreads + threadIdx.x;
-    if (t >= total) return;
-    const int row = (int)(t / q);
-    const int v = (int)(t - (long)row * q);
+    using OFF = std::conditional_t<GEN, unsigned long, unsigned>;   // byte offset
+    constexpr int W = VT::W, R = GEN ? 1 : 2;
+    constexpr bool RED = MODE == RB_RED, BLACK = MODE == RB_BLACK, ZERO = MODE == RB_ZERO;
+    const unsigned per = gridDim.x / kXcds;
+    const unsigned logical = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+    const unsigned t = logical * kSplitThreads + threadIdx.x;
+    if (t >= M.total) return;
+    const int nx = L.n[0], ny = L.n[1], half = L.n[2] >> 1;
+    const unsigned g = M.q.div(t);
+    const int m0 = (int)(t - g * M.q.d) * W;
     int i, j;
-    if (L.rtile) {
-        const int jt = L.rtile, tile = row / (nx * jt), rem = row - tile * (nx * jt);
-        i = rem >> __builtin_ctz(jt);
-        j = tile * jt + (rem & (jt - 1));
+    if (DIM == 3) {
+        const unsigned tile = M.tile.div(g), rem = g - tile * M.tile.d, gi = M.wj.div(rem);
+        i = (int)gi;
+        j = R * (int)(tile * M.wj.d + rem - gi * M.wj.d);
     } else {
-        i = row / ny;
-        j = row - i * ny;
+        i = R * (int)g;
+        j = 0;
     }
-    const int h = (i + j + colour) & 1;   // half of this row holding the colour
-    const int m0 = v * W;
-    const long rb = (long)i * L.sx + (long)j * L.sy;
-    const long own = rb + h * L.hz + m0;
-    const long oth = rb + (1 - h) * L.hz + m0;
-    // the cell's own value: always without W1; with it only on rows whose x/y
-    // neighbour lies beyond a wall and at the z-wall ends of a row
-    bool need_c = !W1;
-    if (W1) {
-        need_c = (i + 1 >= nx && L.bc_hi[0] != BC_PER) || (i == 0 && L.bc_lo[0] != BC_PER);
-        if (DIM == 3) need_c = need_c || (j + 1 >= ny && L.bc_hi[1] != BC_PER) || (j == 0 && L.bc_lo[1] != BC_PER);
-        need_c = need_c || (h == 0 && m0 == 0 && L.bc_lo[2] != BC_PER) ||
-                 (h == 1 && m0 + W == half && L.bc_hi[2] != BC_PER);
+    const OFF sx = (OFF)L.sx * sizeof(T), sy = (OFF)L.sy * sizeof(T), hz = (OFF)L.hz * sizeof(T);
+    const OFF vo = (OFF)m0 * sizeof(T);
+    auto xv = [&](OFF o) __attribute__((always_inline)) {
+        return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(x) + o);
+    };
+    auto ld = [](const T *p, OFF o) __attribute__((always_inline)) {
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + o);
+    };
+    // the axis along which the R rows follow one another (P), and x in 3-D (Q)
+    constexpr int AP = DIM == 3 ? 1 : 0;
+    const OFF sp = DIM == 3 ? sy : sx;
+    const int p0 = DIM == 3 ? j : i, np = DIM == 3 ? ny : nx;
+    const int h0 = (i + j + colour) & 1;
+    OFF row[R], own[R], oth[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int h = h0 ^ (r & 1);
+        row[r] = (OFF)i * sx + (OFF)j * sy + (OFF)r * sp;
+        own[r] = row[r] + (h ? hz : 0) + vo;
+        oth[r] = row[r] + (h ? 0 : hz) + vo;
     }
-    V cv{}, ov{};
-    if (!Z && need_c) cv = *reinterpret_cast<const V *>(x + own);
-    if (!Z) ov = *reinterpret_cast<const V *>(x + oth);
-    const V bv = *reinterpret_cast<const V *>(b + own);
-    const V c2v = *reinterpret_cast<const V *>(L.c2zs + h * half + m0);
-    const V c1v = *reinterpret_cast<const V *>(L.c1zs + h * half + m0);
-    // The z neighbour beyond this lane's vector that no adjacent lane of the
-    // wave holds (the periodic wrap at a row end, or the row's previous / next
-    // vector when it sits in another wave), loaded with the row vectors so
-    // that its latency overlaps theirs.  h == 0 (k even): element m0 - 1 of
-    // the other half; h == 1 (k odd): element m0 + W of the other half.
+    // neighbour rows: wrapped, or beyond a wall the row itself
+    const bool inl = p0 > 0, inr = p0 + R < np, perp = L.bc_lo[AP] == BC_PER;
+    const OFF pl = own[0] + (inl ? (OFF)0 - sp : (perp ? (OFF)(np - 1) * sp : (OFF)0));
+    const OFF pr = own[R - 1] + (inr ? sp : (perp ? (OFF)0 - (OFF)(np - 1) * sp : (OFF)0));
+    const bool ine = i + 1 < nx, inw = i > 0, perx = L.bc_lo[0] == BC_PER;
+    const OFF de = ine ? sx : (perx ? (OFF)0 - (OFF)(nx - 1) * sx : (OFF)0);
+    const OFF dw = inw ? (OFF)0 - sx : (perx ? (OFF)(nx - 1) * sx : (OFF)0);
+    const bool perz = L.bc_lo[2] == BC_PER;
     const int lane = threadIdx.x & 63;
-    long zoff = -1;
-    int zK = 0;
-    if (ZPRE) {
-    if (h == 0) {
-        if (m0 == 0) {
-            if (L.bc_lo[2] == BC_PER) {
-                zoff = rb + L.hz + (half - 1);
-                zK = half - 1;
+
+    // ---- loads ----
+    V ov[R], bv[R], plv{}, prv{}, ev[R], wv[R], cv[R];
+    T zx[R];
+    bool zend[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        ov[r] = ev[r] = wv[r] = cv[r] = V{};
+        if (!ZERO) {
+            ov[r] = xv(oth[r]);
+            if (DIM == 3) {
+                ev[r] = xv(own[r] + de);
+                wv[r] = xv(own[r] + dw);
             }
-        } else if (lane == 0) {
-            zoff = oth - 1;
-            zK = m0 - 1;
+            if (!W1) cv[r] = xv(own[r]);
         }
+        bv[r] = *reinterpret_cast<const V *>(reinterpret_cast<const char *>(b) + own[r]);
+    }
+    if (!ZERO) {
+        plv = xv(pl);
+        prv = xv(pr);
+    }
+    // The z neighbour beyond a lane's vector, below its first even cell or
+    // above its last odd one, where no adjacent lane of the wave holds it: the
+    // row's end (wrapped, or the cell itself at a wall) or the next vector in
+    // another wave.
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int h = h0 ^ (r & 1);
+        zend[r] = h ? m0 + W == half : m0 == 0;
+        const OFF zw = h ? row[r] : row[r] + hz + (OFF)(half - 1) * sizeof(T);
+        const OFF zs = h ? own[r] + (W - 1) * sizeof(T) : own[r];
+        const OFF zn = h ? oth[r] + W * sizeof(T) : oth[r] - sizeof(T);
+        zx[r] = T(0);
+        if (!ZERO && (zend[r] || lane == (h ? 63 : 0))) zx[r] = ld(x, zend[r] ? (perz ? zw : zs) : zn);
+    }
+    T c2x, c1x, c2y[R], c1y[R], c2z[R][W], c1z[R][W];
+    if constexpr (UNI) {
+        c2x = L.c2[0][0];
+        c1x = L.c1[0][0];
     } else {
-        if (m0 + W == half) {
-            if (L.bc_hi[2] == BC_PER) {
-                zoff = rb;
-                zK = 0;
-            }
-        } else if (lane == 63) {
-            zoff = oth + W;
-            zK = m0 + W;
-        }
+        c2x = DIM == 3 ? L.c2[0][i] : T(0);
+        c1x = DIM == 3 ? L.c1[0][i] : T(0);
     }
-    }
-    const T zx = (!Z && ZPRE && zoff >= 0) ? x[zoff] : T(0);
-    T c[W], o[W];
+    T c2r[R], c1r[R];   // planar: the x coefficients of each row
 #pragma unroll
-    for (int q = 0; q < W; ++q) {
-        c[q] = VT::get(cv, q);
-        o[q] = VT::get(ov, q);
-    }
-    // own coarse row of the prolongation: cells m0.. of both halves map to K = m0..
-    // The black pass of W1 reads no cell of its own colour (its neighbours are
-    // the red values just written), so it needs the correction only where it
-    // reads its own cells: on wall rows, or for a zero quotient (loaded there).
-    const long ebase = (long)(i >> 1) * esx + (long)(j >> 1) * esy;
-    T evo[W];
-    const bool evo_now = PRO && (colour == 0 || !W1 || need_c);
-    if (evo_now) {
-        coarse_vec(e, ebase, ehz, m0, evo);
-#pragma unroll
-        for (int q = 0; q < W; ++q) {
-            c[q] = evo[q] + c[q];
-            if (colour == 0) o[q] = evo[q] + o[q];
-        }
-    }
-    // x and y neighbour rows: whole vectors, or the wall rule per cell
-    auto kk = [&](int e) { return 2 * (m0 + e) + h; };
-    T xe[W], xw[W], yn[W], ys[W];
-    // nbr_i, nbr_j: the neighbour row's indices (wrapped), for its coarse row
-    auto side = [&](T(&out)[W], bool inside, long off, int bc, int axis, int nbr_i, int nbr_j) {
-        if (inside || bc == BC_PER) {
-            V nv{};
-            if (!Z) nv = *reinterpret_cast<const V *>(x + own + off);
-#pragma unroll
-            for (int q = 0; q < W; ++q) out[q] = VT::get(nv, q);
-            if (PRO && colour == 0) {
-                // a neighbour row in the same coarse row shares this lane's correction
-                if ((nbr_i >> 1) == (i >> 1) && (nbr_j >> 1) == (j >> 1)) {
-#pragma unroll
-                    for (int q = 0; q < W; ++q) out[q] = evo[q] + out[q];
-                } else {
-                    T ev[W];
-                    coarse_vec(e, (long)(nbr_i >> 1) * esx + (long)(nbr_j >> 1) * esy, ehz, m0, ev);
-#pragma unroll
-                    for (int q = 0; q < W; ++q) out[q] = ev[q] + out[q];
-                }
-            }
-        } else {
+    for (int r = 0; r < R; ++r) {
+        c2r[r] = DIM == 3 || UNI ? c2x : L.c2[0][i + r];
+        c1r[r] = DIM == 3 || UNI ? c1x : L.c1[0][i + r];
+        c2y[r] = DIM == 3 ? (UNI ? L.c2[1][0] : L.c2[1][j + r]) : T(0);
+        c1y[r] = DIM == 3 ? (UNI ? L.c1[1][0] : L.c1[1][j + r]) : T(0);
+        if constexpr (UNI) {
 #pragma unroll
             for (int q = 0; q < W; ++q) {
-                T wv = T(0);
-                if (bc == BC_DIRV) {
-                    const int k = kk(q);
-                    if (axis == 0) wv = DIM == 3 ? L.wall[0][(j + 1) * (nz + 2) + k + 1] : L.wall[0][k + 1];
-                    else wv = L.wall[1][(i + 1) * (nz + 2) + k + 1];
-                }
-                out[q] = bc_value(bc, c[q], T(0), wv);
-            }
-        }
-    };
-    side(xe, i + 1 < nx, i + 1 < nx ? L.sx : -(long)(nx - 1) * L.sx, L.bc_hi[0], 0, i + 1 < nx ? i + 1 : 0, j);
-    side(xw, i > 0, i > 0 ? -L.sx : (long)(nx - 1) * L.sx, L.bc_lo[0], 0, i > 0 ? i - 1 : nx - 1, j);
-    if (DIM == 3) {
-        side(yn, j + 1 < ny, j + 1 < ny ? L.sy : -(long)(ny - 1) * L.sy, L.bc_hi[1], 1, i, j + 1 < ny ? j + 1 : 0);
-        side(ys, j > 0, j > 0 ? -L.sy : (long)(ny - 1) * L.sy, L.bc_lo[1], 1, i, j > 0 ? j - 1 : ny - 1);
-    }
-    // the z value beyond the vector, with the correction when the red pass of
-    // a prolongation sweep reads it (coarse cell K): prefetched (ZPRE) or read here
-    auto zread = [&](long off, int K) -> T {
-        const T v = Z ? T(0) : x[off];
-        return (PRO && colour == 0) ? coarse_at(e, ebase, ehz, K) + v : v;
-    };
-    auto zfix = [&](long off, int K) -> T {
-        if (ZPRE) return (PRO && colour == 0) ? coarse_at(e, ebase, ehz, zK) + zx : zx;
-        return zread(off, K);
-    };
-    // z neighbours: k - 1 and k + 1 lie in the other half.  h == 0 (k even):
-    // other[m - 1], other[m]; h == 1 (k odd): other[m], other[m + 1].  The
-    // element beyond this lane's vector comes from the adjacent lane when it
-    // holds the same row.
-    const T from_prev = __shfl_up(o[W - 1], 1, 64);
-    const T from_next = __shfl_down(o[0], 1, 64);
-    T zlo0 = T(0), zhi_last = T(0);
-    if (h == 0) {
-        if (m0 == 0) {
-            if (L.bc_lo[2] == BC_PER) zlo0 = zfix(rb + L.hz + (half - 1), half - 1);
-            else {
-                const T wv = L.bc_lo[2] == BC_DIRV ? (DIM == 3 ? L.wall[2][(i + 1) * (ny + 2) + j + 1] : L.wall[2][i + 1])
-                                                   : T(0);
-                zlo0 = bc_value(L.bc_lo[2], c[0], T(0), wv);
+                c2z[r][q] = L.c2[2][0];
+                c1z[r][q] = L.c1[2][0];
             }
         } else {
-            zlo0 = lane > 0 ? from_prev : zfix(oth - 1, m0 - 1);
-        }
-    } else {
-        if (m0 + W == half) {
-            if (L.bc_hi[2] == BC_PER) zhi_last = zfix(rb, 0);
-            else {
-                const T wv = L.bc_hi[2] == BC_DIRV ? (DIM == 3 ? L.wall[2][(i + 1) * (ny + 2) + j + 1] : L.wall[2][i + 1])
-                                                   : T(0);
-                zhi_last = bc_value(L.bc_hi[2], c[W - 1], T(0), wv);
+            const int at = (h0 ^ (r & 1)) * half + m0;
+            const V a = *reinterpret_cast<const V *>(L.c2zs + at), c = *reinterpret_cast<const V *>(L.c1zs + at);
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                c2z[r][q] = VT::get(a, q);
+                c1z[r][q] = VT::get(c, q);
             }
-        } else {
-            zhi_last = lane < 63 ? from_next : zfix(oth + W, m0 + W);
         }
     }
-    const T c2x = L.c2[0][i], c1x = L.c1[0][i];
-    const T c2y = DIM == 3 ? L.c2[1][j] : T(0), c1y = DIM == 3 ? L.c1[1][j] : T(0);
-    T r[W];
-    bool zero = false;
+    // ---- the prolongation: the coarse vector over cells m0.. of a row ----
+    auto coarse = [&](int ci, int cj, T(&out)[W]) __attribute__((always_inline)) {
+        coarse_vec(e, (long)ci * esx + (long)cj * esy, ehz, m0, out);
+    };
+    // the rows of a pair lie in one coarse row (j, or i in a planar level, is even)
+    T eo[W];
+#pragma unroll
+    for (int q = 0; q < W; ++q) eo[q] = T(0);
+    const bool walls = !perz || !perp || (DIM == 3 && !perx);
+    if (RED || (BLACK && (walls || !W1))) coarse(i >> 1, j >> 1, eo);
+    T o[R][W], xe[R][W], xw[R][W], yl[W], yr[W], c[R][W], z[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int q = 0; q < W; ++q) {
+            o[r][q] = VT::get(ov[r], q);
+            xe[r][q] = VT::get(ev[r], q);
+            xw[r][q] = VT::get(wv[r], q);
+            c[r][q] = VT::get(cv[r], q);
+        }
 #pragma unroll
     for (int q = 0; q < W; ++q) {
-        Stencil<T, DIM> s;
-        s.c = c[q];
-        s.xE = xe[q];
-        s.xW = xw[q];
-        if (DIM == 3) {
-            s.yN = yn[q];
-            s.yS = ys[q];
-        }
-        if (h == 0) {
-            s.zB = q > 0 ? o[q - 1] : zlo0;
-            s.zT = o[q];
-        } else {
-            s.zB = o[q];
-            s.zT = q < W - 1 ? o[q + 1] : zhi_last;
-        }
-        r[q] = sor_quot<T, DIM>(s, c2x, c1x, c2y, c1y, VT::get(c2v, q), VT::get(c1v, q), VT::get(bv, q), w);
-        zero = zero || r[q] == T(0);
+        yl[q] = VT::get(plv, q);
+        yr[q] = VT::get(prv, q);
     }
-    if (W1 && zero && !need_c) {
-        // a zero quotient takes the sign of (1 - w) x + q: read the cells now
-        V lv{};
-        if (!Z) lv = *reinterpret_cast<const V *>(x + own);
-        if (PRO && !evo_now) coarse_vec(e, ebase, ehz, m0, evo);
+    if (RED) {
+        // every cell read is e + x; one of the x rows, and in a row pair both y
+        // rows, lie in another coarse row
+        T el[W], er[W], eq[W];
+        const int lp = inl ? p0 - 1 : (perp ? np - 1 : p0), rp = inr ? p0 + R : (perp ? 0 : p0 + R - 1);
+        coarse(DIM == 3 ? i >> 1 : lp >> 1, DIM == 3 ? lp >> 1 : 0, el);
+        coarse(DIM == 3 ? i >> 1 : rp >> 1, DIM == 3 ? rp >> 1 : 0, er);
+        const int ie = ine ? i + 1 : (perx ? 0 : i), iw = inw ? i - 1 : (perx ? nx - 1 : i);
+        // i even: x+ lies in the cell's coarse row; i odd: x- does (an even extent's wrap: i = n - 1 and 0)
+        const bool eshare = (ie >> 1) == (i >> 1), wshare = (iw >> 1) == (i >> 1);
+        if (DIM == 3) coarse(eshare ? iw >> 1 : ie >> 1, j >> 1, eq);
 #pragma unroll
-        for (int q = 0; q < W; ++q) c[q] = PRO ? evo[q] + VT::get(lv, q) : VT::get(lv, q);
+        for (int q = 0; q < W; ++q) {
+            yl[q] = el[q] + yl[q];
+            yr[q] = er[q] + yr[q];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                o[r][q] = eo[q] + o[r][q];
+                c[r][q] = eo[q] + c[r][q];
+                if (DIM == 3) {
+                    xe[r][q] = (eshare ? eo[q] : eq[q]) + xe[r][q];
+                    xw[r][q] = (wshare ? eo[q] : eq[q]) + xw[r][q];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int h = h0 ^ (r & 1);
+            const int kz = zend[r] ? (perz ? (h ? 0 : half - 1) : (h ? m0 + W - 1 : m0)) : (h ? m0 + W : m0 - 1);
+            if (zend[r] || lane == (h ? 63 : 0)) zx[r] = coarse_at(e, (long)(i >> 1) * esx + (long)(j >> 1) * esy, ehz, kz) + zx[r];
+        }
+    }
+    if (BLACK && (walls || !W1)) {
+        // the cells' own values, which walls and (1 - w) x read
+#pragma unroll
+        for (int q = 0; q < W; ++q) {
+            if (!inl && !perp) yl[q] = eo[q] + yl[q];
+            if (!inr && !perp) yr[q] = eo[q] + yr[q];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                c[r][q] = eo[q] + c[r][q];
+                if (DIM == 3 && !ine && !perx) xe[r][q] = eo[q] + xe[r][q];
+                if (DIM == 3 && !inw && !perx) xw[r][q] = eo[q] + xw[r][q];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (zend[r] && !perz) zx[r] = ((h0 ^ (r & 1)) ? eo[W - 1] : eo[0]) + zx[r];
+    }
+    // ---- wall rules ----
+    auto flip = [&](bool wall, int bc, T v) __attribute__((always_inline)) { return wall && bc == BC_DIR ? -v : v; };
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+        yl[q] = flip(!inl, L.bc_lo[AP], yl[q]);
+        yr[q] = flip(!inr, L.bc_hi[AP], yr[q]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (DIM == 3) {
+                xe[r][q] = flip(!ine, L.bc_hi[0], xe[r][q]);
+                xw[r][q] = flip(!inw, L.bc_lo[0], xw[r][q]);
+            }
+        }
     }
 #pragma unroll
-    for (int q = 0; q < W; ++q)
-        if (!W1 || r[q] == T(0)) r[q] = (T(1.0) - w) * c[q] + r[q];
-    *reinterpret_cast<V *>(x + own) = VT::make(r);
-    if (Z) *reinterpret_cast<V *>(x + oth) = V{};
-}
-
-template <typename T, int DIM, bool FINE, bool PRO, bool W1, bool Z = false>
-__global__ void __launch_bounds__(kSplitThreads) k_rb_split(LevelArgs<T> L, T *__restrict__ x,
-                                                            const T *__restrict__ b, int colour, T w, int nblocks,
-                                                            const T *__restrict__ e, long esx, long esy, long ehz) {
-    rb_split_body<T, DIM, PRO, false, W1, Z>(L, x, b, colour, w, nblocks, e, esx, esy, ehz);
-}
-
-template <typename T, int DIM, bool FINE, bool PRO, bool W1, bool Z = false>
-__global__ void __launch_bounds__(kSplitThreads) k_rb_split_zp(LevelArgs<T> L, T *__restrict__ x,
-                                                               const T *__restrict__ b, int colour, T w, int nblocks,
-                                                               const T *__restrict__ e, long esx, long esy, long ehz) {
-    rb_split_body<T, DIM, PRO, true, W1, Z>(L, x, b, colour, w, nblocks, e, esx, esy, ehz);
+    for (int r = 0; r < R; ++r) {
+        const int h = h0 ^ (r & 1);
+        const T edge = flip(zend[r], h ? L.bc_hi[2] : L.bc_lo[2], zx[r]);
+        // the adjacent lane's value where it holds the same row
+        const T prev = __shfl_up(o[r][W - 1], 1, 64), next = __shfl_down(o[r][0], 1, 64);
+        z[r] = zend[r] || lane == (h ? 63 : 0) ? edge : (h ? next : prev);
+    }
+    if (GEN) {
+        // inhomogeneous walls: 2 w - x (bc_value)
+        const int nz = L.n[2];
+#pragma unroll
+        for (int q = 0; q < W; ++q) {
+            const int k = 2 * (m0 + q) + h0;
+            const T own_c = c[0][q];
+            if (DIM == 3) {
+                if (!ine && L.bc_hi[0] == BC_DIRV) xe[0][q] = bc_value(BC_DIRV, own_c, T(0), L.wall[0][(j + 1) * (nz + 2) + k + 1]);
+                if (!inw && L.bc_lo[0] == BC_DIRV) xw[0][q] = bc_value(BC_DIRV, own_c, T(0), L.wall[0][(j + 1) * (nz + 2) + k + 1]);
+                if (!inr && L.bc_hi[1] == BC_DIRV) yr[q] = bc_value(BC_DIRV, own_c, T(0), L.wall[1][(i + 1) * (nz + 2) + k + 1]);
+                if (!inl && L.bc_lo[1] == BC_DIRV) yl[q] = bc_value(BC_DIRV, own_c, T(0), L.wall[1][(i + 1) * (nz + 2) + k + 1]);
+            } else {
+                if (!inr && L.bc_hi[0] == BC_DIRV) yr[q] = bc_value(BC_DIRV, own_c, T(0), L.wall[0][k + 1]);
+                if (!inl && L.bc_lo[0] == BC_DIRV) yl[q] = bc_value(BC_DIRV, own_c, T(0), L.wall[0][k + 1]);
+            }
+        }
+        const T zw = (zend[0] && (h0 ? L.bc_hi[2] : L.bc_lo[2]) == BC_DIRV)
+                         ? (DIM == 3 ? L.wall[2][(i + 1) * (ny + 2) + j + 1] : L.wall[2][i + 1])
+                         : T(0);
+        if (zend[0] && (h0 ? L.bc_hi[2] : L.bc_lo[2]) == BC_DIRV) z[0] = bc_value(BC_DIRV, h0 ? c[0][W - 1] : c[0][0], T(0), zw);
+    }
+    // ---- the updates ----
+    const T dinv = UNI ? sor_inv(sor_den<T, DIM>(c2x, c2y[0], c2z[0][0])) : T(0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int h = h0 ^ (r & 1);
+        T out[W];
+        bool zero = false;
+#pragma unroll
+        for (int q = 0; q < W; ++q) {
+            Stencil<T, DIM> s;
+            // along P: the neighbour rows, within the pair the other row's other-colour vector
+            const T lo = r > 0 ? o[r > 0 ? r - 1 : 0][q] : yl[q], hi = r < R - 1 ? o[r < R - 1 ? r + 1 : r][q] : yr[q];
+            s.c = c[r][q];
+            if (DIM == 3) {
+                s.xE = xe[r][q];
+                s.xW = xw[r][q];
+                s.yN = hi;
+                s.yS = lo;
+            } else {
+                s.xE = hi;
+                s.xW = lo;
+            }
+            s.zB = h ? o[r][q] : (q > 0 ? o[r][q > 0 ? q - 1 : 0] : z[r]);
+            s.zT = h ? (q < W - 1 ? o[r][q < W - 1 ? q + 1 : q] : z[r]) : o[r][q];
+            const T num = sor_num<T, DIM>(s, c2r[r], c1r[r], c2y[r], c1y[r], c2z[r][q], c1z[r][q], VT::get(bv[r], q), w);
+            out[q] = UNI ? sor_quot_inv(num, dinv) : sor_div(num, sor_den<T, DIM>(c2r[r], c2y[r], c2z[r][q]));
+            zero = zero || out[q] == T(0);
+        }
+        if (W1 && zero) {
+            // a zero quotient takes the sign of (1 - w) x + q: read the cells now
+            V lv{};
+            if (!ZERO) lv = xv(own[r]);
+            if (BLACK && !walls) coarse(i >> 1, j >> 1, eo);
+#pragma unroll
+            for (int q = 0; q < W; ++q) c[r][q] = RED || BLACK ? eo[q] + VT::get(lv, q) : VT::get(lv, q);
+        }
+#pragma unroll
+        for (int q = 0; q < W; ++q)
+            if (!W1 || out[q] == T(0)) out[q] = (T(1.0) - w) * c[r][q] + out[q];
+        *reinterpret_cast<V *>(reinterpret_cast<char *>(x) + own[r]) = VT::make(out);
+        if (ZERO) *reinterpret_cast<V *>(reinterpret_cast<char *>(x) + oth[r]) = V{};
+    }
 }
 
 // ---------------------------------------------------------------------------
