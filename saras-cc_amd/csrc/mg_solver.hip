@@ -637,11 +637,10 @@ struct Ops {
     }
 
     // One colour pass of a split level.  The paired form (k_rb_split with R = 2)
-    // takes levels whose rows pair up along y (x in a planar level), whose
-    // arrays 32-bit byte offsets reach and whose walls are homogeneous -- every
-    // level but a DIRICHLET_TEST level 0, odd row counts (a coarsest level's
-    // parent has even ones) and FP64 arrays of 4 GB and more, which the
-    // general form takes.
+    // takes levels whose rows pair up along y (x in a planar level) and whose
+    // walls are homogeneous -- every level but a DIRICHLET_TEST level 0 (the
+    // levels above the coarsest have even row counts), with 64-bit offsets for
+    // arrays of 4 GB and more; the general form the rest.
     // Time of a pass, one row per lane with branches around each load / now:
     // FP32 256^3 19.6 / 16.8 us (after the prolongation: red 33 / 20, black
     // 20 / 16.4), 512^3 180 / 150 us (279 / 197, 183 / 147), tanh z 256^3 20.1 /
@@ -653,7 +652,8 @@ struct Ops {
         DevLevel<T> &L = H.lv[l];
         const int np = DIM == 3 ? L.n[1] : L.n[0];
         const bool dirv = a.bc_lo[0] == BC_DIRV || a.bc_lo[2] == BC_DIRV;
-        const bool gen = (np & 1) || L.elems * sizeof(T) > 0xffffffffull || dirv || m->rb_general;
+        const bool big = L.elems * sizeof(T) > 0xffffffffull;
+        const bool gen = (np & 1) || dirv || m->rb_general || (big && w != T(1));
         const int R = gen ? 1 : 2;
         RowMap M;
         const unsigned q = (unsigned)(L.n[2] / 2 / Vec16<T>::W);
@@ -671,13 +671,15 @@ struct Ops {
         const unsigned nb = (unsigned)((total + kSplitThreads - 1) / kSplitThreads);
         const dim3 g((nb + kXcds - 1) / kXcds * kXcds), bl(kSplitThreads);
         if (gen)
-            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, true>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, RB_GENERAL>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+        else if (big)
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, false, RB_PAIR64>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
         else if (w != T(1))
-            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, false>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, RB_PAIR>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
         else if (L.uniform)
-            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, true, false>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, true, RB_PAIR>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
         else
-            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, false, false>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
+            hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, false, RB_PAIR>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
     }
 
     template <int DIM>
@@ -769,6 +771,50 @@ struct Ops {
         for (int c = 0; c < count; ++c) rb_sweep(l, zero_bc);
     }
 
+    // Residual and restriction of a split 3-D level.  Time of a launch, one
+    // row per lane with branches around each load / now: FP32 256^3 36 / 29 us,
+    // 512^3 351 / 278 us (290 without the j-tiles); FP64 256^3 75 / 53 us.
+    template <bool RED>
+    void rr_pair(const DevLevel<T> &F, const saras::LevelArgs<T> &fa, const saras::LevelArgs<T> &ca, DevLevel<T> &C,
+                 const saras::RestrictArgs<T> &r) {
+        using namespace saras;
+        const unsigned q = (unsigned)(F.n[2] / 2 / Vec16<T>::W);
+        const size_t total = (size_t)C.n[0] * C.n[1] * q;
+        // host-side guard: task numbers stay below 2^31
+        if (total + kRrTasks * kXcds > 0x7fffffffull) {
+            refuse("a level too large for one restriction");
+            return;
+        }
+        const unsigned ntask = (unsigned)total, nb = (ntask + kRrTasks - 1) / kRrTasks;
+        const dim3 g((nb + kXcds - 1) / kXcds * kXcds), bl(kSplitThreads);
+        // The next coarse row reads two of the four x-planes again: where those
+        // and b's exceed half of an XCD's 4 MB L2, the coarse rows run in
+        // j-tiles whose share of them is 512 KB at most (a power of two that
+        // divides the rows).
+        unsigned wj = (unsigned)C.n[1];
+        const size_t plane = 4 * (size_t)F.n[2] * sizeof(T);   // of one fine row of x and b, two planes
+        if (plane * F.n[1] >= (2u << 20)) {
+            unsigned t = 1;
+            while (t < 256 && plane * 4 * t <= (512u << 10)) t *= 2;
+            while (t > 1 && C.n[1] % t) t /= 2;
+            if (t >= 4) wj = t;
+        }
+        RowMap M;
+        M.q = FastDiv::of(q);
+        M.tile = FastDiv::of((unsigned)C.n[0] * wj);
+        M.wj = FastDiv::of(wj);
+        M.total = ntask;
+        const bool dirv = fa.bc_lo[0] == BC_DIRV || fa.bc_lo[2] == BC_DIRV;
+        if (dirv || m->rb_general)
+            hipLaunchKernelGGL((k_rr_pair<T, RED, false, RB_GENERAL>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
+        else if (F.elems * sizeof(T) > 0xffffffffull)
+            hipLaunchKernelGGL((k_rr_pair<T, RED, false, RB_PAIR64>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
+        else if (F.uniform)
+            hipLaunchKernelGGL((k_rr_pair<T, RED, true, RB_PAIR>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
+        else
+            hipLaunchKernelGGL((k_rr_pair<T, RED, false, RB_PAIR>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
+    }
+
     // red_next: the restriction also applies the coarse level's first
     // pre-smoothing red pass (split levels; see k_rr_split)
     void resid_restrict(int l, bool red_next = false) {
@@ -788,17 +834,10 @@ struct Ops {
         }
         const long n = (long)C.n[0] * C.n[1] * C.n[2];
         if (F.hz && H.dim == 3 && !m->rr_lane) {
-            const long ntask = (long)C.n[0] * C.n[1] * (F.n[2] / 2 / saras::Vec16<T>::W);
-            const int nb = (int)((ntask + saras::kRrTasks - 1) / saras::kRrTasks);
-            const int grid = (nb + saras::kXcds - 1) / saras::kXcds * saras::kXcds;
             const bool red = red_next && C.hz;
             if (red) skip_red = l + 1;
-            if (red)
-                hipLaunchKernelGGL((saras::k_rr_split4<T, true>), dim3(grid), dim3(saras::kSplitThreads), 0, s, fa,
-                                   F.x, F.b, ca, C.b, C.x, r, nb, w);
-            else
-                hipLaunchKernelGGL((saras::k_rr_split4<T, false>), dim3(grid), dim3(saras::kSplitThreads), 0, s, fa,
-                                   F.x, F.b, ca, C.b, C.x, r, nb, w);
+            if (red) rr_pair<true>(F, fa, ca, C, r);
+            else rr_pair<false>(F, fa, ca, C, r);
             return;
         }
         if (F.hz) {

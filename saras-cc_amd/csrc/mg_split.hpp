@@ -156,6 +156,7 @@ struct RowMap {
 //             neighbours are the red values just written), so the separate
 //             prolongation pass is not needed.
 enum RbMode { RB_PLAIN, RB_ZERO, RB_RED, RB_BLACK };
+enum RbForm { RB_PAIR, RB_PAIR64, RB_GENERAL };
 
 // One colour pass over a split level; the grid is a multiple of kXcds blocks.
 // A lane updates one vector of each of R rows that follow one another along y
@@ -169,7 +170,8 @@ enum RbMode { RB_PLAIN, RB_ZERO, RB_RED, RB_BLACK };
 // (to give the sign the reference's sum has).
 // UNI: every axis is uniform, so the coefficients are one value per axis and
 // the divisor (FP32: its reciprocal) is formed once.
-// GEN: the general form (R = 1, any w, 64-bit offsets, inhomogeneous walls).
+// FORM: RB_PAIR; RB_PAIR64, the same with 64-bit offsets (arrays of 4 GB and
+// more); RB_GENERAL (R = 1, any w, 64-bit offsets, inhomogeneous walls).
 //
 // No load waits behind a lane-dependent branch: a neighbour beyond a wall is
 // read at the cell's own place (which is the Neumann rule) and its sign
@@ -178,14 +180,15 @@ enum RbMode { RB_PLAIN, RB_ZERO, RB_RED, RB_BLACK };
 // length are multiplications.  Issuing that arithmetic and waiting for one
 // load after another took as long as the traffic before: see the measured
 // times at Ops::rb_pass (mg_solver.hip).
-template <typename T, int DIM, int MODE, bool W1, bool UNI, bool GEN>
+template <typename T, int DIM, int MODE, bool W1, bool UNI, int FORM>
 __global__ void __launch_bounds__(kSplitThreads) k_rb_split(LevelArgs<T> L, RowMap M, T *__restrict__ x,
                                                             const T *__restrict__ b, int colour, T w,
                                                             const T *__restrict__ e, long esx, long esy, long ehz) {
+    constexpr bool GEN = FORM == RB_GENERAL;
     static_assert(!GEN || (!W1 && !UNI), "the general form takes any w and any metric");
     using VT = Vec16<T>;
     using V = typename VT::V;
-    using OFF = std::conditional_t<GEN, unsigned long, unsigned>;   // byte offset
+    using OFF = std::conditional_t<FORM != RB_PAIR, unsigned long, unsigned>;   // byte offset
     constexpr int W = VT::W, R = GEN ? 1 : 2;
     constexpr bool RED = MODE == RB_RED, BLACK = MODE == RB_BLACK, ZERO = MODE == RB_ZERO;
     const unsigned per = gridDim.x / kXcds;
@@ -658,18 +661,21 @@ __global__ void __launch_bounds__(kSplitThreads) k_rr_split(LevelArgs<T> F, cons
 }
 
 // ---------------------------------------------------------------------------
-// Residual + restriction of a split 3-D level with the eight children of a
-// coarse cell spread over the four waves of a block.  A block owns 64
-// consecutive (coarse row, vector) tasks; wave w = (di, dj) = (w / 2, w % 2)
-// computes, for every task, the residuals of fine row (2I + di, 2J + dj) at
-// the 2W fine cells under the task's W coarse cells -- whole 16-byte vectors,
-// as in a colour pass -- and leaves the products v_{di dj dk} r in LDS.  After
-// one barrier each thread adds the eight products of one coarse cell in the
+// Residual + restriction of a split 3-D level.  A task is one vector of W
+// coarse cells of a coarse row; a block owns kRrTasks of them.  A lane takes
+// the fine rows (2I + di, 2J) and (2I + di, 2J + 1) under a task -- di by wave --
+// both halves of each at the task's W fine positions, as whole 16-byte vectors
+// (each row is the other's y neighbour: 20 vectors for the pair where single
+// rows load 32), and leaves the products v_{di dj dk} r in LDS.  After one
+// barrier each thread adds the eight products of one coarse cell in the
 // reference's order and divides by the volume (poisson_d3.cc:494-511).  Every
-// product and partial sum is the same rounding as in the one-lane form, so
-// the values are identical.  RED as in k_rr_split.
+// product and partial sum is the same rounding as in the one-lane form, so the
+// values are identical.  RED as in k_rr_split; UNI, FORM and the form of the
+// loads as in k_rb_split.
+// Measured per launch, one row per lane with branches around each load / now:
+// see Ops::resid_restrict (mg_solver.hip).
 // ---------------------------------------------------------------------------
-constexpr int kRrTasks = 64;
+constexpr int kRrTasks = 128;
 
 // position of v_{di dj dk} r_{di dj dk} in the reference's sum
 // v111 r111 + v000 r000 + v110 r110 + v001 r001 + v101 r101 + v010 r010 + v011 r011 + v100 r100
@@ -686,148 +692,158 @@ __device__ __forceinline__ int rr_slot(int di, int dj, int dk) {
     }
 }
 
-template <typename T, bool RED>
-__global__ void __launch_bounds__(kSplitThreads) k_rr_split4(LevelArgs<T> F, const T *__restrict__ x,
-                                                             const T *__restrict__ b, LevelArgs<T> C,
-                                                             T *__restrict__ bc, T *__restrict__ xc, RestrictArgs<T> R,
-                                                             int nblocks, T w) {
+template <typename T, bool RED, bool UNI, int FORM>
+__global__ void __launch_bounds__(kSplitThreads) k_rr_pair(LevelArgs<T> F, const T *__restrict__ x,
+                                                           const T *__restrict__ b, LevelArgs<T> C,
+                                                           T *__restrict__ bc, T *__restrict__ xc, RestrictArgs<T> R,
+                                                           RowMap M, T w) {
     using VT = Vec16<T>;
+    using V = typename VT::V;
+    using OFF = std::conditional_t<FORM != RB_PAIR, unsigned long, unsigned>;   // byte offset
     constexpr int W = VT::W;
     __shared__ __align__(16) T prod[8][kRrTasks * W];
-    const int per = gridDim.x / kXcds;
-    const int logical = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
-    if (logical >= nblocks) return;
-    const int nx = F.n[0], ny = F.n[1], nz = F.n[2];
-    const int half = nz >> 1, q = half / W;
-    const int cy = C.n[1];
-    const long ntask = (long)C.n[0] * cy * q;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int di = wave >> 1, dj = wave & 1;
-    const long task = (long)logical * kRrTasks + lane;
+    const unsigned per = gridDim.x / kXcds;
+    const unsigned logical = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
+    const unsigned ntask = M.total;
+    if (logical * kRrTasks >= ntask) return;
+    // coarse row and first coarse cell of a task
+    auto place = [&](unsigned tk, int &I, int &J, int &K) __attribute__((always_inline)) {
+        const unsigned g = M.q.div(tk), tile = M.tile.div(g), rem = g - tile * M.tile.d, gi = M.wj.div(rem);
+        I = (int)gi;
+        J = (int)(tile * M.wj.d + rem - gi * M.wj.d);
+        K = (int)(tk - g * M.q.d) * W;
+    };
+    const int nx = F.n[0], ny = F.n[1], nz = F.n[2], half = nz >> 1;
+    const int lane = threadIdx.x & 63, di = threadIdx.x >> 7, slot = threadIdx.x & 127;
+    const unsigned task = logical * kRrTasks + slot;
     const bool live = task < ntask;
-    const long hz = F.hz;
-
-    int I = 0, J = 0, K0 = 0, i = 0, j = 0;
-    long rb = 0;
-    T xe[W], xo[W], zl = T(0), zh = T(0);
-    for (int e = 0; e < W; ++e) xe[e] = xo[e] = T(0);
-    if (live) {
-        const long crow = task / q;
-        const int v = (int)(task - crow * q);
-        I = (int)(crow / cy);
-        J = (int)(crow - (long)I * cy);
-        K0 = v * W;
-        i = 2 * I + di;
-        j = 2 * J + dj;
-        rb = (long)i * F.sx + (long)j * F.sy;
-        load_n<T, W>(x + rb + K0, xe);
-        load_n<T, W>(x + rb + hz + K0, xo);
-        // z neighbours no adjacent lane holds, loaded with the row vectors
-        if (K0 == 0 ? F.bc_lo[2] == BC_PER : lane == 0) zl = K0 == 0 ? x[rb + hz + (half - 1)] : x[rb + hz + K0 - 1];
-        if (K0 + W == half ? F.bc_hi[2] == BC_PER : lane == 63) zh = K0 + W == half ? x[rb] : x[rb + K0 + W];
+    const unsigned tt = live ? task : ntask - 1;   // a lane without a task repeats the last one, unread
+    int I, J, K0;
+    place(tt, I, J, K0);
+    const int i = 2 * I + di, j = 2 * J;
+    const OFF sx = (OFF)F.sx * sizeof(T), sy = (OFF)F.sy * sizeof(T), hz = (OFF)F.hz * sizeof(T);
+    const OFF r0 = (OFF)i * sx + (OFF)j * sy, ko = (OFF)K0 * sizeof(T);
+    const bool perx = F.bc_lo[0] == BC_PER, pery = F.bc_lo[1] == BC_PER, perz = F.bc_lo[2] == BC_PER;
+    const bool ine = i + 1 < nx, inw = i > 0, inn = j + 2 < ny, ins = j > 0;
+    const OFF de = ine ? sx : (perx ? (OFF)0 - (OFF)(nx - 1) * sx : (OFF)0);
+    const OFF dw = inw ? (OFF)0 - sx : (perx ? (OFF)(nx - 1) * sx : (OFF)0);
+    // the rows beyond the pair: row j - 1 of row j, row j + 2 of row j + 1
+    const OFF ps = ins ? (OFF)0 - sy : (pery ? (OFF)(ny - 1) * sy : (OFF)0);
+    const OFF pn = (inn ? sy : (pery ? (OFF)0 - (OFF)(ny - 1) * sy : (OFF)0)) + sy;
+    auto ldv = [](const T *p, OFF o) __attribute__((always_inline)) {
+        return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + o);
+    };
+    auto ld = [](const T *p, OFF o) __attribute__((always_inline)) {
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + o);
+    };
+    // ---- loads: [row of the pair][half] ----
+    V xv[2][2], bv[2][2], ev[2][2], wv[2][2], sv[2], nv[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const OFF o = r0 + ko + (h ? hz : 0);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            xv[r][h] = ldv(x, o + (r ? sy : 0));
+            ev[r][h] = ldv(x, o + (r ? sy : 0) + de);
+            wv[r][h] = ldv(x, o + (r ? sy : 0) + dw);
+            bv[r][h] = ldv(b, o + (r ? sy : 0));
+        }
+        sv[h] = ldv(x, o + ps);
+        nv[h] = ldv(x, o + pn);
     }
-    // cross-vector z neighbours from the adjacent lanes (all lanes take part;
-    // a live lane's predecessor is live, and a live lane whose successor is
-    // not ends its row, where the boundary rule applies instead)
-    const T from_prev = __shfl_up(xo[W - 1], 1, 64);
-    const T from_next = __shfl_down(xe[0], 1, 64);
-    if (live) {
-        T be[W], bo[W], cz2e[W], cz1e[W], cz2o[W], cz1o[W];
-        load_n<T, W>(b + rb + K0, be);
-        load_n<T, W>(b + rb + hz + K0, bo);
-        load_n<T, W>(F.c2zs + K0, cz2e);
-        load_n<T, W>(F.c1zs + K0, cz1e);
-        load_n<T, W>(F.c2zs + half + K0, cz2o);
-        load_n<T, W>(F.c1zs + half + K0, cz1o);
-        // neighbour rows: [0] E, [1] W, [2] N, [3] S; even and odd halves
-        T ne[4][W], no[4][W];
-        auto nbr = [&](int slot, bool inside, long off, int bcode, int axis) {
-            if (inside || bcode == BC_PER) {
-                load_n<T, W>(x + rb + off + K0, ne[slot]);
-                load_n<T, W>(x + rb + off + hz + K0, no[slot]);
-            } else {
+    // z neighbours no adjacent lane holds: below the first even cell and above the last odd one
+    const bool zlo = K0 == 0, zhi = K0 + W == half;
+    T zl[2], zh[2];
 #pragma unroll
-                for (int e = 0; e < W; ++e) {
-                    T wve = T(0), wvo = T(0);
-                    if (bcode == BC_DIRV) {
-                        const int ke = 2 * (K0 + e), ko = ke + 1;
-                        if (axis == 0) {
-                            wve = F.wall[0][(j + 1) * (nz + 2) + ke + 1];
-                            wvo = F.wall[0][(j + 1) * (nz + 2) + ko + 1];
-                        } else {
-                            wve = F.wall[1][(i + 1) * (nz + 2) + ke + 1];
-                            wvo = F.wall[1][(i + 1) * (nz + 2) + ko + 1];
-                        }
-                    }
-                    ne[slot][e] = bc_value(bcode, xe[e], T(0), wve);
-                    no[slot][e] = bc_value(bcode, xo[e], T(0), wvo);
+    for (int r = 0; r < 2; ++r) {
+        const OFF row = r0 + (r ? sy : 0);
+        zl[r] = zh[r] = T(0);
+        if (zlo || lane == 0)
+            zl[r] = ld(x, zlo ? (perz ? row + hz + (OFF)(half - 1) * sizeof(T) : row + ko) : row + hz + ko - sizeof(T));
+        if (zhi || lane == 63)
+            zh[r] = ld(x, zhi ? (perz ? row : row + hz + ko + (W - 1) * sizeof(T)) : row + ko + W * sizeof(T));
+    }
+    T c2z[2][W], c1z[2][W], c2y[2], c1y[2];
+    const T c2x = F.c2[0][UNI ? 0 : i], c1x = F.c1[0][UNI ? 0 : i];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        c2y[r] = F.c2[1][UNI ? 0 : j + r];
+        c1y[r] = F.c1[1][UNI ? 0 : j + r];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if constexpr (UNI) {
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                c2z[h][q] = F.c2[2][0];
+                c1z[h][q] = F.c1[2][0];
+            }
+        } else {
+            load_n<T, W>(F.c2zs + h * half + K0, c2z[h]);
+            load_n<T, W>(F.c1zs + h * half + K0, c1z[h]);
+        }
+    }
+    const T ax = di ? R.hi[0][I] : R.lo[0][I], ay[2] = {R.lo[1][J], R.hi[1][J]};
+    T fz[2][W];
+    load_n<T, W>(R.lo[2] + K0, fz[0]);
+    load_n<T, W>(R.hi[2] + K0, fz[1]);
+    // ---- residuals ----
+    auto flip = [](bool wall, int code, T v) __attribute__((always_inline)) { return wall && code == BC_DIR ? -v : v; };
+    T xs[2][2][W];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < W; ++q) xs[r][h][q] = VT::get(xv[r][h], q);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        // cross-vector z neighbours: the adjacent lanes', or the loaded ones
+        const T prev = __shfl_up(xs[r][1][W - 1], 1, 64), next = __shfl_down(xs[r][0][0], 1, 64);
+        T zb = zlo || lane == 0 ? flip(zlo, F.bc_lo[2], zl[r]) : prev;
+        T zt = zhi || lane == 63 ? flip(zhi, F.bc_hi[2], zh[r]) : next;
+        if (FORM == RB_GENERAL) {
+            const T wz = F.bc_lo[2] == BC_DIRV ? F.wall[2][(i + 1) * (ny + 2) + j + r + 1] : T(0);
+            if (zlo && F.bc_lo[2] == BC_DIRV) zb = bc_value(BC_DIRV, xs[r][0][0], T(0), wz);
+            if (zhi && F.bc_hi[2] == BC_DIRV) zt = bc_value(BC_DIRV, xs[r][1][W - 1], T(0), wz);
+        }
+        const T axy = ax * ay[r];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            T p[W];
+#pragma unroll
+            for (int q = 0; q < W; ++q) {
+                Stencil<T, 3> s;
+                s.c = xs[r][h][q];
+                s.xE = flip(!ine, F.bc_hi[0], VT::get(ev[r][h], q));
+                s.xW = flip(!inw, F.bc_lo[0], VT::get(wv[r][h], q));
+                s.yN = r == 0 ? xs[1][h][q] : flip(!inn, F.bc_hi[1], VT::get(nv[h], q));
+                s.yS = r == 1 ? xs[0][h][q] : flip(!ins, F.bc_lo[1], VT::get(sv[h], q));
+                s.zB = h ? xs[r][0][q] : (q > 0 ? xs[r][1][q > 0 ? q - 1 : 0] : zb);
+                s.zT = h ? (q < W - 1 ? xs[r][0][q < W - 1 ? q + 1 : q] : zt) : xs[r][1][q];
+                if (FORM == RB_GENERAL) {
+                    const int k = 2 * (K0 + q) + h;
+                    if (!ine && F.bc_hi[0] == BC_DIRV) s.xE = bc_value(BC_DIRV, s.c, T(0), F.wall[0][(j + r + 1) * (nz + 2) + k + 1]);
+                    if (!inw && F.bc_lo[0] == BC_DIRV) s.xW = bc_value(BC_DIRV, s.c, T(0), F.wall[0][(j + r + 1) * (nz + 2) + k + 1]);
+                    if (r == 1 && !inn && F.bc_hi[1] == BC_DIRV) s.yN = bc_value(BC_DIRV, s.c, T(0), F.wall[1][(i + 1) * (nz + 2) + k + 1]);
+                    if (r == 0 && !ins && F.bc_lo[1] == BC_DIRV) s.yS = bc_value(BC_DIRV, s.c, T(0), F.wall[1][(i + 1) * (nz + 2) + k + 1]);
                 }
+                const T d = residual<T, 3>(s, c2x, c1x, c2y[r], c1y[r], c2z[h][q], c1z[h][q], VT::get(bv[r][h], q));
+                p[q] = (axy * fz[h][q]) * d;
             }
-        };
-        nbr(0, i + 1 < nx, i + 1 < nx ? F.sx : -(long)(nx - 1) * F.sx, F.bc_hi[0], 0);
-        nbr(1, i > 0, i > 0 ? -F.sx : (long)(nx - 1) * F.sx, F.bc_lo[0], 0);
-        nbr(2, j + 1 < ny, j + 1 < ny ? F.sy : -(long)(ny - 1) * F.sy, F.bc_hi[1], 1);
-        nbr(3, j > 0, j > 0 ? -F.sy : (long)(ny - 1) * F.sy, F.bc_lo[1], 1);
-        // z: even cell 2K has zB = odd[K-1], zT = odd[K]; odd cell has zB = even[K], zT = even[K+1]
-        T zlo0, zhi_last;
-        if (K0 == 0) {
-            if (F.bc_lo[2] == BC_PER) zlo0 = zl;
-            else {
-                const T wv = F.bc_lo[2] == BC_DIRV ? F.wall[2][(i + 1) * (ny + 2) + j + 1] : T(0);
-                zlo0 = bc_value(F.bc_lo[2], xe[0], T(0), wv);
-            }
-        } else {
-            zlo0 = lane > 0 ? from_prev : zl;
+            *reinterpret_cast<V *>(&prod[rr_slot(di, r, h)][slot * W]) = VT::make(p);
         }
-        if (K0 + W == half) {
-            if (F.bc_hi[2] == BC_PER) zhi_last = zh;
-            else {
-                const T wv = F.bc_hi[2] == BC_DIRV ? F.wall[2][(i + 1) * (ny + 2) + j + 1] : T(0);
-                zhi_last = bc_value(F.bc_hi[2], xo[W - 1], T(0), wv);
-            }
-        } else {
-            zhi_last = lane < 63 ? from_next : zh;
-        }
-        const T c2x = F.c2[0][i], c1x = F.c1[0][i], c2y = F.c2[1][j], c1y = F.c1[1][j];
-        const T ax = di ? R.hi[0][I] : R.lo[0][I], ay = dj ? R.hi[1][J] : R.lo[1][J];
-        const T axy = ax * ay;
-        T lz[W], hzf[W];
-        load_n<T, W>(R.lo[2] + K0, lz);
-        load_n<T, W>(R.hi[2] + K0, hzf);
-        T p0[W], p1[W];
-#pragma unroll
-        for (int e = 0; e < W; ++e) {
-            Stencil<T, 3> s;
-            s.c = xe[e];
-            s.xE = ne[0][e];
-            s.xW = ne[1][e];
-            s.yN = ne[2][e];
-            s.yS = ne[3][e];
-            s.zB = e > 0 ? xo[e - 1] : zlo0;
-            s.zT = xo[e];
-            const T r0 = residual<T, 3>(s, c2x, c1x, c2y, c1y, cz2e[e], cz1e[e], be[e]);
-            s.c = xo[e];
-            s.xE = no[0][e];
-            s.xW = no[1][e];
-            s.yN = no[2][e];
-            s.yS = no[3][e];
-            s.zB = xe[e];
-            s.zT = e < W - 1 ? xe[e + 1] : zhi_last;
-            const T r1 = residual<T, 3>(s, c2x, c1x, c2y, c1y, cz2o[e], cz1o[e], bo[e]);
-            p0[e] = (axy * lz[e]) * r0;
-            p1[e] = (axy * hzf[e]) * r1;
-        }
-        *reinterpret_cast<typename VT::V *>(&prod[rr_slot(di, dj, 0)][lane * W]) = VT::make(p0);
-        *reinterpret_cast<typename VT::V *>(&prod[rr_slot(di, dj, 1)][lane * W]) = VT::make(p1);
     }
     __syncthreads();
-    for (int c = threadIdx.x; c < kRrTasks * W; c += blockDim.x) {
-        const long tk = (long)logical * kRrTasks + c / W;
+    // ---- sums: coarse cell c of the block's tasks ----
+#pragma unroll
+    for (int u = 0; u < kRrTasks * W / kSplitThreads; ++u) {
+        const int c = threadIdx.x + u * kSplitThreads;
+        const unsigned tk = logical * kRrTasks + c / W;
         if (tk >= ntask) continue;
-        const long crow = tk / q;
-        const int v = (int)(tk - crow * q);
-        const int CI = (int)(crow / cy), CJ = (int)(crow - (long)CI * cy);
-        const int K = v * W + c % W;
+        int CI, CJ, K;
+        place(tk, CI, CJ, K);
+        K += c % W;
         T sum = prod[0][c] + prod[1][c];
         sum = sum + prod[2][c];
         sum = sum + prod[3][c];
