@@ -1091,13 +1091,60 @@ saras_status run_vcycle(saras_mg *m, Ops<T> &ops) {
     return SARAS_OK;
 }
 
+// Whether the FP64 residual passes of level 0 take k_refine_march: split rows,
+// homogeneous walls, and arrays (the caller's padded one the largest) and
+// vector numbers within 32 bits.
+bool refine_marches(const saras_mg *m, const saras::LevelArgs<double> &a) {
+    const size_t full = (size_t)(a.n[0] + 2 * m->g.pad) * (a.n[1] + 2 * m->g.pad) * (a.n[2] + 2 * m->g.pad) * 8;
+    const size_t own = (size_t)a.sx * a.n[0] * 8, vecs = (size_t)a.n[0] * a.n[1] * (a.n[2] / 4);
+    return a.hz && a.bc_lo[0] != saras::BC_DIRV && a.bc_lo[2] != saras::BC_DIRV && std::max(full, own) <= 0xffffffffull &&
+           vecs + saras::kNormBlocks * saras::kNormThreads <= 0x7fffffffull && !m->rb_general;
+}
+
+// One FP64 residual pass (see k_refine_split for what the flags mean).  Times,
+// k_refine_split / k_refine_march (us), 256^3 and 512^3: the norm alone 63 / 44
+// (6.1 TB/s) at 256^3; the initial residual of a mixed solve 104 / 75, 914 / 658;
+// the refinement from the caller's iterate 144 / 114, 1235 / 944, between
+// split arrays 142 / 113, 1193 / 928, into the caller's iterate 166 / 126,
+// 1414 / 1010.  (Issuing all loads of k_refine_split first, without the march,
+// gave 133 and 1240 for the third: its re-reads bound it.)
+template <int TYPE, int DIM, bool NORM_ONLY, bool E, bool CX, bool CB, bool CXO, bool NOXW>
+void launch_refine_march(saras_mg *m, const saras::LevelArgs<double> &a, const double *x, const float *e, long esx,
+                        long esy, long ehz, const double *b, float *r32, const saras::FullRows &fr, hipStream_t s) {
+    using namespace saras;
+    MarchMap M;
+    const unsigned q = (unsigned)(a.n[2] / 4);
+    M.plane = (DIM == 3 ? (unsigned)a.n[1] : 1u) * q;
+    const unsigned pb = (M.plane + kNormThreads - 1) / kNormThreads;
+    // as many chunks of planes as there are blocks for: a chunk reads two
+    // planes more than it owns, but on the levels where chunks get that short
+    // (single planes up to about 160 x 64 x 96) the pass is bound by latency
+    const unsigned chunks = std::max(1u, std::min((unsigned)kNormBlocks / std::min(pb, (unsigned)kNormBlocks), (unsigned)a.n[0]));
+    M.len = (int)((a.n[0] + chunks - 1) / chunks);
+    M.q = FastDiv::of(q);
+    M.pb = FastDiv::of(pb);
+    M.items = pb * (unsigned)((a.n[0] + M.len - 1) / M.len);
+    const dim3 g(kNormBlocks), bl(kNormThreads);
+    if (TYPE == 0 && m->h64.lv[0].uniform)
+        hipLaunchKernelGGL((k_refine_march<TYPE, DIM, NORM_ONLY, E, CX, CB, CXO, NOXW, TYPE == 0>), g, bl, 0, s, a, M, x, e,
+                           esx, esy, ehz, b, m->x64b, r32, m->partial, fr);
+    else
+        hipLaunchKernelGGL((k_refine_march<TYPE, DIM, NORM_ONLY, E, CX, CB, CXO, NOXW, false>), g, bl, 0, s, a, M, x, e, esx,
+                           esy, ehz, b, m->x64b, r32, m->partial, fr);
+}
+
 template <int DIM>
 void launch_norm(int type, saras_mg *m, const saras::LevelArgs<double> &a, const double *x, const double *b,
                  hipStream_t s) {
     if (a.hz) {
         // split rows: the vectorised residual pass, norms only
         const unsigned nb = saras::kNormBlocks, nt = saras::kNormThreads;
-        if (type == 0)
+        const saras::FullRows none{};
+        if (refine_marches(m, a)) {
+            if (type == 0) launch_refine_march<0, DIM, true, false, false, false, false, false>(m, a, x, nullptr, 0, 0, 0, b, nullptr, none, s);
+            else if (type == 1) launch_refine_march<1, DIM, true, false, false, false, false, false>(m, a, x, nullptr, 0, 0, 0, b, nullptr, none, s);
+            else launch_refine_march<2, DIM, true, false, false, false, false, false>(m, a, x, nullptr, 0, 0, 0, b, nullptr, none, s);
+        } else if (type == 0)
             hipLaunchKernelGGL((saras::k_refine_split<0, DIM, true>), dim3(nb), dim3(nt), 0, s, a, x, nullptr, 0L, 0L,
                                0L, b, nullptr, nullptr, m->partial, saras::FullRows{});
         else if (type == 1)
@@ -1440,8 +1487,14 @@ void launch_refine_split(saras_mg *m, const saras::LevelArgs<double> &a, const f
                          float *r32, const saras::FullRows &fr, hipStream_t s) {
     auto &L0 = m->h64.lv[0];
     const unsigned nb = saras::kNormBlocks, nt = saras::kNormThreads;
-    hipLaunchKernelGGL((saras::k_refine_split<TYPE, DIM, false, CX, CB, CXO, NOXW>), dim3(nb), dim3(nt), 0, s, a,
-                       L0.x, e, esx, esy, ehz, L0.b, m->x64b, r32, m->partial, fr);
+    if (refine_marches(m, a)) {
+        if (e && !NOXW)
+            launch_refine_march<TYPE, DIM, false, !NOXW, CX, CB, CXO, NOXW>(m, a, L0.x, e, esx, esy, ehz, L0.b, r32, fr, s);
+        else
+            launch_refine_march<TYPE, DIM, false, false, CX, CB, CXO, NOXW>(m, a, L0.x, nullptr, esx, esy, ehz, L0.b, r32, fr, s);
+    } else
+        hipLaunchKernelGGL((saras::k_refine_split<TYPE, DIM, false, CX, CB, CXO, NOXW>), dim3(nb), dim3(nt), 0, s, a,
+                           L0.x, e, esx, esy, ehz, L0.b, m->x64b, r32, m->partial, fr);
     hipLaunchKernelGGL((saras::k_norm_final<TYPE>), dim3(1), dim3(nt), 0, s, m->partial, saras::kNormBlocks,
                        m->norm_host, m->norm_seq, ++m->norm_ticket);
 }

@@ -1184,4 +1184,226 @@ __global__ void __launch_bounds__(kNormThreads) k_refine_split(LevelArgs<double>
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_refine_split for the levels it mostly meets: homogeneous walls and arrays
+// below 4 GB.  The same values and the same norms.  Bound by memory: walking
+// the rows in order, each plane was read again for its x neighbours from
+// beyond L2 (1.3 to 2 times the words a pass cannot do without).  Here a lane
+// keeps its place in the (y, z) plane -- W positions of both halves of a row --
+// and marches along x through one chunk of planes, with the plane behind and
+// its own in registers, so a plane is read once; its y neighbours are read by
+// the blocks beside it at about the same time, on the same XCD.  E: with a
+// correction; UNI: every axis uniform, so the coefficients are one value per
+// axis; loads do not wait behind a lane-dependent branch, byte offsets have 32
+// bits.  Measured: see launch_refine_march (mg_solver.hip).
+// ---------------------------------------------------------------------------
+// two doubles of a caller's row, whose start need not be 16-byte aligned (a
+// 16-byte global access needs 4-byte alignment only)
+typedef double double2u __attribute__((ext_vector_type(2), aligned(8)));
+
+// The items of a march: block vectors of the (y, z) plane times chunks of
+// planes, chunk by chunk.
+struct MarchMap {
+    FastDiv q, pb;            // vectors of a half-row; items of a chunk
+    unsigned plane;           // vectors of a plane
+    unsigned items;
+    int len;                  // planes of a chunk
+};
+
+template <int TYPE, int DIM, bool NORM_ONLY, bool E, bool CX, bool CB, bool CXO, bool NOXW, bool UNI>
+__global__ void __launch_bounds__(kNormThreads) k_refine_march(LevelArgs<double> L, MarchMap M,
+                                                               const double *__restrict__ xold,
+                                                               const float *__restrict__ e, long esx_, long esy_,
+                                                               long ehz_, const double *__restrict__ b,
+                                                               double *__restrict__ xnew, float *__restrict__ r32,
+                                                               double *__restrict__ partial, FullRows F) {
+    static_assert(!(CX && CXO), "x_old and x_new cannot both be the caller's array");
+    constexpr int W = 2;
+    using u32 = unsigned;
+    const int nx = L.n[0], ny = DIM == 3 ? L.n[1] : 1, nz = L.n[2], half = nz >> 1;
+    const int lane = threadIdx.x & 63;
+    const u32 sx = (u32)L.sx * 8u, sy = (u32)L.sy * 8u, hz = (u32)L.hz * 8u;
+    const u32 esx = (u32)esx_ * 4u, esy = (u32)esy_ * 4u, ehz = (u32)ehz_ * 4u;
+    const u32 fi = (u32)F.si * 8u, fj = (u32)F.sj * 8u, f0 = (u32)F.off * 8u;
+    const bool perx = L.bc_lo[0] == BC_PER, pery = DIM == 3 && L.bc_lo[1] == BC_PER, perz = L.bc_lo[2] == BC_PER;
+    auto at = [](const void *p, u32 o) __attribute__((always_inline)) { return reinterpret_cast<const char *>(p) + o; };
+    const char *X = reinterpret_cast<const char *>(CX ? F.x : xold);
+    double ar = 0.0, ab = 0.0;
+    // each XCD takes one contiguous range of items
+    const u32 per = gridDim.x / kXcds;
+    for (u32 it = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds; it < M.items; it += gridDim.x) {
+        const u32 chunk = M.pb.div(it), s0 = (it - chunk * M.pb.d) * kNormThreads + threadIdx.x;
+        const bool live = s0 < M.plane;
+        const u32 sv = live ? s0 : M.plane - 1;   // a lane beyond the plane repeats its last vector, unwritten
+        const int j = (int)M.q.div(sv), m0 = (int)(sv - (u32)j * M.q.d) * W;
+        const int i0 = (int)chunk * M.len, i1 = min(nx, i0 + M.len);
+        const u32 mo = (u32)m0 * 8u, me = (u32)m0 * 4u;
+        const u32 row = (u32)j * sy, erow = (u32)j * esy, frow = f0 + (u32)j * fj;
+        const bool inn = j + 1 < ny, ins = j > 0;
+        const u32 jn = (u32)(inn ? 1 : (pery ? 1 - ny : 0)), js = (u32)(ins ? -1 : (pery ? ny - 1 : 0));
+        struct Raw {
+            double2 a, b;   // split rows: even, odd; caller rows: cells 2 m0.., 2 m0 + 2..
+            float2 ea, eb;
+        };
+        // the lane's four cells of row (i, j + dj)
+        auto load = [&](int i, u32 dj) __attribute__((always_inline)) {
+            Raw r;
+            if (CX) {
+                const u32 o = frow + (u32)i * fi + dj * fj + 2u * mo;
+                const double2u p = *reinterpret_cast<const double2u *>(X + o), t = *reinterpret_cast<const double2u *>(X + o + 16u);
+                r.a = make_double2(p.x, t.x);
+                r.b = make_double2(p.y, t.y);
+            } else {
+                const u32 o = row + (u32)i * sx + dj * sy + mo;
+                r.a = *reinterpret_cast<const double2 *>(X + o);
+                r.b = *reinterpret_cast<const double2 *>(X + o + hz);
+            }
+            if (E) {
+                const u32 o = erow + (u32)i * esx + dj * esy + me;
+                r.ea = *reinterpret_cast<const float2 *>(at(e, o));
+                r.eb = *reinterpret_cast<const float2 *>(at(e, o + ehz));
+            }
+            return r;
+        };
+        struct Cells {
+            double v[2][W];   // [half][position]
+        };
+        auto value = [&](const Raw &r) __attribute__((always_inline)) {
+            Cells c{{{r.a.x, r.a.y}, {r.b.x, r.b.y}}};
+            if (E) {
+                c.v[0][0] = c.v[0][0] + (double)r.ea.x;
+                c.v[0][1] = c.v[0][1] + (double)r.ea.y;
+                c.v[1][0] = c.v[1][0] + (double)r.eb.x;
+                c.v[1][1] = c.v[1][1] + (double)r.eb.y;
+            }
+            return c;
+        };
+        auto flip = [](bool wall, int code, Cells c) __attribute__((always_inline)) {
+            if (code == BC_DIR && wall) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int p = 0; p < W; ++p) c.v[h][p] = -c.v[h][p];
+            }
+            return c;
+        };
+        const double c2y = DIM == 3 ? L.c2[1][UNI ? 0 : j] : 0.0, c1y = DIM == 3 ? L.c1[1][UNI ? 0 : j] : 0.0;
+        double c2z[2][W], c1z[2][W];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (UNI) {
+#pragma unroll
+                for (int p = 0; p < W; ++p) {
+                    c2z[h][p] = L.c2[2][0];
+                    c1z[h][p] = L.c1[2][0];
+                }
+            } else {
+                load_n<double, W>(L.c2zs + h * half + m0, c2z[h]);
+                load_n<double, W>(L.c1zs + h * half + m0, c1z[h]);
+            }
+        }
+        // z neighbours no adjacent lane holds: below the first even cell, above the last odd one
+        const bool zlo = m0 == 0, zhi = m0 + W == half;
+        const bool zll = zlo || lane == 0, zhl = zhi || lane == 63;
+        const int kl = zlo ? (perz ? nz - 1 : 0) : 2 * m0 - 1, kh = zhi ? (perz ? 0 : nz - 1) : 2 * (m0 + W);
+        auto cell = [&](int i, int k) __attribute__((always_inline)) {
+            double v = CX ? *reinterpret_cast<const double *>(X + frow + (u32)i * fi + (u32)k * 8u)
+                          : *reinterpret_cast<const double *>(X + row + (u32)i * sx + (k & 1 ? hz : 0u) + (u32)(k >> 1) * 8u);
+            if (E)
+                v = v + (double)*reinterpret_cast<const float *>(
+                            at(e, erow + (u32)i * esx + (k & 1 ? ehz : 0u) + (u32)(k >> 1) * 4u));
+            return v;
+        };
+        // the plane behind, and the first one
+        Cells west, cur;
+        {
+            const Raw w = load(i0 > 0 ? i0 - 1 : (perx ? nx - 1 : 0), 0u), c = load(i0, 0u);
+            cur = value(c);
+            west = flip(i0 == 0 && !perx, L.bc_lo[0], value(w));
+        }
+        for (int i = i0; i < i1; ++i) {
+            const bool ine = i + 1 < nx;
+            const Raw re = load(ine ? i + 1 : (perx ? 0 : i), 0u);
+            Raw rn{}, rs{};
+            if (DIM == 3) {
+                rn = load(i, jn);
+                rs = load(i, js);
+            }
+            double2 ba, bb;
+            if (CB) {
+                const char *p = at(F.b, frow + (u32)i * fi + 2u * mo);
+                const double2u u = *reinterpret_cast<const double2u *>(p), t = *reinterpret_cast<const double2u *>(p + 16);
+                ba = make_double2(u.x, t.x);
+                bb = make_double2(u.y, t.y);
+            } else {
+                ba = *reinterpret_cast<const double2 *>(at(b, row + (u32)i * sx + mo));
+                bb = *reinterpret_cast<const double2 *>(at(b, row + (u32)i * sx + mo + hz));
+            }
+            double zl = 0.0, zh = 0.0;
+            if (zll) zl = cell(i, kl);
+            if (zhl) zh = cell(i, kh);
+            const double c2x = L.c2[0][UNI ? 0 : i], c1x = L.c1[0][UNI ? 0 : i];
+            const Cells next = value(re);
+            const Cells east = flip(!ine && !perx, L.bc_hi[0], next);
+            Cells north{}, south{};
+            if (DIM == 3) {
+                north = flip(!inn, L.bc_hi[1], value(rn));
+                south = flip(!ins, L.bc_lo[1], value(rs));
+            }
+            const double prev = __shfl_up(cur.v[1][W - 1], 1, 64), foll = __shfl_down(cur.v[0][0], 1, 64);
+            const double zb = zll ? (zlo && L.bc_lo[2] == BC_DIR ? -zl : zl) : prev;
+            const double zt = zhl ? (zhi && L.bc_hi[2] == BC_DIR ? -zh : zh) : foll;
+            const double bv[2][W] = {{ba.x, ba.y}, {bb.x, bb.y}};
+            double r[2][W];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int p = 0; p < W; ++p) {
+                    Stencil<double, DIM> s;
+                    s.c = cur.v[h][p];
+                    s.xE = east.v[h][p];
+                    s.xW = west.v[h][p];
+                    if (DIM == 3) {
+                        s.yN = north.v[h][p];
+                        s.yS = south.v[h][p];
+                    }
+                    s.zB = h ? cur.v[0][p] : (p > 0 ? cur.v[1][p > 0 ? p - 1 : 0] : zb);
+                    s.zT = h ? (p < W - 1 ? cur.v[0][p < W - 1 ? p + 1 : p] : zt) : cur.v[1][p];
+                    r[h][p] = residual<double, DIM>(s, c2x, c1x, c2y, c1y, c2z[h][p], c1z[h][p], bv[h][p]);
+                }
+            if (live) {
+                if (!NORM_ONLY) {
+                    if (NOXW) {
+                    } else if (CXO) {
+                        char *p = reinterpret_cast<char *>(F.xo) + frow + (u32)i * fi + 2u * mo;
+                        *reinterpret_cast<double2u *>(p) = double2u{cur.v[0][0], cur.v[1][0]};
+                        *reinterpret_cast<double2u *>(p + 16) = double2u{cur.v[0][1], cur.v[1][1]};
+                    } else {
+                        char *p = reinterpret_cast<char *>(xnew) + row + (u32)i * sx + mo;
+                        *reinterpret_cast<double2 *>(p) = make_double2(cur.v[0][0], cur.v[0][1]);
+                        *reinterpret_cast<double2 *>(p + hz) = make_double2(cur.v[1][0], cur.v[1][1]);
+                    }
+                    char *p = reinterpret_cast<char *>(r32) + erow + (u32)i * esx + me;
+                    *reinterpret_cast<float2 *>(p) = make_float2((float)r[0][0], (float)r[0][1]);
+                    *reinterpret_cast<float2 *>(p + ehz) = make_float2((float)r[1][0], (float)r[1][1]);
+                }
+#pragma unroll
+                for (int p = 0; p < W; ++p) {
+                    ar = norm_acc<TYPE>(ar, r[0][p]);
+                    ab = norm_acc<TYPE>(ab, bv[0][p]);
+                    ar = norm_acc<TYPE>(ar, r[1][p]);
+                    ab = norm_acc<TYPE>(ab, bv[1][p]);
+                }
+            }
+            west = cur;
+            cur = next;
+        }
+    }
+    block_reduce2<TYPE>(ar, ab);
+    if (threadIdx.x == 0) {
+        partial[2 * blockIdx.x] = ar;
+        partial[2 * blockIdx.x + 1] = ab;
+    }
+}
+
 }  // namespace saras
