@@ -436,6 +436,284 @@ __global__ void __launch_bounds__(256) k_rhs_v(Geom G, StageCoef c, CoreField V0
         rhs_v_cell<C>(G, c, V0, V1, V2, T, P, H, R, les, Sa, Sb, Sc, i, j, k);
 }
 
+// ---------------------------------------------------------------------------
+// The explicit part of one RK3 sub-stage for every field at once: the values
+// of k_rhs_v<0..2> and k_rhs_t for dScheme 2 and Morinishi's term (the decks'
+// choice), 3-D.
+//
+// The per-component kernels read each velocity component, pressure and
+// temperature again for every field, and every plane again for its x neighbours
+// (102-114 bytes fetched per cell and launch where 40-48 are needed), and were
+// bound by that.  Here a lane keeps its (j, k) and marches along x with the five
+// planes of each field that the x stencils need in registers; the terms are
+// accumulated axis by axis, each in the order of the per-component expressions,
+// so the values are the same.  What bounds it is the latency of a plane's loads
+// at two wavefronts a SIMD, so all of them are issued before the first is used:
+// with the reach-2 loads behind the edge tests, where the compiler puts them, a
+// stage took 1.01 instead of 0.84 ms (256^3 with T) and 4.9 instead of 3.1 ms
+// (384^3 with the stresses).  Blocks are 64 cells of z by 4 rows (8 rows: 0.88
+// and 3.26 ms), dealt so that an XCD holds neighbouring rows.
+// ---------------------------------------------------------------------------
+// first and second derivatives along `ax` at index q from the five values
+// around it (d1 and d2 for dScheme 2)
+__device__ __forceinline__ double d1_of(const Geom &G, int ax, int q, double m, double fm2, double fm, double fp, double fp2) {
+    double v;
+    if (q == 0 || q == G.n[ax] - 1) v = 0.5 * (fp - fm);
+    else v = (8.0 * (fp - fm) - (fp2 - fm2)) * kRecip12;
+    v = v * G.ih[ax];
+    return m * v;
+}
+__device__ __forceinline__ double d2_of(const Geom &G, int ax, int q, double xx, double x2, double fm2, double fm, double f,
+                                        double fp, double fp2) {
+    double t, o;
+    if (q == 0 || q == G.n[ax] - 1) {
+        t = 0.5 * (fp - fm);
+        o = fp - 2.0 * f + fm;
+    } else {
+        t = (8.0 * (fp - fm) - (fp2 - fm2)) * kRecip12;
+        o = ((-30.0 * f + 16.0 * (fp + fm)) - (fp2 + fm2)) * kRecip12;
+    }
+    t = t * G.ih[ax];
+    o = o * G.ih2[ax];
+    return xx * t + x2 * o;
+}
+// a / 6, the correctly rounded quotient, in four instructions: a product with
+// the rounded reciprocal, corrected by its exact remainder (v_div_fixup gives
+// infinities and NaN their quotients).  Of 6e8 values compared with the
+// division none differs; only subnormal quotients may, by one unit.
+__device__ __forceinline__ double by6(double a) {
+    const double y = 1.0 / 6.0, q = a * y;
+    return __builtin_amdgcn_div_fixup(fma(fma(-6.0, q, a), y, q), 6.0, a);
+}
+// Morinishi's pair of mor_pair from the values around q
+__device__ __forceinline__ double mor_of(const Geom &G, int a, int q, double xm, double u, double cm2, double cm, double cp,
+                                         double cp2, double um2, double um, double up, double up2) {
+    const double pp = up * cp, pm = um * cm;
+    double adv, dv;
+    if (mor_edge(G, a, q)) {
+        adv = u * xm * (cp - cm) * G.i2d[a];
+        dv = xm * (pp - pm) * G.i2d[a];
+    } else {
+        const double pp2 = up2 * cp2, pm2 = um2 * cm2;
+        adv = by6(u * xm * (-cp2 + 8.0 * cp - 8.0 * cm + cm2) * G.i2d[a]);
+        dv = by6(xm * (-pp2 + 8.0 * pp - 8.0 * pm + pm2) * G.i2d[a]);
+    }
+    return (adv + dv) / 2;
+}
+
+// One field of a march: its core and, on z walls, the two ghosts as the wall
+// rule gives them from the edge cell v: cst - v (Dirichlet, cst = 2 val) or
+// v - cst (Neumann, cst = kh).
+struct MarchField {
+    const double *f;
+    double cst[2];   // z-lo, z-hi
+    int dir[2];
+};
+
+struct RhsMarch {
+    MarchField F[5];      // Vx, Vy, Vz, P, T
+    double *H[4], *R[4];
+    const double *S[6];   // LES: Txx, Tyy, Tzz, Txy, Tyz, Tzx
+    int len;              // planes of a chunk
+    unsigned nz, ny, nblock;   // blocks along z and y; blocks in all
+};
+
+constexpr int kRhsZ = 64, kRhsY = 4;
+
+// x and y periodic, z periodic or with Dirichlet / Neumann walls; fields below
+// 4 GB (32-bit byte offsets, the same for every field).
+template <bool HAS_T, bool LES>
+__global__ void __launch_bounds__(kRhsZ * kRhsY) __attribute__((amdgpu_waves_per_eu(2)))
+k_rhs_march(Geom G, StageCoef c, RhsMarch A) {
+    constexpr int NF = HAS_T ? 4 : 3;   // transported fields; index 3 of q[] is T
+    using u32 = unsigned;
+    // XCD-contiguous order: chunk by chunk, row groups, then z
+    const u32 per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (lb >= A.nblock) return;
+    const u32 bz = lb % A.nz, br = lb / A.nz, by = br % A.ny, chunk = br / A.ny;
+    const int k = (int)bz * kRhsZ + (int)(threadIdx.x & (kRhsZ - 1)), j = (int)by * kRhsY + (int)(threadIdx.x / kRhsZ);
+    const int nx = G.n[0], ny = G.n[1], nz = G.n[2];
+    if (k >= nz || j >= ny) return;
+    const int i0 = (int)chunk * A.len, i1 = min(nx, i0 + A.len);
+    const double ym = G.xi_x[1][j], yx = G.xixx[1][j], y2 = G.xix2[1][j];
+    const double zm = G.xi_x[2][k], zx = G.xixx[2][k], z2 = G.xix2[2][k];
+    const u32 sx = (u32)G.sx * 8u, sy = (u32)G.sy * 8u;
+    const bool zwall = !G.per[2];
+    auto at = [](const double *f, u32 o) __attribute__((always_inline)) {
+        return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(f) + o);
+    };
+    // (a value no other lane reads: kept out of the caches' way)
+    auto once = [](const double *f, u32 o) __attribute__((always_inline)) {
+        return __builtin_nontemporal_load(reinterpret_cast<const double *>(reinterpret_cast<const char *>(f) + o));
+    };
+    // offsets within a plane of the cell and of its y and z neighbours at -2, -1, 1, 2
+    const u32 oc = (u32)j * sy + (u32)k * 8u;
+    u32 oy[4], oz[4];
+    bool zlo[4], zhi[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const int s = d < 2 ? d - 2 : d - 1;
+        oy[d] = (u32)core_index(1, j + s, ny) * sy + (u32)k * 8u;
+        oz[d] = (u32)j * sy + (u32)core_index(G.per[2], k + s, nz) * 8u;
+        zlo[d] = zwall && k + s < 0;
+        zhi[d] = zwall && k + s >= nz;
+    }
+    auto plane = [&](int i) __attribute__((always_inline)) { return (u32)core_index(1, i, nx) * sx; };
+    auto zrule = [&](const MarchField &f, int d, double v) __attribute__((always_inline)) {
+        if (zlo[d]) v = f.dir[0] ? f.cst[0] - v : v - f.cst[0];
+        if (zhi[d]) v = f.dir[1] ? f.cst[1] - v : v - f.cst[1];
+        return v;
+    };
+    // field of transported quantity f, and its stresses along x, y, z
+    auto fld = [&](int f) -> const MarchField & { return A.F[f < 3 ? f : 4]; };
+    constexpr int SX[3] = {0, 3, 5}, SY[3] = {3, 1, 4}, SZ[3] = {5, 4, 2};
+    // planes i-2 .. i+2 of the fields, the pressure and the stresses
+    double q[NF][5], p[5], sg_[3][5];
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+        // (planes i0-2 .. i0+1 at slots 1 .. 4: the loop shifts before it uses them)
+        const u32 po = plane(i0 + o - 2) + oc;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) q[f][o + 1] = at(fld(f).f, po);
+        p[o + 1] = at(A.F[3].f, po);
+        if (LES)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) sg_[m][o + 1] = at(A.S[SX[m]], po);
+    }
+    for (int i = i0; i < i1; ++i) {
+        const u32 pi = (u32)i * sx, pe = plane(i + 2) + oc, o = pi + oc;
+        // every load of the plane before any of them is waited for (with the
+        // stresses, as many as the registers hold)
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) q[f][d] = q[f][d + 1];
+            q[f][4] = at(fld(f).f, pe);
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) p[d] = p[d + 1];
+        p[4] = at(A.F[3].f, pe);
+        if (LES)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+#pragma unroll
+                for (int d = 0; d < 4; ++d) sg_[m][d] = sg_[m][d + 1];
+                sg_[m][4] = m == 0 ? once(A.S[SX[m]], pe) : at(A.S[SX[m]], pe);
+            }
+        double cv[2][NF][4], pv[2][4], sv[2][3][4], hv[NF];
+        auto side = [&](int a) __attribute__((always_inline)) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                const u32 on = pi + (a == 0 ? oy[d] : oz[d]);
+#pragma unroll
+                for (int f = 0; f < NF; ++f) cv[a][f][d] = at(fld(f).f, on);
+                pv[a][d] = at(A.F[3].f, on);
+            }
+        };
+        auto side_s = [&](int a) __attribute__((always_inline)) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+#pragma unroll
+                for (int m = 0; m < 3; ++m) sv[a][m][d] = at(A.S[a == 0 ? SY[m] : SZ[m]], pi + (a == 0 ? oy[d] : oz[d]));
+        };
+        side(0);
+        if (LES) side_s(0);
+        if (!(LES && HAS_T)) side(1);
+        auto last_h = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) hv[f] = c.stage > 0 ? once(A.H[f], o) : 0.0;
+        };
+        if (!LES) last_h();
+        __builtin_amdgcn_sched_barrier(0);
+        double lap[NF], h[NF], force[3], sg[3];
+        // forcing in rhs_v_cell's order: buoyancy, the mean gradient, -dP
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            force[d] = 0.0;
+            if (HAS_T) force[d] -= c.buoy[d] * q[NF - 1][2];
+            if (d == 0 && c.mpg != 0.0) force[d] += c.mpg;
+            sg[d] = 0.0;
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f) lap[f] = h[f] = 0.0;
+        {
+            const double m = G.xi_x[0][i], xx = G.xixx[0][i], x2 = G.xix2[0][i];
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                lap[f] += d2_of(G, 0, i, xx, x2, q[f][0], q[f][1], q[f][2], q[f][3], q[f][4]);
+                h[f] -= mor_of(G, 0, i, m, q[0][2], q[f][0], q[f][1], q[f][3], q[f][4], q[0][0], q[0][1], q[0][3], q[0][4]);
+            }
+            force[0] -= d1_of(G, 0, i, m, p[0], p[1], p[3], p[4]);
+            if (LES)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) sg[d] = d1_of(G, 0, i, m, sg_[d][0], sg_[d][1], sg_[d][3], sg_[d][4]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ax = 1; ax < 3; ++ax) {
+            const int a = ax - 1, s = ax == 1 ? j : k;
+            const double m = ax == 1 ? ym : zm, xx = ax == 1 ? yx : zx, x2 = ax == 1 ? y2 : z2;
+            if (LES && ax == 2) {
+                if (HAS_T) side(1);
+                side_s(1);
+                last_h();
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // (held here: a load used on one side of an edge test only would
+            // otherwise be moved behind the test, and wait there by itself)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f) asm volatile("" : "+v"(cv[a][f][d]));
+                asm volatile("" : "+v"(pv[a][d]));
+                if (LES)
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) asm volatile("" : "+v"(sv[a][e][d]));
+            }
+            if (ax == 2 && zwall)
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+#pragma unroll
+                    for (int f = 0; f < NF; ++f) cv[a][f][d] = zrule(fld(f), d, cv[a][f][d]);
+                    pv[a][d] = zrule(A.F[3], d, pv[a][d]);
+                }
+            const double(&u)[4] = cv[a][ax];
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                const double(&v)[4] = cv[a][f];
+                lap[f] += d2_of(G, ax, s, xx, x2, v[0], v[1], q[f][2], v[2], v[3]);
+                h[f] -= mor_of(G, ax, s, m, q[ax][2], v[0], v[1], v[2], v[3], u[0], u[1], u[2], u[3]);
+            }
+            force[ax] -= d1_of(G, ax, s, m, pv[a][0], pv[a][1], pv[a][2], pv[a][3]);
+            if (LES)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const double(&v)[4] = sv[a][d];
+                    sg[d] = sg[d] + d1_of(G, ax, s, m, v[0], v[1], v[2], v[3]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            double r = 0.0;
+            if (c.stage > 0) r += c.zeta * hv[f];
+            if (f < 3) {
+                r += c.a_nu * lap[f];
+                r += c.ab * force[f < 3 ? f : 0];
+                if (LES) h[f] = h[f] - sg[f < 3 ? f : 0];
+            } else {
+                r += c.a_kappa * lap[f];
+                r += c.ab * 0.0;
+            }
+            r += c.gamma * h[f];
+            r *= c.dt;
+            r += q[f][2];
+            __builtin_nontemporal_store(h[f], reinterpret_cast<double *>(reinterpret_cast<char *>(A.H[f]) + o));
+            __builtin_nontemporal_store(r, reinterpret_cast<double *>(reinterpret_cast<char *>(A.R[f]) + o));
+        }
+    }
+}
+
 // the same for the scalar (tmpRHS / tempSF); its forcing term is zero
 template <class F>
 __device__ __forceinline__ void rhs_t_cell(const Geom &G, const StageCoef &c, const F &V0, const F &V1, const F &V2,
