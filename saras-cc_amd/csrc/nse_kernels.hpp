@@ -830,210 +830,296 @@ __device__ __forceinline__ double sf_integral(double d) {   // spiral.cc:620-631
     return 12.2946 * (c * c) - 6.0 - 0.573159 / (d * sqrt(d)) * sin(3.14159 * d - 0.785398);
 }
 
+// Correctly rounded single-precision root and quotients, the values of sqrtf and
+// of the division, without the scaling of arguments near the ends of the range
+// (11 and 3 or 9 issue slots instead of 17 and 11).  Compared with them on the
+// device: the root at every significand at 120 exponents, 0.573159 / b at every
+// significand at 52, 1e9 pairs of quot_rn; none differs.
+__device__ __forceinline__ float sqrt_rn(float a) {
+    const float y = __builtin_amdgcn_rsqf(a);
+    float g = a * y, h = 0.5f * y;
+    const float e = fmaf(-h, g, 0.5f);
+    g = fmaf(g, e, g);
+    h = fmaf(h, e, h);
+    return a < 0x1p-100f ? 0.0f : fmaf(fmaf(-g, g, a), h, g);
+}
+// a / b from the rounded reciprocal y of b
+__device__ __forceinline__ float quot_rn(float a, float b, float y) {
+    const float q = a * y;
+    return fmaf(fmaf(-b, q, a), y, q);
+}
+
 // sf_integral in single precision (the same expression)
 __device__ __forceinline__ float sf_integral_f(float d) {
     const float d2 = d * d;
-    if (d < 0.873469f) return 7.4022f * d2 - 1.82642f * d2 * d2;
-    const float c = cbrtf(d);
-    return 12.2946f * (c * c) - 6.0f - 0.573159f / (d * sqrtf(d)) * sinf(3.14159f * d - 0.785398f);
+    const float near = 7.4022f * d2 - 1.82642f * d2 * d2;
+    if (d < 0.873469f) return near;
+    const float c = cbrtf(d), b = d * sqrt_rn(d), y = __builtin_amdgcn_rcpf(b);
+    return 12.2946f * (c * c) - 6.0f -
+           quot_rn(0.573159f, b, fmaf(fmaf(-b, y, 1.0f), y, y)) * sinf(3.14159f * d - 0.785398f);
 }
 
-// One core cell of spiral::computeSG (spiral.cc:157-206 with sgsStress
-// :472-548, eigenvalueSymm :643-~690, eigenvectorSymm :702-~742) on a fully
-// periodic box: writes the six stresses, returns false where the reference
-// aborts.  SF32: the structure-function integral Qd (the 13 or 26
-// sfIntegral terms, most of the cell's arithmetic) in single precision; the
-// velocity gradients, eigen-decomposition, F2 and the energy integral stay
-// in double, so the stress carries the single-precision rounding of Qd only.
-template <bool SF32 = false>
-__device__ bool sgs_cell(const Geom &G, const CoreField *V, double nu, int i, int j, int k, double T[6],
-                         double &K, double S[6]) {
-    double dudx[3][3];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-        dudx[r][0] = d1(G, V[r], 0, i, j, k);
-        dudx[r][1] = d1(G, V[r], 1, i, j, k);
-        dudx[r][2] = d1(G, V[r], 2, i, j, k);
-    }
-    const double Sxx = 0.5 * (dudx[0][0] + dudx[0][0]), Syy = 0.5 * (dudx[1][1] + dudx[1][1]);
-    const double Szz = 0.5 * (dudx[2][2] + dudx[2][2]), Sxy = 0.5 * (dudx[0][1] + dudx[1][0]);
-    const double Syz = 0.5 * (dudx[1][2] + dudx[2][1]), Szx = 0.5 * (dudx[2][0] + dudx[0][2]);
-    S[0] = Sxx; S[1] = Syy; S[2] = Szz; S[3] = Sxy; S[4] = Syz; S[5] = Szx;
-    // eigenvalueSymm
+// spiral::sgsStress (spiral.cc:472-548 with eigenvalueSymm :643-~690 and
+// eigenvectorSymm :702-~742): the vortex axis e (up to its sign: only products
+// of two components enter) and the stretching along it from the strain rates
+// S = (xx, yy, zz, xy, yz, zx); false where the reference aborts.
+__device__ __forceinline__ bool sgs_axis(const double (&S)[6], double (&e)[3], double &ax) {
+    const double Sxx = S[0], Syy = S[1], Szz = S[2], Sxy = S[3], Syz = S[4], Szx = S[5];
     const double a = -(Sxx + Syy + Szz);
     const double b = Sxx * Syy - Sxy * Sxy + Syy * Szz - Syz * Syz + Szz * Sxx - Szx * Szx;
     const double cc = -(Sxx * (Syy * Szz - Syz * Syz) + Sxy * (Syz * Szx - Sxy * Szz) + Szx * (Sxy * Syz - Syy * Szx));
     const double q = (3.0 * b - a * a) / 9.0;
     const double r = (9.0 * a * b - 27.0 * cc - 2.0 * a * a * a) / 54.0;
     if (q >= 0.0) return false;
-    const double costheta = r / sqrt(-q * q * q);
+    const double sq = sqrt(-q), costheta = r / (-q * sq);
     const double theta = costheta > 1.0 ? 0.0 : costheta < -1.0 ? kPi : acos(costheta);
-    double ev[3];
-    ev[0] = 2.0 * sqrt(-q) * cos((theta) / 3.0) - a / 3.0;
-    ev[1] = 2.0 * sqrt(-q) * cos((theta + 2.0 * kPi) / 3.0) - a / 3.0;
-    ev[2] = 2.0 * sqrt(-q) * cos((theta + 4.0 * kPi) / 3.0) - a / 3.0;
-    double tt;
-    if (ev[0] > ev[1]) { tt = ev[0]; ev[0] = ev[1]; ev[1] = tt; }
-    if (ev[1] > ev[2]) { tt = ev[1]; ev[1] = ev[2]; ev[2] = tt; }
-    if (ev[0] > ev[1]) { tt = ev[0]; ev[0] = ev[1]; ev[1] = tt; }
-    const double lam = ev[2];
-    // eigenvectorSymm
-    const double fNorm = sqrt(Sxx * Sxx + Syy * Syy + Szz * Szz + Sxy * Sxy + Syz * Syz + Szx * Szx);
+    // the largest of the three roots: theta / 3 is at most pi / 3 and the cosine
+    // there at least 1/2, at the angles (theta + 2 pi) / 3 and (theta + 4 pi) / 3
+    // at most 1/2
+    const double lam = 2.0 * sq * cos(theta / 3.0) - a / 3.0;
+    const double f = sqrt(Sxx * Sxx + Syy * Syy + Szz * Szz + Sxy * Sxy + Syz * Syz + Szx * Szx);
     if (fabs((Sxx - lam) * ((Syy - lam) * (Szz - lam) - Syz * Syz) + Sxy * (Syz * Szx - Sxy * (Szz - lam)) +
-             Szx * (Sxy * Syz - (Syy - lam) * Szx)) / fabs(fNorm) > kSgsEps)
+             Szx * (Sxy * Syz - (Syy - lam) * Szx)) > kSgsEps * f)
         return false;
+    // the row of the adjugate of S - lam with the largest diagonal, normalised
     const double det0 = (Syy - lam) * (Szz - lam) - Syz * Syz, det1 = (Szz - lam) * (Sxx - lam) - Szx * Szx;
     const double det2 = (Sxx - lam) * (Syy - lam) - Sxy * Sxy;
+    const double a01 = -Sxy * (Szz - lam) + Szx * Syz, a02 = -Szx * (Syy - lam) + Sxy * Syz;
+    const double a12 = -Syz * (Sxx - lam) + Sxy * Szx;
     const double f0 = fabs(det0), f1 = fabs(det1), f2 = fabs(det2);
-    double e[3];
-    if (f0 >= f1 && f0 >= f2) {
-        e[0] = 1.0;
-        e[1] = (-Sxy * (Szz - lam) + Szx * Syz) / det0;
-        e[2] = (-Szx * (Syy - lam) + Sxy * Syz) / det0;
-    } else if (f1 >= f2 && f1 >= f0) {
-        e[0] = (-Sxy * (Szz - lam) + Syz * Szx) / det1;
-        e[1] = 1.0;
-        e[2] = (-Syz * (Sxx - lam) + Sxy * Szx) / det1;
-    } else if (f2 >= f0 && f2 >= f1) {
-        e[0] = (-Szx * (Syy - lam) + Syz * Sxy) / det2;
-        e[1] = (-Syz * (Sxx - lam) + Szx * Sxy) / det2;
-        e[2] = 1.0;
-    } else {
-        return false;
-    }
-    const double length = sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
-    e[0] /= length;
-    e[1] /= length;
-    e[2] /= length;
-    const double ax = e[0] * e[0] * Sxx + e[0] * e[1] * Sxy + e[0] * e[2] * Szx + e[1] * e[0] * Sxy +
-                      e[1] * e[1] * Syy + e[1] * e[2] * Syz + e[2] * e[0] * Szx + e[2] * e[1] * Syz +
-                      e[2] * e[2] * Szz;
-    const double lv = sqrt(2.0 * nu / (3.0 * (fabs(ax) + kSgsEps)));
-    // structure function over the 26 neighbours (periodic wrap)
-    const double dxv = G.xc[0][i] - G.xc[0][i - 1], dyv = G.xc[1][j] - G.xc[1][j - 1];
-    const double dzv = G.xc[2][k] - G.xc[2][k - 1];
-    const double del = cbrt(dxv * dyv * dzv);
-    const double u0 = V[0].at(G, i, j, k), v0 = V[1].at(G, i, j, k), w0 = V[2].at(G, i, j, k);
-    double F2 = 0.0, Qd = 0.0;
-    int cnt = 0;
-#pragma unroll 1
-    for (int di = -1; di <= 1; ++di) {
-        const int ii = i + di < 0 ? i + di + G.n[0] : (i + di >= G.n[0] ? i + di - G.n[0] : i + di);
-        for (int dj = -1; dj <= 1; ++dj) {
-            const int jj = j + dj < 0 ? j + dj + G.n[1] : (j + dj >= G.n[1] ? j + dj - G.n[1] : j + dj);
-            for (int dk = -1; dk <= 1; ++dk) {
-                if (!(di || dj || dk)) continue;
-                const int kk = k + dk < 0 ? k + dk + G.n[2] : (k + dk >= G.n[2] ? k + dk - G.n[2] : k + dk);
-                const double du = V[0].at(G, ii, jj, kk) - u0, dv = V[1].at(G, ii, jj, kk) - v0;
-                const double dw = V[2].at(G, ii, jj, kk) - w0;
-                F2 += du * du + dv * dv + dw * dw;
-                ++cnt;
-            }
-        }
-    }
-    // sfIntegral of each neighbour offset's distance from the vortex axis.  The
-    // distance is even in the offset, so where the spacing on the two sides of
-    // the cell agrees to rounding (uniform axes) each of the 13 offsets of one
-    // half stands for its mirror image too; elsewhere all 26 are evaluated.
-    const double dxp = G.xc[0][i + 1] - G.xc[0][i], dxm = G.xc[0][i - 1] - G.xc[0][i];
-    const double dyp = G.xc[1][j + 1] - G.xc[1][j], dym = G.xc[1][j - 1] - G.xc[1][j];
-    const double dzp = G.xc[2][k + 1] - G.xc[2][k], dzm = G.xc[2][k - 1] - G.xc[2][k];
-    auto close = [](double a, double b) { return fabs(a + b) <= 1e-12 * fabs(a); };
-    const bool mirror = close(dxp, dxm) && close(dyp, dym) && close(dzp, dzm);
-    const float fdxm = (float)dxm, fdxp = (float)dxp, fdym = (float)dym, fdyp = (float)dyp;
-    const float fdzm = (float)dzm, fdzp = (float)dzp, fe0 = (float)e[0], fe1 = (float)e[1], fe2 = (float)e[2];
-    const float fdel = (float)del;
-    auto sf_at = [&](int di, int dj, int dk) -> double {
-        if (SF32) {
-            const float dx = di < 0 ? fdxm : (di > 0 ? fdxp : 0.0f);
-            const float dy = dj < 0 ? fdym : (dj > 0 ? fdyp : 0.0f);
-            const float dz = dk < 0 ? fdzm : (dk > 0 ? fdzp : 0.0f);
-            const float dx2 = dx * dx + dy * dy + dz * dz;
-            const float dxe = dx * fe0 + dy * fe1 + dz * fe2;
-            return (double)sf_integral_f(sqrtf(fmaxf(dx2 - dxe * dxe, 0.0f)) / fdel);
-        }
-        const double dx = di < 0 ? dxm : (di > 0 ? dxp : 0.0);
-        const double dy = dj < 0 ? dym : (dj > 0 ? dyp : 0.0);
-        const double dz = dk < 0 ? dzm : (dk > 0 ? dzp : 0.0);
-        const double dx2 = dx * dx + dy * dy + dz * dz;
-        const double dxe = dx * e[0] + dy * e[1] + dz * e[2];
-        return sf_integral(sqrt(dx2 - dxe * dxe) / del);
-    };
-    if (mirror) {
-        // the 13 offsets before (0, 0, 0) in (di, dj, dk) order
-#pragma unroll 1
-        for (int t = 0; t < 13; ++t) {
-            const int di = t / 9 - 1, dj = (t / 3) % 3 - 1, dk = t % 3 - 1;
-            Qd += 2.0 * sf_at(di, dj, dk);
-        }
-    } else {
-#pragma unroll 1
-        for (int t = 0; t < 27; ++t) {
-            if (t == 13) continue;
-            Qd += sf_at(t / 9 - 1, (t / 3) % 3 - 1, t % 3 - 1);
-        }
-    }
-    F2 /= (double)cnt;
-    Qd /= (double)cnt;
-    const double prefac = F2 / Qd;
-    const double kc = kPi / del;
-    K = prefac * ke_integral(kc * lv);
-    T[0] = (1.0 - e[0] * e[0]) * K;
-    T[1] = (1.0 - e[1] * e[1]) * K;
-    T[2] = (1.0 - e[2] * e[2]) * K;
-    T[3] = (-e[0] * e[1]) * K;
-    T[4] = (-e[1] * e[2]) * K;
-    T[5] = (-e[2] * e[0]) * K;
+    const bool is0 = f0 >= f1 && f0 >= f2, is1 = f1 >= f2 && f1 >= f0, is2 = f2 >= f0 && f2 >= f1;
+    if (!(is0 || is1 || is2)) return false;
+    e[0] = is0 ? det0 : is1 ? a01 : a02;
+    e[1] = is0 ? a01 : is1 ? det1 : a12;
+    e[2] = is0 ? a02 : is1 ? a12 : det2;
+    const double il = 1.0 / sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) e[c] *= il;
+    ax = e[0] * e[0] * Sxx + e[1] * e[1] * Syy + e[2] * e[2] * Szz +
+         2.0 * (e[0] * e[1] * Sxy + e[1] * e[2] * Syz + e[2] * e[0] * Szx);
     return true;
 }
 
-// sub-grid stresses of every core cell, per-block partial diagnostics
-// [sum |K| dV, sum dissipation dV, sum nu_t dV], failure flag
+// Blocks of k_sgs_stress: kSgsZ x kSgsY columns and a chunk of planes; the
+// three velocities' planes i-1 .. i+2 with a rim of two cells in the LDS.
+struct SgsMarch {
+    const double *V[3];
+    double *T[6];         // xx, yy, zz, xy, yz, zx
+    double *part;
+    int *fail;
+    int len;              // planes of a chunk
+    unsigned nz, ny, nblock;
+};
+constexpr int kSgsZ = 64, kSgsY = 4, kSgsThreads = kSgsZ * kSgsY;
+constexpr int kSgsW = kSgsZ + 4, kSgsTile = kSgsW * (kSgsY + 4), kSgsSlots = (kSgsTile + kSgsThreads - 1) / kSgsThreads;
+
+// Sub-grid stresses of every core cell of a fully periodic box
+// (spiral::computeSG, spiral.cc:157-206), per-block partial diagnostics
+// [sum |K| dV, sum dissipation dV, sum nu_t dV], failure flag.  SF32: the
+// structure-function integral Qd (the 13 or 26 sfIntegral terms, most of the
+// cell's arithmetic) in single precision; the velocity gradients,
+// eigen-decomposition, F2 and the energy integral stay in double, so the stress
+// carries the single-precision rounding of Qd only.
+//
+// Bound by instructions: 3540 of them a cell, 96 % of the cycles, when each cell
+// by itself took three cosines and a sort for the largest root, six divisions
+// for the axis (one of three branches each) and exactly rounded single-precision
+// roots and divisions in the 13 terms; and, next, by the 126 loads a cell, 16
+// cycles each in the vector cache.  Now a block marches along x and keeps the
+// planes in the LDS (a plane's loads are issued one plane ahead), the roots and
+// divisions that cancel are left out, and the 13 terms are unrolled.  Two
+// wavefronts a SIMD: at three the registers spill, and the call takes 5.1
+// instead of 4.2 ms at 384^3.
 template <bool SF32>
-__global__ void __launch_bounds__(256) k_sgs_stress(Geom G, CoreField V0, CoreField V1, CoreField V2, double nu,
-                                                    double *__restrict__ Txx, double *__restrict__ Tyy,
-                                                    double *__restrict__ Tzz, double *__restrict__ Txy,
-                                                    double *__restrict__ Tyz, double *__restrict__ Tzx,
-                                                    double *__restrict__ part, int *__restrict__ fail) {
-    int i, j, k;
-    row_cell(G, i, j, k);
-    double v[3] = {0.0, 0.0, 0.0};
-    if (k < G.n[2]) {
-        const CoreField V[3] = {V0, V1, V2};
-        double T[6], K, S[6];
-        if (!sgs_cell<SF32>(G, V, nu, i, j, k, T, K, S)) {
-            atomicOr(fail, 1);
-            T[0] = T[1] = T[2] = T[3] = T[4] = T[5] = 0.0;
-            K = 0.0;
-        }
-        const long idx = (long)i * G.sx + (long)j * G.sy + k;
-        Txx[idx] = T[0];
-        Tyy[idx] = T[1];
-        Tzz[idx] = T[2];
-        Txy[idx] = T[3];
-        Tyz[idx] = T[4];
-        Tzx[idx] = T[5];
-        const double A = (1.0 / G.n[0]) / G.xi_x[0][i], B = (1.0 / G.n[1]) / G.xi_x[1][j];
-        const double C = (1.0 / G.n[2]) / G.xi_x[2][k];
-        v[0] = fabs(K) * A * B * C;
-        const double sgDiss = -(S[0] * T[0] + S[1] * T[1] + S[2] * T[2] + 2.0 * (S[3] * T[3] + S[4] * T[4] + S[5] * T[5]));
-        v[1] = sgDiss * A * B * C;
-        const double sNorm = sqrt(S[0] * S[0] + S[1] * S[1] + S[2] * S[2] + 2.0 * (S[3] * S[3] + S[4] * S[4] + S[5] * S[5]));
-        const double tNorm = sqrt(T[0] * T[0] + T[1] * T[1] + T[2] * T[2] + 2.0 * (T[3] * T[3] + T[4] * T[4] + T[5] * T[5]));
-        v[2] = ((tNorm / sNorm) / 2) * A * B * C;
+__global__ void __launch_bounds__(kSgsThreads) __attribute__((amdgpu_waves_per_eu(2)))
+k_sgs_stress(Geom G, double nu, SgsMarch A) {
+    __shared__ double tile[4][3][kSgsTile];
+    __shared__ double red[3][kSgsThreads / 64];
+    using u32 = unsigned;
+    const u32 per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (lb >= A.nblock) return;
+    const u32 bz = lb % A.nz, br = lb / A.nz, by = br % A.ny, chunk = br / A.ny;
+    const int nx = G.n[0], ny = G.n[1], nz = G.n[2], tid = threadIdx.x;
+    const int lz = tid & (kSgsZ - 1), ly = tid / kSgsZ;
+    const int k = (int)bz * kSgsZ + lz, j = (int)by * kSgsY + ly;
+    const int i0 = (int)chunk * A.len, i1 = min(nx, i0 + A.len);
+    const bool on = k < nz && j < ny;
+    auto wrap = [](int q, int n) { return core_index(1, q, n); };
+    // this thread's share of a tile: offsets within a plane
+    u32 off[kSgsSlots];
+#pragma unroll
+    for (int s = 0; s < kSgsSlots; ++s) {
+        const int t = min(tid + s * kSgsThreads, kSgsTile - 1);
+        off[s] = (u32)wrap((int)by * kSgsY + t / kSgsW - 2, ny) * (u32)G.sy + (u32)wrap((int)bz * kSgsZ + t % kSgsW - 2, nz);
     }
-    __shared__ double red[3][4];
+    const u32 oc = (u32)min(j, ny - 1) * (u32)G.sy + (u32)min(k, nz - 1);
+    auto fetch = [&](int i, double (&v)[3][kSgsSlots]) __attribute__((always_inline)) {
+        const long p = (long)wrap(i, nx) * G.sx;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int s = 0; s < kSgsSlots; ++s)
+                if ((s + 1) * kSgsThreads <= kSgsTile || tid + s * kSgsThreads < kSgsTile) v[c][s] = (A.V[c] + p)[off[s]];
+    };
+    auto stash = [&](int i, const double (&v)[3][kSgsSlots]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int s = 0; s < kSgsSlots; ++s)
+                if ((s + 1) * kSgsThreads <= kSgsTile || tid + s * kSgsThreads < kSgsTile)
+                    tile[i & 3][c][tid + s * kSgsThreads] = v[c][s];
+    };
+    double pre[3][kSgsSlots], m2[3], p2[3];
+    for (int i = i0 - 1; i < i0 + 2; ++i) {
+        fetch(i, pre);
+        stash(i, pre);
+    }
+    fetch(i0 + 2, pre);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        m2[c] = (A.V[c] + (long)wrap(i0 - 2, nx) * G.sx)[oc];
+        p2[c] = (A.V[c] + (long)wrap(i0 + 2, nx) * G.sx)[oc];
+    }
+    const double inx = 1.0 / G.n[0];
+    const int jj = min(j, ny - 1), kk = min(k, nz - 1);
+    const double volB = (1.0 / G.n[1]) / G.xi_x[1][jj], volC = (1.0 / G.n[2]) / G.xi_x[2][kk];
+    const double ym = G.xi_x[1][jj], zm = G.xi_x[2][kk];
+    const double dyp = G.xc[1][jj + 1] - G.xc[1][jj], dym = G.xc[1][jj - 1] - G.xc[1][jj];
+    const double dzp = G.xc[2][kk + 1] - G.xc[2][kk], dzm = G.xc[2][kk - 1] - G.xc[2][kk];
+    auto close = [](double a, double b) { return fabs(a + b) <= 1e-12 * fabs(a); };
+    const bool mirror_yz = close(dyp, dym) && close(dzp, dzm);
+    // first derivative along ax at index q from the four values around it
+    auto der = [&](int ax, int q, double m, double fm2, double fm, double fp, double fp2) __attribute__((always_inline)) {
+        double v = (8.0 * (fp - fm) - (fp2 - fm2)) * kRecip12;
+        if (G.dscheme == 1 || q == 0 || q == G.n[ax] - 1) v = 0.5 * (fp - fm);
+        return m * (v * G.ih[ax]);
+    };
+    double sum[3] = {0.0, 0.0, 0.0};
+    bool failed = false;
+    const int own = (ly + 2) * kSgsW + lz + 2;
+    for (int i = i0; i < i1; ++i) {
+        // one barrier a plane: what this plane's stash overwrites (plane i-2) was
+        // last read before it, and what it reads was stashed before it
+        __syncthreads();
+        stash(i + 2, pre);
+        fetch(i + 3, pre);
+        double p3[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) p3[c] = (A.V[c] + (long)wrap(i + 3, nx) * G.sx)[oc];
+        double g[3][3], f0[3], F2 = 0.0;
+        {
+            const double xm = G.xi_x[0][i];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const double *w = tile[(i - 1) & 3][c] + own, *o = tile[i & 3][c] + own, *n = tile[(i + 1) & 3][c] + own;
+                f0[c] = o[0];
+                g[c][0] = der(0, i, xm, m2[c], w[0], n[0], p2[c]);
+                g[c][1] = der(1, j, ym, o[-2 * kSgsW], o[-kSgsW], o[kSgsW], o[2 * kSgsW]);
+                g[c][2] = der(2, k, zm, o[-2], o[-1], o[1], o[2]);
+                m2[c] = w[0];
+                p2[c] = p3[c];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // the structure function over the 26 neighbours
+#pragma unroll
+        for (int di = -1; di <= 1; ++di) {
+            const double(*p)[kSgsTile] = tile[(i + di) & 3];
+#pragma unroll
+            for (int dj = -1; dj <= 1; ++dj)
+#pragma unroll
+                for (int dk = -1; dk <= 1; ++dk) {
+                    if (!(di || dj || dk)) continue;
+                    const int o = own + dj * kSgsW + dk;
+                    const double du = p[0][o] - f0[0], dv = p[1][o] - f0[1], dw = p[2][o] - f0[2];
+                    F2 += du * du + dv * dv + dw * dw;
+                }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // (summed here, not where it is used: the 81 values would be held until then)
+        asm volatile("" : "+v"(F2));
+        if (!on) continue;
+        const double S[6] = {0.5 * (g[0][0] + g[0][0]), 0.5 * (g[1][1] + g[1][1]), 0.5 * (g[2][2] + g[2][2]),
+                             0.5 * (g[0][1] + g[1][0]), 0.5 * (g[1][2] + g[2][1]), 0.5 * (g[2][0] + g[0][2])};
+        double T[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, K = 0.0, e[3], ax;
+        if (sgs_axis(S, e, ax)) {
+            const double lv = sqrt(2.0 * nu / (3.0 * (fabs(ax) + kSgsEps)));
+            const double dxp = G.xc[0][i + 1] - G.xc[0][i], dxm = G.xc[0][i - 1] - G.xc[0][i];
+            const double del = cbrt(-dxm * -dym * -dzm);
+            // sfIntegral of each neighbour offset's distance from the vortex
+            // axis.  The distance is even in the offset, so where the spacing on
+            // the two sides of the cell agrees to rounding (uniform axes) each of
+            // the 13 offsets of one half stands for its mirror image too;
+            // elsewhere all 26 are evaluated.
+            const bool mirror = mirror_yz && close(dxp, dxm);
+            double Qd = 0.0;
+            if (SF32) {
+                const float sx[3] = {(float)dxm, 0.0f, (float)dxp}, sy[3] = {(float)dym, 0.0f, (float)dyp};
+                const float sz[3] = {(float)dzm, 0.0f, (float)dzp}, fe[3] = {(float)e[0], (float)e[1], (float)e[2]};
+                const float fdel = (float)del, idel = 1.0f / fdel;
+                auto term = [&](float dx, float dy, float dz) __attribute__((always_inline)) {
+                    const float dx2 = dx * dx + dy * dy + dz * dz, dxe = dx * fe[0] + dy * fe[1] + dz * fe[2];
+                    return (double)sf_integral_f(quot_rn(sqrt_rn(dx2 - dxe * dxe), fdel, idel));
+                };
+                if (mirror) {
+                    // the 13 offsets before (0, 0, 0) in (di, dj, dk) order
+#pragma unroll
+                    for (int t = 0; t < 13; ++t) Qd += 2.0 * term(sx[t / 9], sy[(t / 3) % 3], sz[t % 3]);
+                } else {
+#pragma unroll 1
+                    for (int t = 0; t < 27; ++t) {
+                        const int a = t / 9, b = (t / 3) % 3, c = t % 3;
+                        if (t != 13)
+                            Qd += term(a == 0 ? sx[0] : a == 1 ? 0.0f : sx[2], b == 0 ? sy[0] : b == 1 ? 0.0f : sy[2],
+                                       c == 0 ? sz[0] : c == 1 ? 0.0f : sz[2]);
+                    }
+                }
+            } else {
+                const int nt = mirror ? 13 : 27;
+#pragma unroll 1
+                for (int t = 0; t < nt; ++t) {
+                    const int a = t / 9, b = (t / 3) % 3, c = t % 3;
+                    if (t == 13) continue;
+                    const double dx = a == 0 ? dxm : a == 1 ? 0.0 : dxp, dy = b == 0 ? dym : b == 1 ? 0.0 : dyp;
+                    const double dz = c == 0 ? dzm : c == 1 ? 0.0 : dzp;
+                    const double dx2 = dx * dx + dy * dy + dz * dz, dxe = dx * e[0] + dy * e[1] + dz * e[2];
+                    const double v = sf_integral(sqrt(dx2 - dxe * dxe) / del);
+                    Qd += mirror ? 2.0 * v : v;
+                }
+            }
+            K = F2 / Qd * ke_integral(kPi / del * lv);   // (both over the same 26 neighbours)
+            T[0] = (1.0 - e[0] * e[0]) * K;
+            T[1] = (1.0 - e[1] * e[1]) * K;
+            T[2] = (1.0 - e[2] * e[2]) * K;
+            T[3] = (-e[0] * e[1]) * K;
+            T[4] = (-e[1] * e[2]) * K;
+            T[5] = (-e[2] * e[0]) * K;
+        } else {
+            failed = true;
+        }
+        const long idx = (long)i * G.sx + oc;
+#pragma unroll
+        for (int m = 0; m < 6; ++m) __builtin_nontemporal_store(T[m], A.T[m] + idx);
+        const double volA = inx / G.xi_x[0][i];
+        sum[0] += fabs(K) * volA * volB * volC;
+        const double dis = -(S[0] * T[0] + S[1] * T[1] + S[2] * T[2] + 2.0 * (S[3] * T[3] + S[4] * T[4] + S[5] * T[5]));
+        sum[1] += dis * volA * volB * volC;
+        const double s2 = S[0] * S[0] + S[1] * S[1] + S[2] * S[2] + 2.0 * (S[3] * S[3] + S[4] * S[4] + S[5] * S[5]);
+        const double t2 = T[0] * T[0] + T[1] * T[1] + T[2] * T[2] + 2.0 * (T[3] * T[3] + T[4] * T[4] + T[5] * T[5]);
+        sum[2] += sqrt(t2 / s2) / 2 * volA * volB * volC;
+    }
+    if (failed) atomicOr(A.fail, 1);
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-        double x = v[q];
+        double x = sum[q];
         for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-        if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = x;
+        if ((tid & 63) == 0) red[q][tid >> 6] = x;
     }
     __syncthreads();
-    if (threadIdx.x < 3) {
-        double x = red[threadIdx.x][0];
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w) x += red[threadIdx.x][w];
-        part[(((long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * 3 + threadIdx.x] = x;
+    if (tid < 3) {
+        double x = red[tid][0];
+        for (int w = 1; w < kSgsThreads / 64; ++w) x += red[tid][w];
+        A.part[(long)lb * 3 + tid] = x;
     }
 }
 
