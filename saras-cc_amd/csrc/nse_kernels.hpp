@@ -1238,6 +1238,86 @@ __global__ void __launch_bounds__(256) k_jacobi(Geom G, CoreField F, const doubl
     if (RES) block_max_store(res, part, ((long)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
 }
 
+// k_jacobi in 3-D where every wall is a plain Dirichlet or Neumann one: a lane
+// keeps its (j, k) and marches along x with the planes behind and ahead in
+// registers and the next plane's values on their way.  k_jacobi already fetches
+// each value once from memory; what bounds it are its 170 instructions a cell
+// (indexes, wraps and wall rules of six neighbours) and its short blocks, and its
+// 150000 partial maxima at 384^3 took another 50 us to reduce.  The march is
+// bound by the latency of a plane's loads: waited for where they are used, without
+// the plane ahead, it took 541 us at 384^3 instead of 389 (k_jacobi: 432).
+// Measured: see launch_jacobi (nse_solver.hip).
+struct JacobiMarch {
+    const double *f, *rhs;
+    double *out, *part;
+    double cst[6];        // ghost = cst - edge (Dirichlet) or edge - cst (Neumann)
+    int dir[6];
+    int len;
+    unsigned nz, ny, nblock;
+};
+constexpr int kJacZ = 64, kJacY = 4;
+
+template <bool RES>
+__global__ void __launch_bounds__(kJacZ * kJacY) k_jacobi_march(Geom G, JacobiMarch A, double dt, double diff, double beta) {
+    using u32 = unsigned;
+    const u32 per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (lb >= A.nblock) return;
+    const u32 bz = lb % A.nz, br = lb / A.nz, by = br % A.ny, chunk = br / A.ny;
+    const int k = (int)bz * kJacZ + (int)(threadIdx.x & (kJacZ - 1)), j = (int)by * kJacY + (int)(threadIdx.x / kJacZ);
+    const int nx = G.n[0], ny = G.n[1], nz = G.n[2];
+    const int i0 = (int)chunk * A.len, i1 = min(nx, i0 + A.len);
+    double res = 0.0;
+    if (k < nz && j < ny) {
+        const u32 oc = (u32)j * (u32)G.sy + (u32)k;
+        const u32 oS = (u32)core_index(G.per[1], j - 1, ny) * (u32)G.sy + (u32)k;
+        const u32 oN = (u32)core_index(G.per[1], j + 1, ny) * (u32)G.sy + (u32)k;
+        const u32 oB = (u32)j * (u32)G.sy + (u32)core_index(G.per[2], k - 1, nz);
+        const u32 oT = (u32)j * (u32)G.sy + (u32)core_index(G.per[2], k + 1, nz);
+        // the ghost across wall w where `at` says the neighbour is one
+        auto rule = [&](int w, bool at, double v) __attribute__((always_inline)) {
+            const double g = A.dir[w] ? A.cst[w] - v : v - A.cst[w];
+            return at && !G.per[w / 2] ? g : v;
+        };
+        auto plane = [&](int i) __attribute__((always_inline)) { return (long)core_index(G.per[0], i, nx) * G.sx; };
+        const double y2 = G.xix2[1][j], yy = G.xixx[1][j], z2 = G.xix2[2][k], zz = G.xixx[2][k];
+        double W = rule(0, i0 == 0, (A.f + plane(i0 - 1))[oc]), C = (A.f + (long)i0 * G.sx)[oc];
+        // a plane's values: rhs, plane i+1, and the y and z neighbours
+        struct Plane { double r, e, n, s, t, b; };
+        auto fetch = [&](int i) __attribute__((always_inline)) {
+            const double *p = A.f + (long)i * G.sx;
+            return Plane{(A.rhs + (long)i * G.sx)[oc], (A.f + plane(i + 1))[oc], p[oN], p[oS], p[oT], p[oB]};
+        };
+        Plane nx_ = fetch(i0);
+        for (int i = i0; i < i1; ++i) {
+            const Plane v = nx_;
+            nx_ = fetch(min(i + 1, nx - 1));
+            const double r = v.r, e = v.e;
+            const double N = rule(3, j == ny - 1, v.n), S = rule(2, j == 0, v.s);
+            const double Tp = rule(5, k == nz - 1, v.t), B = rule(4, k == 0, v.b);
+            const double E = rule(1, i == nx - 1, e);
+            const double x2 = G.xix2[0][i], xx = G.xixx[0][i];
+            const double o =
+                ((G.tsih2[0] * x2 * (E + W) + G.tsi2h[0] * xx * (E - W) + G.tsih2[1] * y2 * (N + S) +
+                  G.tsi2h[1] * yy * (N - S) + G.tsih2[2] * z2 * (Tp + B) + G.tsi2h[2] * zz * (Tp - B)) *
+                     dt * diff * beta +
+                 r) /
+                (1.0 + 2.0 * dt * diff * beta * (G.tsih2[0] * x2 + G.tsih2[1] * y2 + G.tsih2[2] * z2));
+            __builtin_nontemporal_store(o, A.out + (long)i * G.sx + oc);
+            if (RES) {
+                const double t = C - beta * dt * diff *
+                                         (x2 * (E - 2.0 * C + W) * G.tsih2[0] + xx * (E - W) * G.tsi2h[0] +
+                                          y2 * (N - 2.0 * C + S) * G.tsih2[1] + yy * (N - S) * G.tsi2h[1] +
+                                          z2 * (Tp - 2.0 * C + B) * G.tsih2[2] + zz * (Tp - B) * G.tsi2h[2]);
+                const double q = fabs(t - r);
+                res = (q > res || q != q) ? q : res;
+            }
+            W = C;
+            C = e;
+        }
+    }
+    if (RES) block_max_store(res, A.part, (long)lb);
+}
+
 // vfield::divergence (vfield.cc:721-737) scaled into the Poisson RHS:
 // b = (((0 + dVx/dx) + dVy/dy) + dVz/dz) * sc   (lsRK3_d3.cc:278-279)
 __global__ void __launch_bounds__(256) k_div(Geom G, CoreField V0, CoreField V1, CoreField V2, double sc,

@@ -52,10 +52,10 @@ const double kZeta[3] = {0.0, -17.0 / 60.0, -5.0 / 12.0};
 // (eight for each CU, so that the last ones do not leave it idle)
 constexpr unsigned kRhsBlocks = 2048;
 
-// planes of a chunk of a march along x over `plane` blocks a plane, and the
-// number of blocks (at most a quarter of nx plane)
-int march_chunk(unsigned plane, int nx, unsigned &nblock) {
-    const unsigned chunks = std::max(1u, std::min((kRhsBlocks + plane - 1) / plane, (unsigned)nx / 4));
+// planes of a chunk (at least `least`) of a march along x over `plane` blocks a
+// plane, and the number of blocks
+int march_chunk(unsigned plane, int nx, int least, unsigned &nblock) {
+    const unsigned chunks = std::max(1u, std::min((kRhsBlocks + plane - 1) / plane, (unsigned)(nx / least)));
     const int len = (int)((nx + chunks - 1) / chunks);
     nblock = plane * (unsigned)((nx + len - 1) / len);
     return len;
@@ -109,6 +109,7 @@ struct saras_nse {
     double wall_area() const { return planar ? g.len[0] : g.len[0] * g.len[1]; }
     int threads = 256;
     bool rhs_march = false;              // the RK3 right-hand sides by k_rhs_march
+    bool jacobi_march[4] = {};           // field q's Crank-Nicolson iterations by k_jacobi_march
     // LES (spiral.cc): sub-grid stresses Txx, Tyy, Tzz, Txy, Tyz, Tzx
     double *Tsg[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     double *sgs_part = nullptr;          // per-block [sum |K| dV, dissipation dV, nu_t dV]
@@ -189,7 +190,7 @@ unsigned launch_sgs(saras_nse *s) {
     A.fail = reinterpret_cast<int *>(s->sgs_dev + 3);
     A.nz = (unsigned)((s->G.n[2] + kSgsZ - 1) / kSgsZ);
     A.ny = (unsigned)((s->G.n[1] + kSgsY - 1) / kSgsY);
-    A.len = march_chunk(A.nz * A.ny, s->G.n[0], A.nblock);
+    A.len = march_chunk(A.nz * A.ny, s->G.n[0], 4, A.nblock);
     const dim3 gr((A.nblock + 7) / 8 * 8), bl(kSgsThreads);
     if (s->p.les_sf32) hipLaunchKernelGGL(k_sgs_stress<true>, gr, bl, 0, s->s, s->G, s->p.nu, A);
     else hipLaunchKernelGGL(k_sgs_stress<false>, gr, bl, 0, s->s, s->G, s->p.nu, A);
@@ -260,7 +261,7 @@ void launch_rhs_march(saras_nse *s, const saras::nse::StageCoef &c, int les) {
     for (int m = 0; m < 6; ++m) A.S[m] = s->Tsg[m];
     A.nz = (unsigned)((s->G.n[2] + kRhsZ - 1) / kRhsZ);
     A.ny = (unsigned)((s->G.n[1] + kRhsY - 1) / kRhsY);
-    A.len = march_chunk(A.nz * A.ny, s->G.n[0], A.nblock);
+    A.len = march_chunk(A.nz * A.ny, s->G.n[0], 4, A.nblock);
     const dim3 gr((A.nblock + 7) / 8 * 8), bl(kRhsZ * kRhsY);
     if (les && s->p.has_T) hipLaunchKernelGGL((k_rhs_march<true, true>), gr, bl, 0, s->s, s->G, c, A);
     else if (les) hipLaunchKernelGGL((k_rhs_march<false, true>), gr, bl, 0, s->s, s->G, c, A);
@@ -312,14 +313,44 @@ saras_status rhs(saras_nse *s, int stage) {
     return SARAS_OK;
 }
 
+// One Jacobi iteration of field f from `in` to `out`; with `res`, the partial
+// maxima of the input's residual in s->part.  Returns their number.  An iteration
+// with its maximum by k_jacobi / k_jacobi_march: 256^3 154 / 122 us, 384^3 486 /
+// 393 us (84 and 283 at the copy rate).
+long launch_jacobi(saras_nse *s, int f, const double *in, double *out, double diff, double beta, bool res) {
+    using namespace saras::nse;
+    const double dt = s->p.dt;
+    if (!s->jacobi_march[f]) {
+        const CoreField F{const_cast<double *>(in), s->bc[f]};
+        if (res) hipLaunchKernelGGL(k_jacobi<true>, s->grid3(), dim3(s->threads), 0, s->s, s->G, F, s->R[f], out, dt, diff, beta, s->part);
+        else hipLaunchKernelGGL(k_jacobi<false>, s->grid3(), dim3(s->threads), 0, s->s, s->G, F, s->R[f], out, dt, diff, beta, nullptr);
+        return s->nblocks;
+    }
+    const FieldBC &b = s->bc[f];
+    JacobiMarch A{};
+    A.f = in;
+    A.rhs = s->R[f];
+    A.out = out;
+    A.part = s->part;
+    for (int w = 0; w < 6; ++w) {
+        A.dir[w] = b.type[w] == 0;
+        A.cst[w] = b.type[w] == 0 ? 2.0 * b.val[w] : b.kh[w];
+    }
+    A.nz = (unsigned)((s->G.n[2] + kJacZ - 1) / kJacZ);
+    A.ny = (unsigned)((s->G.n[1] + kJacY - 1) / kJacY);
+    A.len = march_chunk(A.nz * A.ny, s->G.n[0], 2, A.nblock);
+    const dim3 gr((A.nblock + 7) / 8 * 8), bl(kJacZ * kJacY);
+    if (res) hipLaunchKernelGGL(k_jacobi_march<true>, gr, bl, 0, s->s, s->G, A, dt, diff, beta);
+    else hipLaunchKernelGGL(k_jacobi_march<false>, gr, bl, 0, s->s, s->G, A, dt, diff, beta);
+    return A.nblock;
+}
+
 // timestep::solveVx/Vy/Vz/solveT: Jacobi iterations until the residual of the
 // updated field is below cn_tol, at most maxIterations extra iterations.
 saras_status solve_field(saras_nse *s, int f, double beta, int *iters) {
     const double diff = f == 3 ? s->p.kappa : s->p.nu;
-    const double dt = s->p.dt;
     double *cur = s->scratch, *other = s->F[f];
-    hipLaunchKernelGGL(saras::nse::k_jacobi<false>, s->grid3(), dim3(s->threads), 0, s->s, s->G,
-                       CoreField{s->F[f], s->bc[f]}, s->R[f], cur, dt, diff, beta, nullptr);
+    launch_jacobi(s, f, s->F[f], cur, diff, beta, false);
     NSE_TRY(hipGetLastError());
     // solveT imposes T's walls after each update (predictors.cc:376): from the
     // first one on, the plume flags see the predicted Vz
@@ -329,9 +360,8 @@ saras_status solve_field(saras_nse *s, int f, double beta, int *iters) {
     }
     int it = 0;
     for (;;) {
-        hipLaunchKernelGGL(saras::nse::k_jacobi<true>, s->grid3(), dim3(s->threads), 0, s->s, s->G,
-                           CoreField{cur, s->bc[f]}, s->R[f], other, dt, diff, beta, s->part);
-        hipLaunchKernelGGL(saras::nse::k_max_final, dim3(1), dim3(1024), 0, s->s, s->part, s->nblocks, s->res_host,
+        const long parts = launch_jacobi(s, f, cur, other, diff, beta, true);
+        hipLaunchKernelGGL(saras::nse::k_max_final, dim3(1), dim3(1024), 0, s->s, s->part, parts, s->res_host,
                            s->res_seq, ++s->res_ticket);
         NSE_TRY(hipGetLastError());
         NSE_TRY(saras::wait_ticket(s->res_seq, s->res_ticket, s->s));
@@ -805,7 +835,7 @@ saras_status saras_nse_create(const saras_grid_desc *grid, const saras_mg_params
         s->nblocks = (long)gr.x * gr.y * gr.z;
     }
     {
-        const char *env = std::getenv("SARAS_NO_RHS_MARCH");
+        const char *env = std::getenv("SARAS_NO_NSE_MARCH");
         // dScheme 2 with Morinishi's term in boxes periodic in x and y, whose z
         // walls are none or plain Dirichlet / Neumann ones (no stored ghosts, no
         // column flags, the z edge test at the last cell); every other form
@@ -817,6 +847,13 @@ saras_status saras_nse_create(const saras_grid_desc *grid, const saras_mg_params
             ok = ok && (g.periodic[2] || (b.type[4] <= 1 && b.type[5] <= 1 && !b.top2)) && g.n[0] >= 4;
         }
         s->rhs_march = ok;
+        // (rows of one cell along y are the planar grids)
+        const bool march3 = !planar && g.n[1] > 1 && !(env && env[0] == '1');
+        for (int q = 0; q < 4; ++q) {
+            s->jacobi_march[q] = march3;
+            for (int w = 0; w < 6; ++w)
+                s->jacobi_march[q] = s->jacobi_march[q] && (g.periodic[w / 2] || s->bc[q].type[w] <= 1);
+        }
     }
     if (hipMalloc((void **)&s->part, sizeof(double) * s->nblocks) != hipSuccess) return fail(SARAS_OOM);
     // written by the maximum's last reduction directly (pinned, host-coherent)
