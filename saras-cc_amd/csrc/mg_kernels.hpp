@@ -633,6 +633,31 @@ __global__ void __launch_bounds__(1024) k_coarse(LevelArgs<T> L, T *__restrict__
     if (threadIdx.x == 0 && ctl.mode == 0 && ctl.iters_out) *ctl.iters_out = iter;
 }
 
+// One colour pass of a coarsest level that k_coarse would hold in global memory,
+// out of place: cells of `colour` take their update from x, the others their own
+// value.  Read from the array as it was before the pass, a periodic neighbour is
+// the ghost k_coarse refreshes before it (also where an odd extent makes the two
+// cells one colour), and a wall's ghost follows from the cell beside it, which no
+// pass but its own changes.  Measured: see Ops::coarse (mg_solver.hip).
+template <typename T, int DIM>
+__global__ void __launch_bounds__(256) k_coarse_pass(LevelArgs<T> L, const T *__restrict__ x, T *__restrict__ out,
+                                                     const T *__restrict__ b, int colour, T w) {
+    const int ny = L.n[1], nz = L.n[2];
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (long)L.n[0] * ny * nz) return;
+    int i, j, k;
+    cell_of(t, ny, nz, i, j, k);
+    const long idx = (long)i * L.sx + (long)j * L.sy + kof(L, k);
+    T v = x[idx];
+    if (((i + j + k) & 1) == colour) {
+        Stencil<T, DIM> s;
+        gather<T, DIM>(L, x, i, j, k, idx, s);
+        const T c2y = DIM == 3 ? L.c2[1][j] : T(0), c1y = DIM == 3 ? L.c1[1][j] : T(0);
+        v = sor_update<T, DIM>(s, L.c2[0][i], L.c1[0][i], c2y, c1y, L.c2[2][k], L.c1[2][k], b[idx], w);
+    }
+    out[idx] = v;
+}
+
 // ---------------------------------------------------------------------------
 // transfers between the caller's padded field arrays and the core layout
 // ---------------------------------------------------------------------------
