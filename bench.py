@@ -70,13 +70,13 @@ import saras_amd as S  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
 N = 256
-DOMINANT = "k_rb_split<float,3,0,true,true,false>"
+DOMINANT = "k_rb_split<float,3,0,true,true,0>"
 # HBM bytes per launch of the dominant kernel (one FP32 colour pass of the
 # finest level of the z-periodic 256^3 grid, SOR parameter 1) from rocprofv3
 # --pmc FETCH_SIZE / WRITE_SIZE (KiB per dispatch), calibrated against the
-# copy kernel (FETCH x 2.0, WRITE x 1.0): (2 * 33873.2 + 32768.0) KiB.
+# copy kernel (FETCH x 2.0, WRITE x 1.0): (2 * 33819.6 + 32768.0) KiB.
 # Source: profiles/headline_sweep_hbm_traffic.md
-DOMINANT_TRAFFIC_BYTES = (2 * 33873.2 + 32768.0) * 1024
+DOMINANT_TRAFFIC_BYTES = (2 * 33819.6 + 32768.0) * 1024
 
 
 def bytes_per_vcycle(shapes, s, nu1, nu2):
@@ -453,9 +453,9 @@ def les_history(steps, n=384, sf32=1):
 
 # FP64 operations per cell of the sub-grid stress kernel at 384^3, from
 # rocprofv3 --pmc SQ_INSTS_VALU_{ADD,MUL,FMA,TRANS}_F64 (wave instructions x
-# 64 lanes, an FMA counted twice): 199.2 GFLOP per launch.
+# 64 lanes, an FMA counted twice): 175.3 GFLOP per launch.
 # Source: profiles/les_step_384cubed.md
-SGS_FLOP_PER_CELL = 3518.1
+SGS_FLOP_PER_CELL = 3095.1
 FP64_VECTOR_PEAK_TFLOPS = 78.6
 
 
