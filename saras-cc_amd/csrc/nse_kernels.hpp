@@ -1377,6 +1377,141 @@ __global__ void __launch_bounds__(256) k_correct(Geom G, PF Pp, double *__restri
     V2[idx] -= g2;
 }
 
+// k_div and k_correct in 3-D with dScheme 2 where every wall is a plain Dirichlet
+// or Neumann one: a lane marches along x with the five planes of the x stencil in registers
+// and the next plane's values on their way, as k_jacobi_march does.  Cell by
+// cell they ran at 3.0 and 3.8 TB/s (384^3), bound by the index and wall rules of
+// twelve neighbours and by rows re-read on other XCDs.
+// Measured: see launch_div and launch_correct (nse_solver.hip).
+struct WallField {
+    const double *f;
+    double cst[6];   // ghost = cst - edge (Dirichlet) or edge - cst (Neumann)
+    int dir[6];
+};
+struct GradMarch {
+    int len;
+    unsigned nz, ny, nblock;
+};
+
+// the column of a lane: offsets of its cell and of its y and z neighbours at -2, -1, 1, 2
+struct GradCol {
+    int i0, i1, j, k;
+    bool on;
+    unsigned oc, oy[4], oz[4];
+    __device__ __forceinline__ GradCol(const Geom &G, const GradMarch &A, unsigned lb, long hz) {
+        const unsigned bz = lb % A.nz, br = lb / A.nz, by = br % A.ny, chunk = br / A.ny;
+        k = (int)bz * kJacZ + (int)(threadIdx.x & (kJacZ - 1));
+        j = (int)by * kJacY + (int)(threadIdx.x / kJacZ);
+        i0 = (int)chunk * A.len;
+        i1 = min(G.n[0], i0 + A.len);
+        on = k < G.n[2] && j < G.n[1];
+        // element q of a row: contiguous, or split by colour (hz > 0)
+        auto zo = [&](int q) { return hz ? (unsigned)((q & 1) * hz + (q >> 1)) : (unsigned)q; };
+        const unsigned sy = (unsigned)G.sy;
+        const int jj = min(j, G.n[1] - 1), kk = min(k, G.n[2] - 1);
+        oc = (unsigned)jj * sy + zo(kk);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const int s = d < 2 ? d - 2 : d - 1;
+            oy[d] = (unsigned)core_index(G.per[1], jj + s, G.n[1]) * sy + zo(kk);
+            oz[d] = (unsigned)jj * sy + zo(core_index(G.per[2], kk + s, G.n[2]));
+        }
+    }
+};
+// value at index q along ax of a field, v being the core value its index maps to
+__device__ __forceinline__ double wall_of(const Geom &G, const WallField &F, int ax, int q, double v) {
+    if (G.per[ax]) return v;
+    const double lo = F.dir[2 * ax] ? F.cst[2 * ax] - v : v - F.cst[2 * ax];
+    const double hi = F.dir[2 * ax + 1] ? F.cst[2 * ax + 1] - v : v - F.cst[2 * ax + 1];
+    return q < 0 ? lo : (q >= G.n[ax] ? hi : v);
+}
+// d1 (dScheme 2) along ax at index q from the four core values around it
+__device__ __forceinline__ double d1_four(const Geom &G, const WallField &F, int ax, int q, double m, const double (&c)[4]) {
+    double v[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) v[d] = wall_of(G, F, ax, q + (d < 2 ? d - 2 : d - 1), c[d]);
+    double t = (8.0 * (v[2] - v[1]) - (v[3] - v[0])) * kRecip12;
+    if (q == 0 || q == G.n[ax] - 1) t = 0.5 * (v[2] - v[1]);
+    return m * (t * G.ih[ax]);
+}
+
+__global__ void __launch_bounds__(kJacZ * kJacY) k_div_march(Geom G, GradMarch A, WallField U, WallField V, WallField W,
+                                                             double sc, double *__restrict__ b, long bsx, long bsy, long bhz) {
+    const unsigned per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (lb >= A.nblock) return;
+    const GradCol C(G, A, lb, 0);
+    if (!C.on) return;
+    const int nx = G.n[0], j = C.j, k = C.k;
+    auto xat = [&](int i) __attribute__((always_inline)) { return (U.f + (long)core_index(G.per[0], i, nx) * G.sx)[C.oc]; };
+    const double ym = G.xi_x[1][j], zm = G.xi_x[2][k];
+    double *const out = b + (long)j * bsy + (bhz ? (long)(k & 1) * bhz + (k >> 1) : (long)k);
+    double u[5], y[4], z[4];   // u: planes i-2 .. i+2; y, z: the next plane's
+#pragma unroll
+    for (int o = 0; o < 5; ++o) u[o] = xat(C.i0 + o - 2);
+    auto fetch = [&](int i) __attribute__((always_inline)) {
+        const double *v = V.f + (long)i * G.sx, *w = W.f + (long)i * G.sx;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            y[d] = v[C.oy[d]];
+            z[d] = w[C.oz[d]];
+        }
+    };
+    fetch(C.i0);
+    for (int i = C.i0; i < C.i1; ++i) {
+        const double cx[4] = {u[0], u[1], u[3], u[4]}, cy[4] = {y[0], y[1], y[2], y[3]}, cz[4] = {z[0], z[1], z[2], z[3]};
+#pragma unroll
+        for (int o = 0; o < 4; ++o) u[o] = u[o + 1];
+        u[4] = xat(i + 3);
+        fetch(min(i + 1, nx - 1));
+        double d = 0.0;
+        d += d1_four(G, U, 0, i, G.xi_x[0][i], cx);
+        d += d1_four(G, V, 1, j, ym, cy);
+        d += d1_four(G, W, 2, k, zm, cz);
+        out[(long)i * bsx] = d * sc;
+    }
+}
+
+__global__ void __launch_bounds__(kJacZ * kJacY) k_correct_march(Geom G, GradMarch A, WallField Pp, long hz,
+                                                                 double *__restrict__ P, double *__restrict__ V0,
+                                                                 double *__restrict__ V1, double *__restrict__ V2, double pc) {
+    const unsigned per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (lb >= A.nblock) return;
+    const GradCol C(G, A, lb, hz);
+    if (!C.on) return;
+    const int nx = G.n[0], j = C.j, k = C.k;
+    auto xat = [&](int i) __attribute__((always_inline)) { return (Pp.f + (long)core_index(G.per[0], i, nx) * G.sx)[C.oc]; };
+    const double ym = G.xi_x[1][j], zm = G.xi_x[2][k];
+    double p[5], y[4], z[4];
+#pragma unroll
+    for (int o = 0; o < 5; ++o) p[o] = xat(C.i0 + o - 2);
+    auto fetch = [&](int i) __attribute__((always_inline)) {
+        const double *v = Pp.f + (long)i * G.sx;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            y[d] = v[C.oy[d]];
+            z[d] = v[C.oz[d]];
+        }
+    };
+    fetch(C.i0);
+    const unsigned o0 = (unsigned)j * (unsigned)G.sy + (unsigned)k;
+    for (int i = C.i0; i < C.i1; ++i) {
+        const long pl = (long)i * G.sx;
+        const double q = (P + pl)[o0], a = (V0 + pl)[o0], b = (V1 + pl)[o0], c = (V2 + pl)[o0];
+        const double cx[4] = {p[0], p[1], p[3], p[4]}, cy[4] = {y[0], y[1], y[2], y[3]}, cz[4] = {z[0], z[1], z[2], z[3]};
+        const double own = p[2];
+#pragma unroll
+        for (int o = 0; o < 4; ++o) p[o] = p[o + 1];
+        p[4] = xat(i + 3);
+        fetch(min(i + 1, nx - 1));
+        const double g0 = d1_four(G, Pp, 0, i, G.xi_x[0][i], cx) * pc, g1 = d1_four(G, Pp, 1, j, ym, cy) * pc;
+        const double g2 = d1_four(G, Pp, 2, k, zm, cz) * pc;
+        (P + pl)[o0] = q + own;
+        (V0 + pl)[o0] = a - g0;
+        (V1 + pl)[o0] = b - g1;
+        (V2 + pl)[o0] = c - g2;
+    }
+}
+
 // tseries diagnostics, per-block partial sums (tseries.cc:209-290):
 // [0] sum KE dVol, [1] sum Vz T dVol, [2] max |div V|, [3] sum bottom-wall dTdn dA,
 // [4] sum top-wall dTdn dA.  dxi = 1/n per axis; wall_dn = the top-wall distance.

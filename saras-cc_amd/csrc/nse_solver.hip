@@ -109,6 +109,7 @@ struct saras_nse {
     double wall_area() const { return planar ? g.len[0] : g.len[0] * g.len[1]; }
     int threads = 256;
     bool rhs_march = false;              // the RK3 right-hand sides by k_rhs_march
+    bool div_march = false, correct_march = false;   // k_div_march, k_correct_march
     bool jacobi_march[4] = {};           // field q's Crank-Nicolson iterations by k_jacobi_march
     // LES (spiral.cc): sub-grid stresses Txx, Tyy, Tzz, Txy, Tyz, Tzx
     double *Tsg[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -313,6 +314,56 @@ saras_status rhs(saras_nse *s, int stage) {
     return SARAS_OK;
 }
 
+// a field of a march along x: its core and its walls' rules
+saras::nse::WallField wall_field(const double *f, const FieldBC &b) {
+    saras::nse::WallField F{};
+    F.f = f;
+    for (int w = 0; w < 6; ++w) {
+        F.dir[w] = b.type[w] == 0;
+        F.cst[w] = b.type[w] == 0 ? 2.0 * b.val[w] : b.kh[w];
+    }
+    return F;
+}
+saras::nse::GradMarch grad_march(const saras_nse *s) {
+    using namespace saras::nse;
+    GradMarch A{};
+    A.nz = (unsigned)((s->G.n[2] + kJacZ - 1) / kJacZ);
+    A.ny = (unsigned)((s->G.n[1] + kJacY - 1) / kJacY);
+    A.len = march_chunk(A.nz * A.ny, s->G.n[0], 2, A.nblock);
+    return A;
+}
+
+// div V into the pressure solver's right-hand side.  k_div / k_div_march: 64^3 8.3 /
+// 6.9 us, 160^3 54 / 43, 256^3 200 / 139, 384^3 593 / 459.
+void launch_div(saras_nse *s, double sc, double *b, long bsx, long bsy, long bhz) {
+    using namespace saras::nse;
+    if (s->div_march) {
+        const GradMarch A = grad_march(s);
+        hipLaunchKernelGGL(k_div_march, dim3((A.nblock + 7) / 8 * 8), dim3(kJacZ * kJacY), 0, s->s, s->G, A,
+                           wall_field(s->F[0], s->bc[0]), wall_field(s->F[1], s->bc[1]), wall_field(s->F[2], s->bc[2]), sc, b,
+                           bsx, bsy, bhz);
+    } else
+        hipLaunchKernelGGL(k_div, s->grid3(), dim3(s->threads), 0, s->s, s->G, s->field(0), s->field(1), s->field(2), sc, b,
+                           bsx, bsy, bhz);
+}
+
+// The pressure correction.  k_correct / k_correct_march: 64^3 10.2 / 9.2 us, 160^3
+// 84 / 79, 256^3 318 / 279, 384^3 1078 / 940 (850 at the copy rate).
+void launch_correct(saras_nse *s, double pc) {
+    using namespace saras::nse;
+    const SplitField pp = s->pp();
+    if (s->correct_march) {
+        const GradMarch A = grad_march(s);
+        hipLaunchKernelGGL(k_correct_march, dim3((A.nblock + 7) / 8 * 8), dim3(kJacZ * kJacY), 0, s->s, s->G, A,
+                           wall_field(pp.f, pp.bc), pp.hz, s->F[4], s->F[0], s->F[1], s->F[2], pc);
+    } else if (pp.hz)
+        hipLaunchKernelGGL(k_correct<SplitField>, s->grid3(), dim3(s->threads), 0, s->s, s->G, pp, s->F[4], s->pbc, s->F[0],
+                           s->F[1], s->F[2], pc);
+    else
+        hipLaunchKernelGGL(k_correct<CoreField>, s->grid3(), dim3(s->threads), 0, s->s, s->G, CoreField{pp.f, pp.bc}, s->F[4],
+                           s->pbc, s->F[0], s->F[1], s->F[2], pc);
+}
+
 // One Jacobi iteration of field f from `in` to `out`; with `res`, the partial
 // maxima of the input's residual in s->part.  Returns their number.  An iteration
 // with its maximum by k_jacobi / k_jacobi_march: 256^3 154 / 122 us, 384^3 486 /
@@ -402,19 +453,11 @@ saras_status stage_run(saras_nse *s, int stage) {
     long sx0, sy0, hz0;
     saras::mg_level0(s->mg, &x0, &b0, &sx0, &sy0, &hz0);
     const double sc = euler ? 1.0 / s->p.dt : 1.0 / ((a + b) * s->p.dt);
-    hipLaunchKernelGGL(saras::nse::k_div, s->grid3(), dim3(s->threads), 0, s->s, s->G, s->field(0), s->field(1),
-                       s->field(2), sc, b0, sx0, sy0, hz0);
+    launch_div(s, sc, b0, sx0, sy0, hz0);
     NSE_TRY(hipGetLastError());
     e = saras::mg_solve_resident(s->mg, s->s, &s->mg_stats);
     if (e && e != SARAS_NOT_CONVERGED) return e;
-    const double pc = euler ? s->p.dt : (a + b) * s->p.dt;
-    const saras::nse::SplitField pp = s->pp();
-    if (pp.hz)
-        hipLaunchKernelGGL(saras::nse::k_correct<saras::nse::SplitField>, s->grid3(), dim3(s->threads), 0, s->s, s->G,
-                           pp, s->F[4], s->pbc, s->F[0], s->F[1], s->F[2], pc);
-    else
-        hipLaunchKernelGGL(saras::nse::k_correct<CoreField>, s->grid3(), dim3(s->threads), 0, s->s, s->G,
-                           CoreField{pp.f, pp.bc}, s->F[4], s->pbc, s->F[0], s->F[1], s->F[2], pc);
+    launch_correct(s, euler ? s->p.dt : (a + b) * s->p.dt);
     NSE_TRY(hipGetLastError());
     // V.imposeBCs(); P.imposeBCs(); T.imposeBCs() closing the stage
     return plume_flags(s);
@@ -847,13 +890,27 @@ saras_status saras_nse_create(const saras_grid_desc *grid, const saras_mg_params
             ok = ok && (g.periodic[2] || (b.type[4] <= 1 && b.type[5] <= 1 && !b.top2)) && g.n[0] >= 4;
         }
         s->rhs_march = ok;
-        // (rows of one cell along y are the planar grids)
+        // Jacobi iterations march where their three arrays exceed the 256 MB
+        // Infinity Cache: served from it, cell by cell is as fast (128^3 and
+        // 160^3: 19.5 and 36.9 us against 20.9 and 38.8; 256^3 154 against 122
+        // with the maximum).  SARAS_NO_NSE_MARCH=0 lets every size march.
+        // (Rows of one cell along y are the planar grids.)
         const bool march3 = !planar && g.n[1] > 1 && !(env && env[0] == '1');
+        const bool large = (env && env[0] == '0') || s->elems * 3 * sizeof(double) > (size_t)256 << 20;
+        bool plain[4];
         for (int q = 0; q < 4; ++q) {
-            s->jacobi_march[q] = march3;
-            for (int w = 0; w < 6; ++w)
-                s->jacobi_march[q] = s->jacobi_march[q] && (g.periodic[w / 2] || s->bc[q].type[w] <= 1);
+            plain[q] = march3;
+            for (int w = 0; w < 6; ++w) plain[q] = plain[q] && (g.periodic[w / 2] || s->bc[q].type[w] <= 1);
+            s->jacobi_march[q] = plain[q] && large;
         }
+        // divergence and correction with second-order differences load half of
+        // the neighbours, which the march does not save (72x56x100: 7.8 and
+        // 10.0 us cell by cell against 8.9 and 12.0)
+        s->div_march = P.dscheme == 2 && plain[0] && plain[1] && plain[2];
+        // (the correction has a stored ghost of P to carry along beside other walls)
+        s->correct_march = march3 && P.dscheme == 2;
+        for (int w = 0; w < 6; ++w)
+            s->correct_march = s->correct_march && (g.periodic[w / 2] || (s->pbc.type[w] <= 1 && s->ppbc.type[w] <= 1));
     }
     if (hipMalloc((void **)&s->part, sizeof(double) * s->nblocks) != hipSuccess) return fail(SARAS_OOM);
     // written by the maximum's last reduction directly (pinned, host-coherent)

@@ -1,5 +1,6 @@
-"""The marching right-hand side (k_rhs_march) and Jacobi iteration
-(k_jacobi_march) against the kernels per field, bit for bit: rows shorter and longer than a block, part-filled blocks in y and z,
+"""The marching right-hand side (k_rhs_march), Jacobi iteration (k_jacobi_march),
+divergence and pressure correction (k_div_march, k_correct_march) against the
+kernels per field and per cell, bit for bit: rows shorter and longer than a block, part-filled blocks in y and z,
 one chunk of planes and several, z walls of both kinds with values and without
 walls, with and without temperature, with and without the sub-grid stresses.
 """
@@ -77,7 +78,7 @@ def test_walls_on_every_side(n, scheme, monkeypatch):
         monkeypatch.setenv("SARAS_NO_NSE_MARCH", "0" if march else "1")
         g = S.grid_desc(n, periodic=(0, 0, 0), gtype=(2, 0, 1), beta=(1.1, 1.0, 0.8), pad=2)
         vbc = [([(D, N)[(w + q) % 2] for w in range(6)], [0.1 * w - 0.2 * q for w in range(6)]) for q in range(3)]
-        p = S.nse_params(dscheme=1, nlscheme=1, has_T=1, nu=2e-2, kappa=3e-2, dt=2e-3, cn_tol=1e-9, scheme=scheme, vbc=vbc,
+        p = S.nse_params(dscheme=2, nlscheme=1, has_T=1, nu=2e-2, kappa=3e-2, dt=2e-3, cn_tol=1e-9, scheme=scheme, vbc=vbc,
                          tbc=([N, D, D, N, D, D], [0.3, -0.1, 0.2, 0.0, 1.0, -1.0]), buoy=(0.1, 0.0, -0.9))
         mg = S.mg_params(bc=S.BC_NEUMANN, precision=S.PREC_FP64, vc_count=2, vc_tol=1e-6, solve_flag=0, pre=2, post=2)
         return S.Nse(g, mg, p)
