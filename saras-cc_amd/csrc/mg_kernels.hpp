@@ -435,23 +435,13 @@ struct CoarseCtl {
     double rel_floor;
 };
 
-// Phases of the ghost-array loops below run either on the whole workgroup
-// (separated by barriers) or, for levels of a few hundred cells, on wave 0
-// alone: LDS operations of one wavefront execute in issue order, so a
-// compiler-level fence is all that separates its phases.
+// Between phases that wave 0 runs alone (the tail's levels of at most a
+// wavefront): LDS operations of one wavefront execute in issue order, so a
+// compiler-level fence is all that separates them.
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-template <bool WAVE>
-__device__ __forceinline__ void lsync() {
-    if (WAVE) wave_lds_sync();
-    else __syncthreads();
-}
-template <bool WAVE>
-__device__ __forceinline__ int lthreads() {
-    return WAVE ? 64 : (int)blockDim.x;
 }
 
 // max over the workgroup (WAVE: over wave 0) of one value per thread, the
@@ -483,10 +473,10 @@ __device__ __forceinline__ T wall_rule(int bc, T inner, T wv) {
 // poisson_d3.cc:876-993).  Only ghosts beside core cells are written -- the
 // edges and corners of the shell are never read by the 7-point stencil -- so
 // every write reads core cells alone and one barrier covers all faces.
-template <typename T, int DIM, bool WAVE = false>
+template <typename T, int DIM>
 __device__ void coarse_ghosts(T *X, const LevelArgs<T> &L, const int *per, bool walls, int PY, int PZ) {
     const int nx = L.n[0], ny = DIM == 3 ? L.n[1] : 1, nz = L.n[2];
-    const int tid = threadIdx.x, nt = lthreads<WAVE>();
+    const int tid = threadIdx.x, nt = blockDim.x;
     const int fx = (per[0] || walls) ? ny * nz : 0;
     const int fy = DIM == 3 && (per[1] || walls) ? nx * nz : 0;
     const int fz = (per[2] || walls) ? nx * ny : 0;
@@ -528,14 +518,14 @@ __device__ void coarse_ghosts(T *X, const LevelArgs<T> &L, const int *per, bool 
             }
         }
     }
-    lsync<WAVE>();
+    __syncthreads();
 }
 
-template <typename T, int DIM, bool WAVE = false>
+template <typename T, int DIM>
 __device__ void coarse_colour(T *X, const T *B, const LevelArgs<T> &L, int colour, T w, int PY, int PZ) {
     const int nx = L.n[0], ny = L.n[1], nz = L.n[2];
     const long total = (long)nx * ny * nz;
-    for (long t = threadIdx.x; t < total; t += lthreads<WAVE>()) {
+    for (long t = threadIdx.x; t < total; t += blockDim.x) {
         int i, j, k;
         cell_of(t, ny, nz, i, j, k);
         if (((i + j + k) & 1) != colour) continue;
@@ -553,7 +543,7 @@ __device__ void coarse_colour(T *X, const T *B, const LevelArgs<T> &L, int colou
         const T c2y = DIM == 3 ? L.c2[1][j] : T(0), c1y = DIM == 3 ? L.c1[1][j] : T(0);
         X[c] = sor_update<T, DIM>(s, L.c2[0][i], L.c1[0][i], c2y, c1y, L.c2[2][k], L.c1[2][k], B[t], w);
     }
-    lsync<WAVE>();
+    __syncthreads();
 }
 
 template <typename T, int DIM>
