@@ -1,0 +1,100 @@
+// mg_plan.hpp -- the tiles of k_tile (mg_tile.hpp): how large they are, which
+// rows of a level each of them touches, and the plan of a V-cycle's visit.
+// Plain arithmetic shared by the host code, the kernel and the CPU tests.
+#pragma once
+#include <algorithm>
+#include <cmath>
+#include <cstddef>
+
+namespace saras {
+
+constexpr int kTileThreads = 512;
+// LDS of a tile (k_tile has no static LDS), of the 160 KB a workgroup may hold
+constexpr size_t kTileLds = 156 * 1024;
+
+// 16-byte vectors of one colour in a row of nz cells of `word` bytes
+constexpr int tile_vecs(size_t word, int nz) { return (nz / 2 + 16 / (int)word - 1) / (16 / (int)word); }
+
+// Rows around a tile that `sweeps` sweeps need: pass p runs on the rows of
+// radius 2 sweeps - 1 - p (one more before a residual) and reads one row
+// further, except that the first pass of a zero iterate reads none.
+constexpr int tile_halo(int sweeps, bool zero, bool restr) { return 2 * sweeps + (restr ? 1 : 0) - (zero ? 1 : 0); }
+
+// LDS bytes of a tile: iterate, right-hand side and the coefficients of its rows
+constexpr size_t tile_bytes(size_t word, int dim, int nz, int ti, int tj, int halo) {
+    const size_t ri = ti + 2 * halo, rj = dim == 3 ? tj + 2 * halo : 1;
+    const size_t row = 2 * (size_t)tile_vecs(word, nz) * 16;
+    return 2 * ri * rj * row + 2 * row + 2 * (ri + rj) * word;
+}
+
+// The rows along one axis (x, or y in 3-D) that tiles work on, numbered without
+// wrapping: the level's n and, on a periodic axis, the `halo` images before and
+// after them.  The last tile of an axis covers rows beyond those where its
+// extent does not divide n; no row of the level needs them, and with
+// halo <= n every row named here is an image at most one extent away.
+struct TileAxis {
+    int n, lo, hi;
+    static constexpr TileAxis of(int n, int halo, bool periodic) {
+        return TileAxis{n, periodic ? -halo : 0, periodic ? n + halo : n};
+    }
+    constexpr bool has(int q) const { return q >= lo && q < hi; }
+    constexpr int row(int q) const { return q < 0 ? q + n : (q >= n ? q - n : q); }   // of a row it has
+};
+
+// The visits of a level by tiles: rows of a tile and sweeps of a launch; none
+// (sweeps 0) where separate passes are faster.
+struct TilePlan {
+    int ti = 0, tj = 0, sweeps = 0;
+};
+
+// The plan of one visit of a level of n cells of `word` bytes, or none where
+// separate passes are faster by this estimate (us).  A kernel takes about 4 us
+// however little it does; a pass beyond that is bound by its 1.5 words per cell
+// at about 7 TB/s (levels of this size sit in the Infinity Cache).  A tile launch
+// adds, per workgroup of a compute unit, its rows' vectors: about kVec cycles of
+// vector issue for 64 of them, and about 350 cycles a pass for the barrier and
+// the LDS latency.  Measured over tiles of 2 to 16 by 1 to 8 rows, 1 to 6 sweeps
+// a launch, 32^3..128^3 and 128^2..2048^2 in both precisions: the estimate's
+// choice is within 3 % of the fastest V-cycle, and turns to separate passes where
+// those are (64^3 with six sweeps FP64, 128^3, 2048^2).
+// split: the level's rows are colour-split.
+inline TilePlan plan_tile(size_t word, int dim, const int (&n)[3], bool split, int count, bool zero, bool pro,
+                          bool restr) {
+    TilePlan best;
+    const int nv = tile_vecs(word, n[2]);
+    if (count < 1 || (n[2] & 1) || nv > kTileThreads) return best;
+    constexpr double kLaunch = 4.0, kVec = 125.0, kClock = 2400.0, kCus = 256.0;
+    const double cells = (double)n[0] * n[1] * n[2];
+    const double pass = std::max(kLaunch + 0.2, 2.8 + 1.5 * cells * word / 7e6);
+    double cost = 2 * count * pass + (restr ? 1.4 * pass : 0.0) + (pro ? 0.4 * pass : 0.0);
+    if (!split && pro) cost += pass;   // a prolongation pass of its own
+    cost *= 0.95;
+    const int jmax = dim == 3 ? 8 : 1;
+    for (int ti = 2; ti <= 32; ti *= 2)
+        for (int tj = dim == 3 ? 2 : 1; tj <= jmax; tj *= 2)
+            for (int s = 1; s <= count; ++s) {
+                double c = 0.0;
+                bool ok = true;
+                for (int done = 0; done < count && ok; done += s) {
+                    const bool z = zero && done == 0, r = restr && done + s >= count;
+                    const int sw = std::min(s, count - done), halo = tile_halo(sw, z, r);
+                    ok = tile_bytes(word, dim, n[2], ti, tj, halo) <= kTileLds && halo <= n[0] &&
+                         (dim == 2 || halo <= n[1]);
+                    auto rows = [&](int q) { return (double)(ti + 2 * q) * (dim == 3 ? tj + 2 * q : 1); };
+                    double vecs = (z ? 1.0 : 1.5) * rows(halo) + (r ? 3.0 * rows(0) : 0.0);
+                    for (int p = 0; p < 2 * sw; ++p) vecs += rows(2 * sw - 1 - p + (r ? 1 : 0));
+                    const double tiles = std::ceil((double)n[0] / ti) * (dim == 3 ? std::ceil((double)n[1] / tj) : 1.0);
+                    const double per_cu = std::max(1.0, tiles / kCus);
+                    c += kLaunch + 1.0 + (std::ceil(per_cu) * vecs * nv / 64.0 * kVec + 350.0 * 2 * sw) / kClock;
+                }
+                if (ok && c < cost) {
+                    cost = c;
+                    best.ti = ti;
+                    best.tj = tj;
+                    best.sweeps = s;
+                }
+            }
+    return best;
+}
+
+}  // namespace saras

@@ -70,9 +70,7 @@ struct DevLevel {
     // the visits of a V-cycle by tiles (k_tile): pre-smoothing from a zero
     // iterate (and, level 0, from any) with the restriction, post-smoothing
     // with the prolongation; no launches: by separate passes
-    struct Tile {
-        int ti = 0, tj = 0, sweeps = 0;   // tile rows, sweeps of a launch
-    } pre, pre0, post;
+    saras::TilePlan pre, pre0, post;
     long hz = 0;        // colour-split rows when > 0 (offset of the odd half)
     T *c2zs = nullptr, *c1zs = nullptr;  // z coefficients in split order
     bool uniform = false;                // every axis has one value of c2 and one of c1
@@ -398,61 +396,15 @@ size_t tail_layout(const saras_mg *m, const Hierarchy<T> &H, int S, saras::TailA
     return bytes <= m->tail_lds && w / words < 65536 ? bytes : 0;
 }
 
-// LDS of a tile (k_tile has no static LDS), of the 160 KB a workgroup may hold
-constexpr size_t kTileLds = 156 * 1024;
-
-// The plan of one visit of level l by tiles, or none where separate passes are
-// faster by this estimate (us).  A kernel takes about 4 us however little it
-// does; a pass beyond that is bound by its 1.5 words per cell at about 7 TB/s
-// (levels of this size sit in the Infinity Cache).  A tile launch adds, per
-// workgroup of a compute unit, its rows' vectors: about kVec cycles of vector
-// issue for 64 of them, and about 350 cycles a pass for the barrier and the LDS
-// latency.  Measured over tiles of 2 to 16 by 1 to 8 rows, 1 to 6 sweeps a
-// launch, 32^3..128^3 and 128^2..2048^2 in both precisions: the estimate's choice
-// is within 3 % of the fastest V-cycle, and turns to separate passes where
-// those are (64^3 with six sweeps FP64, 128^3, 2048^2).
+// The plan of one visit of level l by tiles (none: by separate passes).
 template <typename T>
-typename DevLevel<T>::Tile plan_tile(const saras_mg *m, const Hierarchy<T> &H, int l, int count, bool zero, bool pro,
-                                     bool restr) {
-    typename DevLevel<T>::Tile best;
+saras::TilePlan plan_visit(const saras_mg *m, const Hierarchy<T> &H, int l, int count, bool zero, bool pro, bool restr) {
     const DevLevel<T> &L = H.lv[l];
-    const int nv = saras::tile_vecs<T>(L.n[2]);
-    if (m->tile_off || count < 1 || l + 1 >= (int)H.lv.size() || (L.n[2] & 1) || nv > saras::kTileThreads) return best;
+    if (m->tile_off || l + 1 >= (int)H.lv.size()) return {};
     for (int a = 0; a < 3; ++a)
-        if (m->g.periodic[a] && !(H.dim == 2 && a == 1) && (L.n[a] & 1)) return best;
-    if (l == 0 && m->p.bc == SARAS_BC_DIRICHLET_TEST) return best;
-    constexpr double kLaunch = 4.0, kVec = 125.0, kClock = 2400.0, kCus = 256.0;
-    const double cells = (double)L.n[0] * L.n[1] * L.n[2];
-    const double pass = std::max(kLaunch + 0.2, 2.8 + 1.5 * cells * sizeof(T) / 7e6);
-    double cost = 2 * count * pass + (restr ? 1.4 * pass : 0.0) + (pro ? 0.4 * pass : 0.0);
-    if (!L.hz && pro) cost += pass;   // a prolongation pass of its own
-    cost *= 0.95;
-    const int jmax = H.dim == 3 ? 8 : 1;
-    for (int ti = 2; ti <= 32; ti *= 2)
-        for (int tj = H.dim == 3 ? 2 : 1; tj <= jmax; tj *= 2)
-            for (int s = 1; s <= count; ++s) {
-                double c = 0.0;
-                bool ok = true;
-                for (int done = 0; done < count && ok; done += s) {
-                    const bool z = zero && done == 0, r = restr && done + s >= count;
-                    const int sw = std::min(s, count - done), halo = saras::tile_halo(sw, z, r);
-                    ok = saras::tile_bytes<T>(H.dim, L.n[2], ti, tj, halo) <= kTileLds && halo <= L.n[0] &&
-                         (H.dim == 2 || halo <= L.n[1]);
-                    auto rows = [&](int q) { return (double)(ti + 2 * q) * (H.dim == 3 ? tj + 2 * q : 1); };
-                    double vecs = (z ? 1.0 : 1.5) * rows(halo) + (r ? 3.0 * rows(0) : 0.0);
-                    for (int p = 0; p < 2 * sw; ++p) vecs += rows(2 * sw - 1 - p + (r ? 1 : 0));
-                    const double tiles = std::ceil((double)L.n[0] / ti) * (H.dim == 3 ? std::ceil((double)L.n[1] / tj) : 1.0);
-                    const double per_cu = std::max(1.0, tiles / kCus);
-                    c += kLaunch + 1.0 + (std::ceil(per_cu) * vecs * nv / 64.0 * kVec + 350.0 * 2 * sw) / kClock;
-                }
-                if (ok && c < cost) {
-                    cost = c;
-                    best.ti = ti;
-                    best.tj = tj;
-                    best.sweeps = s;
-                }
-            }
-    return best;
+        if (m->g.periodic[a] && !(H.dim == 2 && a == 1) && (L.n[a] & 1)) return {};
+    if (l == 0 && m->p.bc == SARAS_BC_DIRICHLET_TEST) return {};
+    return saras::plan_tile(sizeof(T), H.dim, L.n, L.hz > 0, count, zero, pro, restr);
 }
 
 // plans of every level, and the second iterate buffer of those that tile
@@ -461,9 +413,9 @@ saras_status plan_tiles(const saras_mg *m, Hierarchy<T> &H) {
     const int D = (int)H.lv.size() - 1;
     for (int l = 0; l < std::min(H.tail_first, D); ++l) {
         DevLevel<T> &L = H.lv[l];
-        L.pre = plan_tile(m, H, l, m->p.pre_smooth, true, false, true);
-        if (l == 0) L.pre0 = plan_tile(m, H, l, m->p.pre_smooth, false, false, true);
-        L.post = plan_tile(m, H, l, m->p.post_smooth, false, true, false);
+        L.pre = plan_visit(m, H, l, m->p.pre_smooth, true, false, true);
+        if (l == 0) L.pre0 = plan_visit(m, H, l, m->p.pre_smooth, false, false, true);
+        L.post = plan_visit(m, H, l, m->p.post_smooth, false, true, false);
         if ((L.pre.sweeps || L.pre0.sweeps || L.post.sweeps) && !L.xalt) {
             HIP_TRY(hipMalloc((void **)&L.xalt, L.elems * sizeof(T)));
             HIP_TRY(hipMemset(L.xalt, 0, L.elems * sizeof(T)));
@@ -932,7 +884,7 @@ struct Ops {
 
     // `count` sweeps of level l by tiles of plan t, at most t.sweeps of them a
     // launch: the first launch takes `zero` or `pro`, the last one `restr`
-    void tile(int l, const typename DevLevel<T>::Tile &t, int count, bool zero, bool pro, bool restr) {
+    void tile(int l, const saras::TilePlan &t, int count, bool zero, bool pro, bool restr) {
         DevLevel<T> &L = H.lv[l];
         const int ntj = H.dim == 3 ? (L.n[1] + t.tj - 1) / t.tj : 1;
         for (int done = 0; done < count; done += t.sweeps) {
@@ -970,9 +922,10 @@ struct Ops {
                     A.R.wd[q] = C.rwd[q];
                 }
             }
-            const size_t bytes = saras::tile_bytes<T>(H.dim, L.n[2], t.ti, t.tj, A.halo);
+            const size_t bytes = saras::tile_bytes(sizeof(T), H.dim, L.n[2], t.ti, t.tj, A.halo);
             // host-side guards of what the kernel assumes
-            if (!L.xalt || bytes > kTileLds || (L.n[2] & 1) || saras::tile_vecs<T>(L.n[2]) > saras::kTileThreads) {
+            if (!L.xalt || bytes > saras::kTileLds || (L.n[2] & 1) || saras::tile_vecs(sizeof(T), L.n[2]) > saras::kTileThreads ||
+                A.halo > L.n[0] || (H.dim == 3 && A.halo > L.n[1])) {
                 refuse("a level that does not tile");
                 return;
             }

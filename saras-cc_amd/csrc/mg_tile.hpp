@@ -28,11 +28,10 @@
 #pragma once
 #include <type_traits>
 
+#include "mg_plan.hpp"
 #include "mg_split.hpp"
 
 namespace saras {
-
-constexpr int kTileThreads = 512;
 
 template <typename T>
 struct TileArgs {
@@ -51,24 +50,6 @@ struct TileArgs {
     T *cb, *cx;
     RestrictArgs<T> R;
 };
-
-// 16-byte vectors of one colour in a row of nz cells
-template <typename T>
-constexpr int tile_vecs(int nz) {
-    return (nz / 2 + 16 / (int)sizeof(T) - 1) / (16 / (int)sizeof(T));
-}
-// Rows around a tile that `sweeps` sweeps need: pass p runs on the rows of
-// radius 2 sweeps - 1 - p (one more before a residual) and reads one row
-// further, except that the first pass of a zero iterate reads none.
-constexpr int tile_halo(int sweeps, bool zero, bool restr) { return 2 * sweeps + (restr ? 1 : 0) - (zero ? 1 : 0); }
-
-// LDS bytes of a tile: iterate, right-hand side and the coefficients of its rows
-template <typename T>
-constexpr size_t tile_bytes(int dim, int nz, int ti, int tj, int halo) {
-    const size_t ri = ti + 2 * halo, rj = dim == 3 ? tj + 2 * halo : 1;
-    const size_t row = 2 * (size_t)tile_vecs<T>(nz) * 16;
-    return 2 * ri * rj * row + 2 * row + 2 * (ri + rj) * sizeof(T);
-}
 
 // What the iterate is at the first pass.
 enum TileMode { TILE_PLAIN, TILE_ZERO, TILE_PRO };
@@ -105,11 +86,9 @@ __global__ void __launch_bounds__(kTileThreads) k_tile(TileArgs<T> A) {
     const bool on = slot < nslot;
     const bool ragged = !HZ && half % W != 0;   // the last vector of a row is not full
 
-    // a row of the level inside the domain: its wrapped index
-    auto wrap = [](int q, int n) __attribute__((always_inline)) { return q < 0 ? q + n : (q >= n ? q - n : q); };
-    auto inside = [&](int i, int j) __attribute__((always_inline)) {
-        return (perx || (i >= 0 && i < nx)) && (DIM == 2 || pery || (j >= 0 && j < ny));
-    };
+    // the rows there are to work on (see TileAxis), by their unwrapped numbers
+    const TileAxis AX = TileAxis::of(nx, H, perx), AY = TileAxis::of(ny, HJ, pery);
+    auto inside = [&](int i, int j) __attribute__((always_inline)) { return AX.has(i) && (DIM == 2 || AY.has(j)); };
     // rows of radius r around the tile, dealt to the thread's slot
     auto rows = [&](int r, auto &&f) __attribute__((always_inline)) {
         const int wi = A.ti + 2 * r, wj = DIM == 3 ? A.tj + 2 * r : 1;
@@ -157,7 +136,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile(TileArgs<T> A) {
                 const bool in = on && q < nrow && inside(i, j);
                 at[u] = in ? q * rs : -1;
                 // a row that does not exist: the tile's first one, not stored
-                const int gi = in ? wrap(i, nx) : i0, gj = in && DIM == 3 ? wrap(j, ny) : j0;
+                const int gi = in ? AX.row(i) : i0, gj = in && DIM == 3 ? AY.row(j) : j0;
                 const long g = (long)gi * L.sx + (long)gj * L.sy;
                 load_pairs(A.b + g, be[u], bo[u]);
                 if constexpr (MODE != TILE_ZERO) load_pairs(A.x + g, xe[u], xo[u]);
@@ -180,7 +159,7 @@ __global__ void __launch_bounds__(kTileThreads) k_tile(TileArgs<T> A) {
                 for (int t = tid; t < RI + (DIM == 3 ? RJ : 0); t += kTileThreads) {
                     const int ax = t < RI ? 0 : 1, n = ax ? ny : nx;
                     const int q = ax ? j0 - HJ + t - RI : i0 - H + t;
-                    const int g = min(max(wrap(q, n), 0), n - 1);
+                    const int g = min(max(ax ? AY.row(q) : AX.row(q), 0), n - 1);
                     cx[2 * t] = ax ? L.c2[1][g] : L.c2[0][g];
                     cx[2 * t + 1] = ax ? L.c1[1][g] : L.c1[0][g];
                 }
