@@ -1,5 +1,6 @@
-// mg_plan.hpp -- the tiles of k_tile (mg_tile.hpp): how large they are, which
-// rows of a level each of them touches, and the plan of a V-cycle's visit.
+// mg_plan.hpp -- how a level's work is cut: the tiles of k_tile (mg_tile.hpp), the
+// rows of a level each of them touches and the plan of a V-cycle's visit; the
+// form of a colour pass (k_rb_split, mg_split.hpp) and its vectors.
 // Plain arithmetic shared by the host code, the kernel and the CPU tests.
 #pragma once
 #include <algorithm>
@@ -95,6 +96,36 @@ inline TilePlan plan_tile(size_t word, int dim, const int (&n)[3], bool split, i
                 }
             }
     return best;
+}
+
+// One colour pass of a split level (see k_rb_split): rows a lane takes, byte
+// offsets and vector numbers beyond 32 and 31 bits, and the number of vectors.
+struct PassPlan {
+    int rows = 1;
+    bool off64 = false, div64 = false, ok = false;
+    unsigned total = 0;
+};
+
+// Pairs of rows along y (x in a planar level) where the rows pair up and the
+// walls are homogeneous; the general form (one row a lane, any SOR parameter,
+// 64-bit offsets) elsewhere, and for other parameters than 1 in arrays of 4 GB
+// and more, which no deck has.  A launch numbers its lanes with 32 bits (ok);
+// numbers of 2^31 and more, which the division by multiplication does not take,
+// are divided as they are (div64): general-form levels of 69 GB an array reach
+// them, pairs those of twice that.
+// dirv: stored wall values; w1: SOR parameter 1; general, wide: forced forms.
+inline PassPlan plan_pass(size_t word, int dim, const int (&n)[3], size_t elems, int rtile, bool dirv, bool w1,
+                          bool general, bool wide) {
+    PassPlan P;
+    P.off64 = elems * word > 0xffffffffull || wide;
+    const bool one = ((dim == 3 ? n[1] : n[0]) & 1) || dirv || general || (P.off64 && !w1);
+    P.rows = one ? 1 : 2;
+    const size_t total = (size_t)n[0] * n[1] / P.rows * (n[2] / 2 / (16 / word));
+    // (a launch rounds up to whole blocks on every XCD)
+    P.ok = total + 4096 <= 0xffffffffull && !(rtile && rtile % P.rows);
+    P.total = P.ok ? (unsigned)total : 0;
+    P.div64 = total > 0x7fffffffull || wide;
+    return P;
 }
 
 }  // namespace saras

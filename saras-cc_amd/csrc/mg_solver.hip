@@ -268,6 +268,7 @@ struct saras_mg {
     bool red_fold = true;              // SARAS_NO_RED_FOLD=1: the restriction leaves the first red pass to the sweep
     bool coarse_one = false;           // SARAS_COARSE_ONE=1 smooths every coarsest level in one workgroup
     bool rb_general = false;           // SARAS_RB_GENERAL=1 runs every split colour pass in the general form
+    bool rb_wide = false;              // SARAS_RB_WIDE=1 runs every split colour pass and restriction as in arrays of 4 GB and more
     bool tile_off = false;             // SARAS_NO_TILE=1 runs every pass as a launch of its own
     bool rr_lane = false;              // SARAS_RR_LANE=1: 3-D split restriction with all eight children in one lane
     // V-cycles replayed from captured hipGraphs (saras_mg_set_graphs).  A
@@ -589,11 +590,9 @@ struct Ops {
         return L.n[1] % 16 == 0 && L.n[2] % 64 == 0 && (long)L.n[0] * L.n[1] * L.n[2] >= (8L << 20);
     }
 
-    // One colour pass of a split level.  The paired form (k_rb_split with R = 2)
-    // takes levels whose rows pair up along y (x in a planar level) and whose
-    // walls are homogeneous -- every level but a DIRICHLET_TEST level 0 (the
-    // levels above the coarsest have even row counts), with 64-bit offsets for
-    // arrays of 4 GB and more; the general form the rest.
+    // One colour pass of a split level, in the form that plan_pass chooses (the
+    // levels above the coarsest have even row counts, so all but a
+    // DIRICHLET_TEST level 0 go by row pairs).
     // Time of a pass, one row per lane with branches around each load / now:
     // FP32 256^3 19.6 / 16.8 us (after the prolongation: red 33 / 20, black
     // 20 / 16.4), 512^3 180 / 150 us (279 / 197, 183 / 147), tanh z 256^3 20.1 /
@@ -603,29 +602,26 @@ struct Ops {
     void rb_pass(int l, const saras::LevelArgs<T> &a, int colour, const T *e, long esx, long esy, long ehz) {
         using namespace saras;
         DevLevel<T> &L = H.lv[l];
-        const int np = DIM == 3 ? L.n[1] : L.n[0];
         const bool dirv = a.bc_lo[0] == BC_DIRV || a.bc_lo[2] == BC_DIRV;
-        const bool big = L.elems * sizeof(T) > 0xffffffffull;
-        const bool gen = (np & 1) || dirv || m->rb_general || (big && w != T(1));
-        const int R = gen ? 1 : 2;
-        RowMap M;
-        const unsigned q = (unsigned)(L.n[2] / 2 / Vec16<T>::W);
-        const unsigned wj = DIM == 3 ? (unsigned)((a.rtile ? a.rtile : L.n[1]) / R) : 1u;
-        M.q = FastDiv::of(q);
-        M.tile = FastDiv::of((unsigned)L.n[0] * wj);
-        M.wj = FastDiv::of(wj);
-        const size_t total = (size_t)L.n[0] * L.n[1] / R * q;
-        // host-side guard: vector numbers stay below 2^31
-        if (total + kSplitThreads * kXcds > 0x7fffffffull || (a.rtile && a.rtile % R)) {
+        const PassPlan P = plan_pass(sizeof(T), DIM, L.n, L.elems, a.rtile, dirv, w == T(1), m->rb_general, m->rb_wide);
+        // host-side guard: a launch's vector numbers
+        if (!P.ok) {
             refuse("a level too large for one pass");
             return;
         }
-        M.total = (unsigned)total;
-        const unsigned nb = (unsigned)((total + kSplitThreads - 1) / kSplitThreads);
+        RowMap M;
+        const unsigned q = (unsigned)(L.n[2] / 2 / Vec16<T>::W);
+        const unsigned wj = DIM == 3 ? (unsigned)((a.rtile ? a.rtile : L.n[1]) / P.rows) : 1u;
+        M.q = FastDiv::of(q);
+        M.tile = FastDiv::of((unsigned)L.n[0] * wj);
+        M.wj = FastDiv::of(wj);
+        M.total = P.total;
+        M.div64 = P.div64;
+        const unsigned nb = (unsigned)(((size_t)P.total + kSplitThreads - 1) / kSplitThreads);
         const dim3 g((nb + kXcds - 1) / kXcds * kXcds), bl(kSplitThreads);
-        if (gen)
+        if (P.rows == 1)
             hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, RB_GENERAL>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
-        else if (big)
+        else if (P.off64)
             hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, true, false, RB_PAIR64>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
         else if (w != T(1))
             hipLaunchKernelGGL((k_rb_split<T, DIM, MODE, false, false, RB_PAIR>), g, bl, 0, s, a, M, L.x, L.b, colour, w, e, esx, esy, ehz);
@@ -776,7 +772,7 @@ struct Ops {
         const bool dirv = fa.bc_lo[0] == BC_DIRV || fa.bc_lo[2] == BC_DIRV;
         if (dirv || m->rb_general)
             hipLaunchKernelGGL((k_rr_pair<T, RED, false, RB_GENERAL>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
-        else if (F.elems * sizeof(T) > 0xffffffffull)
+        else if (F.elems * sizeof(T) > 0xffffffffull || m->rb_wide)
             hipLaunchKernelGGL((k_rr_pair<T, RED, false, RB_PAIR64>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
         else if (F.uniform)
             hipLaunchKernelGGL((k_rr_pair<T, RED, true, RB_PAIR>), g, bl, 0, s, fa, F.x, F.b, ca, C.b, C.x, r, M, w);
@@ -1352,6 +1348,8 @@ saras_status saras_mg_create(const saras_grid_desc *grid, const saras_mg_params 
         m->split_off = env5 && env5[0] == '1';
         const char *env11 = std::getenv("SARAS_RB_GENERAL");
         m->rb_general = env11 && env11[0] == '1';
+        const char *env13 = std::getenv("SARAS_RB_WIDE");
+        m->rb_wide = env13 && env13[0] == '1';
         const char *env12 = std::getenv("SARAS_COARSE_ONE");
         m->coarse_one = env12 && env12[0] == '1';
         const char *env10 = std::getenv("SARAS_NO_TILE");

@@ -142,6 +142,7 @@ struct FastDiv {
 struct RowMap {
     FastDiv q, tile, wj;   // vectors of a half-row; groups of a tile; groups of a tile's i-row
     unsigned total;        // vectors of the level
+    bool div64 = false;    // their numbers take no FastDiv (2^31 and more; not in RB_PAIR, see plan_pass)
 };
 
 // What the iterate is when a colour pass reads it.
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(kSplitThreads) k_rb_split(LevelArgs<T> L, RowM
     const unsigned t = logical * kSplitThreads + threadIdx.x;
     if (t >= M.total) return;
     const int nx = L.n[0], ny = L.n[1], half = L.n[2] >> 1;
-    const unsigned g = M.q.div(t);
+    const unsigned g = FORM != RB_PAIR && M.div64 ? t / M.q.d : M.q.div(t);
     const int m0 = (int)(t - g * M.q.d) * W;
     int i, j;
     if (DIM == 3) {
