@@ -26,6 +26,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
+#include "nse_round.hpp"
+
 namespace saras {
 namespace nse {
 
@@ -477,14 +481,6 @@ __device__ __forceinline__ double d2_of(const Geom &G, int ax, int q, double xx,
     o = o * G.ih2[ax];
     return xx * t + x2 * o;
 }
-// a / 6, the correctly rounded quotient, in four instructions: a product with
-// the rounded reciprocal, corrected by its exact remainder (v_div_fixup gives
-// infinities and NaN their quotients).  Of 6e8 values compared with the
-// division none differs; only subnormal quotients may, by one unit.
-__device__ __forceinline__ double by6(double a) {
-    const double y = 1.0 / 6.0, q = a * y;
-    return __builtin_amdgcn_div_fixup(fma(fma(-6.0, q, a), y, q), 6.0, a);
-}
 // Morinishi's pair of mor_pair from the values around q
 __device__ __forceinline__ double mor_of(const Geom &G, int a, int q, double xm, double u, double cm2, double cm, double cp,
                                          double cp2, double um2, double um, double up, double up2) {
@@ -830,33 +826,16 @@ __device__ __forceinline__ double sf_integral(double d) {   // spiral.cc:620-631
     return 12.2946 * (c * c) - 6.0 - 0.573159 / (d * sqrt(d)) * sin(3.14159 * d - 0.785398);
 }
 
-// Correctly rounded single-precision root and quotients, the values of sqrtf and
-// of the division, without the scaling of arguments near the ends of the range
-// (11 and 3 or 9 issue slots instead of 17 and 11).  Compared with them on the
-// device: the root at every significand at 120 exponents, 0.573159 / b at every
-// significand at 52, 1e9 pairs of quot_rn; none differs.
-__device__ __forceinline__ float sqrt_rn(float a) {
-    const float y = __builtin_amdgcn_rsqf(a);
-    float g = a * y, h = 0.5f * y;
-    const float e = fmaf(-h, g, 0.5f);
-    g = fmaf(g, e, g);
-    h = fmaf(h, e, h);
-    return a < 0x1p-100f ? 0.0f : fmaf(fmaf(-g, g, a), h, g);
-}
-// a / b from the rounded reciprocal y of b
-__device__ __forceinline__ float quot_rn(float a, float b, float y) {
-    const float q = a * y;
-    return fmaf(fmaf(-b, q, a), y, q);
-}
-
-// sf_integral in single precision (the same expression)
+// sf_integral in single precision (the same expression); SHORT: with the root and
+// the quotient of nse_round.hpp, for d of at most 2^72
+template <bool SHORT>
 __device__ __forceinline__ float sf_integral_f(float d) {
     const float d2 = d * d;
     const float near = 7.4022f * d2 - 1.82642f * d2 * d2;
     if (d < 0.873469f) return near;
-    const float c = cbrtf(d), b = d * sqrt_rn(d), y = __builtin_amdgcn_rcpf(b);
-    return 12.2946f * (c * c) - 6.0f -
-           quot_rn(0.573159f, b, fmaf(fmaf(-b, y, 1.0f), y, y)) * sinf(3.14159f * d - 0.785398f);
+    const float c = cbrtf(d), b = d * (SHORT ? sqrt_rn(d) : sqrtf(d));
+    const float q = SHORT ? quot_rn(0.573159f, b) : 0.573159f / b;
+    return 12.2946f * (c * c) - 6.0f - q * sinf(3.14159f * d - 0.785398f);
 }
 
 // spiral::sgsStress (spiral.cc:472-548 with eigenvalueSymm :643-~690 and
@@ -988,6 +967,11 @@ k_sgs_stress(Geom G, double nu, SgsMarch A) {
     const double dzp = G.xc[2][kk + 1] - G.xc[2][kk], dzm = G.xc[2][kk - 1] - G.xc[2][kk];
     auto close = [](double a, double b) { return fabs(a + b) <= 1e-12 * fabs(a); };
     const bool mirror_yz = close(dyp, dym) && close(dzp, dzm);
+    // The short single-precision forms hold for cell widths of 2^-35 to 2^35: the
+    // difference of two squares of 2^-70 and more is zero or at least 2^-95, and
+    // distances are at most 2^72 times the mean width.
+    auto brief = [](double a) { return fabs(a) >= 0x1p-35 && fabs(a) <= 0x1p35; };
+    const bool brief_yz = brief(dyp) && brief(dym) && brief(dzp) && brief(dzm);
     // first derivative along ax at index q from the four values around it
     auto der = [&](int ax, int q, double m, double fm2, double fm, double fp, double fp2) __attribute__((always_inline)) {
         double v = (8.0 * (fp - fm) - (fp2 - fm2)) * kRecip12;
@@ -1057,21 +1041,28 @@ k_sgs_stress(Geom G, double nu, SgsMarch A) {
                 const float sx[3] = {(float)dxm, 0.0f, (float)dxp}, sy[3] = {(float)dym, 0.0f, (float)dyp};
                 const float sz[3] = {(float)dzm, 0.0f, (float)dzp}, fe[3] = {(float)e[0], (float)e[1], (float)e[2]};
                 const float fdel = (float)del, idel = 1.0f / fdel;
-                auto term = [&](float dx, float dy, float dz) __attribute__((always_inline)) {
+                auto term = [&](float dx, float dy, float dz, auto shortc) __attribute__((always_inline)) {
+                    constexpr bool SHORT = decltype(shortc)::value;
                     const float dx2 = dx * dx + dy * dy + dz * dz, dxe = dx * fe[0] + dy * fe[1] + dz * fe[2];
-                    return (double)sf_integral_f(quot_rn(sqrt_rn(dx2 - dxe * dxe), fdel, idel));
+                    const float r = dx2 - dxe * dxe;
+                    const float d = SHORT ? quot_rn(sqrt_rn(r), fdel, idel) : sqrtf(fmaxf(r, 0.0f)) / fdel;
+                    return (double)sf_integral_f<SHORT>(d);
                 };
-                if (mirror) {
+                const bool shorts = brief_yz && brief(dxp) && brief(dxm);
+                if (mirror && shorts) {
                     // the 13 offsets before (0, 0, 0) in (di, dj, dk) order
 #pragma unroll
-                    for (int t = 0; t < 13; ++t) Qd += 2.0 * term(sx[t / 9], sy[(t / 3) % 3], sz[t % 3]);
+                    for (int t = 0; t < 13; ++t) Qd += 2.0 * term(sx[t / 9], sy[(t / 3) % 3], sz[t % 3], std::true_type{});
                 } else {
+                    const int nt = mirror ? 13 : 27;
 #pragma unroll 1
-                    for (int t = 0; t < 27; ++t) {
+                    for (int t = 0; t < nt; ++t) {
                         const int a = t / 9, b = (t / 3) % 3, c = t % 3;
-                        if (t != 13)
-                            Qd += term(a == 0 ? sx[0] : a == 1 ? 0.0f : sx[2], b == 0 ? sy[0] : b == 1 ? 0.0f : sy[2],
-                                       c == 0 ? sz[0] : c == 1 ? 0.0f : sz[2]);
+                        if (t == 13) continue;
+                        const float dx = a == 0 ? sx[0] : a == 1 ? 0.0f : sx[2], dy = b == 0 ? sy[0] : b == 1 ? 0.0f : sy[2];
+                        const float dz = c == 0 ? sz[0] : c == 1 ? 0.0f : sz[2];
+                        const double v = shorts ? term(dx, dy, dz, std::true_type{}) : term(dx, dy, dz, std::false_type{});
+                        Qd += mirror ? 2.0 * v : v;
                     }
                 }
             } else {
