@@ -1,6 +1,7 @@
 // mg_plan.hpp -- how a level's work is cut: the tiles of k_tile (mg_tile.hpp), the
 // rows of a level each of them touches and the plan of a V-cycle's visit; the
-// form of a colour pass (k_rb_split, mg_split.hpp) and its vectors.
+// form of a colour pass (k_rb_split, mg_split.hpp) and its vectors; the LDS of
+// the tail (k_tail, mg_tail.hpp).
 // Plain arithmetic shared by the host code, the kernel and the CPU tests.
 #pragma once
 #include <algorithm>
@@ -96,6 +97,105 @@ inline TilePlan plan_tile(size_t word, int dim, const int (&n)[3], bool split, i
                 }
             }
     return best;
+}
+
+constexpr int kTailMaxLevels = 8;
+constexpr int kTailThreads = 512;
+// cells of one colour that a thread of the tail keeps in registers
+constexpr int kTailColourCells = 4;
+// LDS that the tail takes by default, of the 160 KB a workgroup may hold (its
+// static LDS is under 1 KB).  Taking 156 KB lets in 2-D levels of 4096 cells in
+// long boxes, which are faster by tiles (1024 x 64 FP64, four V(2,2) cycles: 1.01
+// against 1.09 ms).
+constexpr size_t kTailLds = 150 * 1024;
+
+// The LDS of the tail (k_tail) for levels S..D, offsets in elements (the
+// tables' in 32-bit words).
+struct TailPlan {
+    size_t bytes = 0;          // 0: the tail does not take these levels
+    bool b_global = false;     // the right-hand side of the single level stays in global memory
+    struct Level {
+        int n[3];
+        int hz, half;          // cells of one colour per row (rounded up) and per level
+        bool odd;              // an odd periodic extent
+        int x, b, old;         // iterate, right-hand side, old values
+        int cell4, cell1;      // tables (see TailLevel); cell1 -1: not in LDS
+    } L[kTailMaxLevels];
+    int res = 0, coff = 0, ncoef = 0, cellw = 0, ncellw = 0;
+};
+
+// n: extents of the levels S..D (`count` of them, 1 along y in 2-D); periodic:
+// per axis; solve: the coarsest level is solved; limit: bytes of LDS.
+//
+// A solved coarsest level holds three arrays, the third the old values that its
+// stopping residual reads; one that fits only without its right-hand side keeps
+// that in global memory, from where each thread reads it into registers once a
+// solve, and in each pass for the cells beyond those.  Four cycles with the
+// coarsest level solved by k_coarse in global memory / here: FP64 82 x 86, 2256
+// iterations a solve at most, 62 / 23 ms; 18 x 18 x 22, 119 iterations, 5.8 / 2.5 ms;
+// 19 x 18 x 19, 125 iterations, 5.7 / 2.4 ms; FP32 115 x 123 189 / 151 ms, 24 x 23 x 25
+// 56 / 28 ms.
+inline TailPlan plan_tail(size_t word, int dim, const int (*n)[3], int count, const int (&periodic)[3], bool solve,
+                          size_t limit) {
+    TailPlan P;
+    if (count < 1 || count > kTailMaxLevels) return P;
+    const size_t reg = (size_t)kTailColourCells * kTailThreads;
+    auto up4 = [](size_t v) { return (v + 3) / 4 * 4; };
+    auto place = [&](bool b_global) -> size_t {
+        size_t off = 0, ncoef = 0, ncell = 0;
+        for (int l = 0; l < count; ++l) {
+            TailPlan::Level &V = P.L[l];
+            const bool last = l == count - 1;
+            for (int a = 0; a < 3; ++a) V.n[a] = n[l][a];
+            const int ny = dim == 3 ? n[l][1] : 1;
+            V.hz = (n[l][2] + 1) / 2;
+            const size_t half = (size_t)n[l][0] * ny * V.hz;
+            if (2 * half > 65535) return 0;   // a cell's LDS offset takes 16 bits
+            V.half = (int)half;
+            V.odd = false;
+            for (int a = 0; a < 3; ++a)
+                if (dim == 3 || a != 1) V.odd = V.odd || (periodic[a] && (n[l][a] & 1));
+            // levels above the coarsest: the cells that the threads keep in
+            // registers; larger ones run faster as multi-workgroup passes
+            if (!last && (half > reg || V.odd)) return 0;
+            V.x = (int)off;
+            off += up4(2 * half);
+            V.b = b_global ? -1 : (int)off;
+            if (!b_global) off += up4(2 * half);
+            V.old = (int)off;
+            if (last && (solve || (V.odd && half > reg))) off += up4(2 * half);
+            ncoef += 2 * ((size_t)n[l][0] + ny + n[l][2]);
+            if (dim == 3 && l > 0) ncoef += 3 * ((size_t)n[l][0] + ny + n[l][2]);
+            // cell tables of levels with at most one cell of a colour per thread
+            V.cell1 = half <= (size_t)kTailThreads ? 0 : -1;
+            V.cell4 = 0;
+            if (V.cell1 >= 0) ncell += 2 * up4(2 * half) * 5 / 2;
+        }
+        P.res = (int)off;
+        if (count > 1) off += up4(2 * (size_t)P.L[0].half);
+        P.coff = (int)off;
+        P.ncoef = (int)ncoef;
+        off += up4(ncoef);
+        const size_t words = word / 4;
+        size_t w = off * words;
+        P.cellw = (int)w;
+        P.ncellw = (int)ncell;
+        for (int l = 0; l < count; ++l) {
+            TailPlan::Level &V = P.L[l];
+            if (V.cell1 < 0) continue;
+            const size_t cells = up4(2 * (size_t)V.half);
+            V.cell4 = (int)w;
+            V.cell1 = (int)(w + 4 * cells);
+            w += 5 * cells;
+        }
+        return w * 4 <= limit && w / words < 65536 ? w * 4 : 0;
+    };
+    P.bytes = place(false);
+    if (!P.bytes && count == 1 && solve) {
+        P.b_global = true;
+        P.bytes = place(true);
+    }
+    return P;
 }
 
 // One colour pass of a split level (see k_rb_split): rows a lane takes, byte

@@ -46,12 +46,6 @@ void set_error(const std::string &s) { g_last_error = s; }
     } while (0)
 
 constexpr int kThreads = 256;
-// default dynamic LDS budget of the single-workgroup tail, of the 160 KB a
-// workgroup may hold (SARAS_TAIL_LDS_KB lowers it; the tail's static LDS is
-// under 1 KB); above the coarsest level the tail also takes only levels whose
-// cells its threads keep in registers (see tail_layout)
-constexpr size_t kTailLdsDefault = 150 * 1024;
-
 inline unsigned blocks_for(long n) { return (unsigned)std::max<long>(1, (n + kThreads - 1) / kThreads); }
 
 template <typename T>
@@ -105,6 +99,7 @@ struct Hierarchy {
     size_t tail_bytes = 0;
     T *tail_coef = nullptr;
     unsigned *tail_cells = nullptr;
+    T *tail_b = nullptr;   // see TailArgs::bcol
 
     // a level takes split rows when each half-row is a whole number of 16-byte vectors
     static bool splittable(int nz) {
@@ -125,6 +120,7 @@ struct Hierarchy {
         (void)hipFree(coarse_scratch);
         (void)hipFree(tail_coef);
         (void)hipFree(tail_cells);
+        (void)hipFree(tail_b);
     }
 
     saras_status build(const saras::GridLevels &G, const std::vector<std::vector<double>> &walls) {
@@ -264,7 +260,7 @@ struct saras_mg {
     int march_wgs = 0;                 // target workgroups of a march sweep (SARAS_MARCH_WGS; 0 = per type)
     bool march_tj8 = false;            // FP32 march with 64 x 8 tiles (SARAS_MARCH_TJ8=1)
     bool split_off = false;            // SARAS_NO_SPLIT=1 keeps every level z-contiguous
-    size_t tail_lds = kTailLdsDefault;  // dynamic LDS budget of the tail kernel
+    size_t tail_lds = saras::kTailLds;  // dynamic LDS budget of the tail kernel (SARAS_TAIL_LDS_KB lowers it)
     bool red_fold = true;              // SARAS_NO_RED_FOLD=1: the restriction leaves the first red pass to the sweep
     bool coarse_one = false;           // SARAS_COARSE_ONE=1 smooths every coarsest level in one workgroup
     bool rb_general = false;           // SARAS_RB_GENERAL=1 runs every split colour pass in the general form
@@ -337,64 +333,42 @@ template <typename T>
 size_t tail_layout(const saras_mg *m, const Hierarchy<T> &H, int S, saras::TailArgs<T> &A) {
     const int D = (int)H.lv.size() - 1;
     if (D - S + 1 > saras::kTailMaxLevels) return 0;
-    auto up4 = [](size_t n) { return (n + 3) / 4 * 4; };
+    // inhomogeneous walls (the finest level of the reference's test problem) are
+    // left to the multi-workgroup kernels
+    if (S == 0 && m->p.bc == SARAS_BC_DIRICHLET_TEST) return 0;
+    int n[saras::kTailMaxLevels][3];
+    for (int l = S; l <= D; ++l)
+        for (int a = 0; a < 3; ++a) n[l - S][a] = H.lv[l].n[a];
+    const int per[3] = {m->g.periodic[0] != 0, m->g.periodic[1] != 0, m->g.periodic[2] != 0};
+    const saras::TailPlan P = saras::plan_tail(sizeof(T), H.dim, n, D - S + 1, per, m->p.solve_flag != 0, m->tail_lds);
+    if (!P.bytes) return 0;
     A = saras::TailArgs<T>{};
     A.first = S;
     A.last = D;
-    size_t off = 0, ncoef = 0, ncell = 0;
+    A.res = P.res;
+    A.coff = P.coff;
+    A.ncoef = P.ncoef;
+    A.cellw = P.cellw;
+    A.ncellw = P.ncellw;
     for (int l = S; l <= D; ++l) {
-        const DevLevel<T> &L = H.lv[l];
+        const saras::TailPlan::Level &Q = P.L[l - S];
         saras::TailLevel &V = A.L[l - S];
-        for (int a = 0; a < 3; ++a) V.n[a] = L.n[a];
-        const int ny = H.dim == 3 ? L.n[1] : 1;
-        V.hz = (L.n[2] + 1) / 2;
-        const size_t half = (size_t)L.n[0] * ny * V.hz;
-        if (2 * half > 65535) return 0;   // a cell's LDS offset takes 16 bits
-        V.half = (int)half;
+        for (int a = 0; a < 3; ++a) V.n[a] = Q.n[a];
+        V.hz = Q.hz;
+        V.half = Q.half;
+        V.x = Q.x;
+        V.b = Q.b;
+        V.old = Q.old;
+        V.cell4 = Q.cell4;
+        V.cell1 = Q.cell1;
+        V.odd = Q.odd;
         for (int a = 0; a < 3; ++a) {
             if (H.dim == 2 && a == 1) continue;
-            const int lo = bc_code(m->p, m->g, a, l, false, false), hi = bc_code(m->p, m->g, a, l, false, true);
-            V.neg |= lo == saras::BC_DIR || hi == saras::BC_DIR;
-            V.odd |= lo == saras::BC_PER && (L.n[a] & 1);
+            V.neg |= bc_code(m->p, m->g, a, l, false, false) == saras::BC_DIR ||
+                     bc_code(m->p, m->g, a, l, false, true) == saras::BC_DIR;
         }
-        const size_t reg = (size_t)saras::kTailColourCells * saras::kTailThreads;
-        // levels above the coarsest: the cells that the threads keep in
-        // registers; larger ones run faster as multi-workgroup passes
-        if (l < D && (half > reg || V.odd)) return 0;
-        // inhomogeneous walls (the finest level of the reference's test
-        // problem) are left to the multi-workgroup kernels
-        if (l == 0 && m->p.bc == SARAS_BC_DIRICHLET_TEST) return 0;
-        V.x = (int)off;
-        off += up4(2 * half);
-        V.b = (int)off;
-        off += up4(2 * half);
-        V.old = (int)off;
-        if (l == D && (m->p.solve_flag || (V.odd && half > reg))) off += up4(2 * half);
-        ncoef += 2 * ((size_t)L.n[0] + ny + L.n[2]);
-        if (H.dim == 3 && l > S) ncoef += 3 * ((size_t)L.n[0] + ny + L.n[2]);
-        // cell tables of levels with at most one cell of a colour per thread
-        V.cell1 = half <= (size_t)saras::kTailThreads ? 0 : -1;
-        if (V.cell1 >= 0) ncell += 2 * up4(2 * half) * 5 / 2;
     }
-    A.res = (int)off;
-    if (S < D) off += up4(2 * (size_t)A.L[0].half);
-    A.coff = (int)off;
-    A.ncoef = (int)ncoef;
-    off += up4(ncoef);
-    const size_t words = sizeof(T) / 4;
-    size_t w = off * words;
-    A.cellw = (int)w;
-    A.ncellw = (int)ncell;
-    for (int l = S; l <= D; ++l) {
-        saras::TailLevel &V = A.L[l - S];
-        if (V.cell1 < 0) continue;
-        const size_t n = up4(2 * (size_t)V.half);
-        V.cell4 = (int)w;
-        V.cell1 = (int)(w + 4 * n);
-        w += 5 * n;
-    }
-    const size_t bytes = w * 4;
-    return bytes <= m->tail_lds && w / words < 65536 ? bytes : 0;
+    return P.bytes;
 }
 
 // The plan of one visit of level l by tiles (none: by separate passes).
@@ -506,6 +480,10 @@ saras_status pack_tail(const saras_mg *m, Hierarchy<T> &H) {
     }
     HIP_TRY(hipMalloc((void **)&H.tail_cells, std::max<size_t>(4, img.size()) * sizeof(unsigned)));
     HIP_TRY(hipMemcpy(H.tail_cells, img.data(), img.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+    if (A.L[0].b < 0) {
+        HIP_TRY(hipMalloc((void **)&H.tail_b, 2 * (size_t)A.L[0].half * sizeof(T)));
+        A.bcol = H.tail_b;
+    }
     A.coef = H.tail_coef;
     A.cellimg = H.tail_cells;
     A.cells4 = reinterpret_cast<const uint4 *>(H.tail_cells + nimg);
@@ -946,7 +924,7 @@ struct Ops {
     void tail(int S) {
         const int D = (int)H.lv.size() - 1;
         // host-side guard: the tail packed for this hierarchy
-        if (S != H.tail_first || S > D || H.tail_bytes > m->tail_lds) {
+        if (S != H.tail_first || S > D || H.tail_bytes > m->tail_lds || (H.tail_args.bcol && S != D)) {
             refuse("tail levels not packed");
             return;
         }
@@ -964,10 +942,14 @@ struct Ops {
         A.tol = m->p.mg_tol;
         A.rel_floor = coarse_rel_floor();
         A.iters_out = m->iters_host;
-        if (H.dim == 3)
-            hipLaunchKernelGGL((saras::k_tail<T, 3>), dim3(1), dim3(saras::kTailThreads), H.tail_bytes, s, A);
-        else
-            hipLaunchKernelGGL((saras::k_tail<T, 2>), dim3(1), dim3(saras::kTailThreads), H.tail_bytes, s, A);
+        if (H.dim == 3) tail_launch<3>(A);
+        else tail_launch<2>(A);
+    }
+    template <int DIM>
+    void tail_launch(const saras::TailArgs<T> &A) {
+        const dim3 g(1), bl(saras::kTailThreads);
+        if (A.bcol) hipLaunchKernelGGL((saras::k_tail<T, DIM, true>), g, bl, H.tail_bytes, s, A);
+        else hipLaunchKernelGGL((saras::k_tail<T, DIM, false>), g, bl, H.tail_bytes, s, A);
     }
 
     // poisson::vCycle (poisson.cc:203-279); levels S..D run in the tail kernel
@@ -1359,7 +1341,7 @@ saras_status saras_mg_create(const saras_grid_desc *grid, const saras_mg_params 
         const char *env8 = std::getenv("SARAS_NO_RED_FOLD");
         m->red_fold = !(env8 && env8[0] == '1');
         const char *env6 = std::getenv("SARAS_TAIL_LDS_KB");
-        if (env6 && std::atoi(env6) > 0) m->tail_lds = (size_t)std::min(150, std::atoi(env6)) * 1024;
+        if (env6 && std::atoi(env6) > 0) m->tail_lds = std::min(saras::kTailLds, (size_t)std::atoi(env6) * 1024);
     }
     if (m->p.inner_cycles <= 0) m->p.inner_cycles = 3;
     if (m->p.max_refine <= 0) m->p.max_refine = 20;

@@ -32,13 +32,9 @@
 #include <type_traits>
 
 #include "mg_kernels.hpp"
+#include "mg_plan.hpp"
 
 namespace saras {
-
-constexpr int kTailMaxLevels = 8;
-constexpr int kTailThreads = 512;
-// cells of one colour a thread keeps in registers
-constexpr int kTailColourCells = 4;
 
 // One cell of a level stored by colour.  Directions: x+, x-, y+, y-, z+, z-.
 struct TailCell {
@@ -55,7 +51,7 @@ constexpr unsigned kTailNoCell = 1u << 15;
 struct TailLevel {
     int n[3];
     int hz, half;              // cells of one colour per row (rounded up) and per level
-    int x, b, old;             // iterate, right-hand side, old values of a coarsest solve
+    int x, b, old;             // iterate, right-hand side (-1: at TailArgs::bcol), old values of a coarsest solve
     int lo[3], hi[3], wd[3];   // restriction factors of this (coarse) level, 3-D
     int neg;                   // some wall is Dirichlet
     int odd;                   // an odd periodic extent (the coarsest level alone can have one)
@@ -77,6 +73,7 @@ struct TailArgs {
     const unsigned *cells1;
     T *x;                                // global core array of level S (in/out)
     const T *b;                          // global core array of level S
+    T *bcol;                             // the right-hand side of a level without room for it in LDS, by colour
     int pre, post, solve_flag, max_count;
     T w;
     double tol;
@@ -227,7 +224,9 @@ __device__ __forceinline__ Stencil<T, DIM> tail_gather(const T *lds, const TailC
 // larger level beyond them (a coarsest one: the others are limited to
 // kTailColourCells) are loaded anew in each pass (and with an odd periodic
 // extent wait at V.old for the others' reads).
-template <typename T, int DIM, int CPT>
+//
+// BG: the right-hand side of the level (a coarsest one by itself) is at A.bcol.
+template <typename T, int DIM, int CPT, bool BG>
 __device__ __forceinline__ int tail_smooth(T *lds, const TailArgs<T> &A, const TailLevel &V, const TailLevel &C,
                                            bool pro, bool solve, int count, bool emit, double *red, int *wflag) {
     // FP64 with several cells per thread: the coefficients do not fit beside them
@@ -270,7 +269,7 @@ __device__ __forceinline__ int tail_smooth(T *lds, const TailArgs<T> &A, const T
     // (the addresses are valid all the same, so a caller may go on with it)
     auto load = [&](int q, Own &o) __attribute__((always_inline)) {
         o.t = cell(q);
-        o.b = lds[V.b + q];
+        o.b = BG ? A.bcol[q] : lds[V.b + q];
         o.x = lds[V.x + q];
         const TailCoef<T> m = tail_coefs<T, DIM>(lds, o.t);
         if constexpr (KEEP) o.m = m;
@@ -422,7 +421,10 @@ __device__ __forceinline__ int tail_smooth(T *lds, const TailArgs<T> &A, const T
     return iter;
 }
 
-template <typename T, int DIM>
+// BG: the coarsest level alone, its right-hand side in global memory (see
+// plan_tail; a kernel of its own, since a pointer to either memory would make
+// each access a flat one)
+template <typename T, int DIM, bool BG>
 __global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A) {
     extern __shared__ __align__(16) unsigned char tail_raw[];
     T *lds = reinterpret_cast<T *>(tail_raw);
@@ -447,7 +449,8 @@ __global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A) {
             const long g = (long)i * A.sx + (long)j * A.sy + (A.hz ? (long)(k & 1) * A.hz + (k >> 1) : (long)k);
             const int at = tail_at<DIM>(V, i, j, k);
             lds[V.x + at] = A.x[g];
-            lds[V.b + at] = A.b[g];
+            if constexpr (BG) A.bcol[at] = A.b[g];
+            else lds[V.b + at] = A.b[g];
         }
         __syncthreads();
     }
@@ -471,10 +474,10 @@ __global__ void __launch_bounds__(kTailThreads) k_tail(TailArgs<T> A) {
         const int count = up ? A.post : A.pre;
         const TailLevel &V = A.L[l - S], &C = A.L[l < D ? l + 1 - S : l - S];
         int it;
-        if (V.cell1 >= 0) it = tail_smooth<T, DIM, 1>(lds, A, V, C, up, solve, count, emit, red, wflag);
-        else it = tail_smooth<T, DIM, kTailColourCells>(lds, A, V, C, up, solve, count, emit, red, wflag);
+        if (!BG && V.cell1 >= 0) it = tail_smooth<T, DIM, 1, false>(lds, A, V, C, up, solve, count, emit, red, wflag);
+        else it = tail_smooth<T, DIM, kTailColourCells, BG>(lds, A, V, C, up, solve, count, emit, red, wflag);
         if (solve) iters = it;
-        if (!emit) continue;
+        if (BG || !emit) continue;
         // computeResidual + coarsen (poisson_d3.cc:71-93, 484-511; poisson_d2.cc:288-297)
         const int ctotal = C.n[0] * C.n[1] * C.n[2];
         const T *R = lds + A.res;
