@@ -72,18 +72,33 @@ struct DevLevel {
     T *rlo[3] = {nullptr, nullptr, nullptr}, *rhi[3] = {nullptr, nullptr, nullptr}, *rwd[3] = {nullptr, nullptr, nullptr};
 };
 
+// The small constant arrays of a hierarchy, gathered on the host and sent in one
+// allocation and one transfer (each pair of them takes about 10 us; a 32^3 mixed
+// handle has some 170 arrays: making one took 1.8 ms with a pair for each).
 template <typename T>
-saras_status upload(T **dst, const std::vector<double> &src) {
-    std::vector<T> tmp(src.begin(), src.end());
-    HIP_TRY(hipMalloc((void **)dst, std::max<size_t>(1, tmp.size()) * sizeof(T)));
-    HIP_TRY(hipMemcpy(*dst, tmp.data(), tmp.size() * sizeof(T), hipMemcpyHostToDevice));
-    return SARAS_OK;
-}
+struct ConstImage {
+    std::vector<T> data;
+    std::vector<std::pair<T **, size_t>> at;   // array pointers to set and their places
+    // every array starts at a multiple of 256 bytes, as an allocation does
+    void add(T **dst, const std::vector<double> &src) {
+        at.emplace_back(dst, data.size());
+        data.insert(data.end(), src.begin(), src.end());
+        constexpr size_t kAlign = 256 / sizeof(T);
+        data.resize((data.size() + kAlign - 1) / kAlign * kAlign);
+    }
+    saras_status send(T **base) {
+        HIP_TRY(hipMalloc((void **)base, std::max<size_t>(1, data.size()) * sizeof(T)));
+        HIP_TRY(hipMemcpy(*base, data.data(), data.size() * sizeof(T), hipMemcpyHostToDevice));
+        for (auto &p : at) *p.first = *base + p.second;
+        return SARAS_OK;
+    }
+};
 
 template <typename T>
 struct Hierarchy {
     int dim = 3;
     std::vector<DevLevel<T>> lv;
+    T *image = nullptr;   // the levels' constant arrays and `wall`
     T *wall[3] = {nullptr, nullptr, nullptr};   // DIRICHLET_TEST level-0 wall values
     T *coarse_scratch = nullptr;
     bool coarse_lds = true;
@@ -97,9 +112,7 @@ struct Hierarchy {
     int tail_first = -1;
     saras::TailArgs<T> tail_args{};
     size_t tail_bytes = 0;
-    T *tail_coef = nullptr;
-    unsigned *tail_cells = nullptr;
-    T *tail_b = nullptr;   // see TailArgs::bcol
+    unsigned *tail_image = nullptr;
 
     // a level takes split rows when each half-row is a whole number of 16-byte vectors
     static bool splittable(int nz) {
@@ -110,23 +123,17 @@ struct Hierarchy {
     ~Hierarchy() {
         for (auto &L : lv) {
             (void)hipFree(L.x); (void)hipFree(L.b); (void)hipFree(L.xalt);
-            (void)hipFree(L.c2zs); (void)hipFree(L.c1zs);
-            for (int a = 0; a < 3; ++a) {
-                (void)hipFree(L.c2[a]); (void)hipFree(L.c1[a]);
-                (void)hipFree(L.rlo[a]); (void)hipFree(L.rhi[a]); (void)hipFree(L.rwd[a]);
-            }
         }
-        for (int a = 0; a < 3; ++a) (void)hipFree(wall[a]);
+        (void)hipFree(image);
         (void)hipFree(coarse_scratch);
-        (void)hipFree(tail_coef);
-        (void)hipFree(tail_cells);
-        (void)hipFree(tail_b);
+        (void)hipFree(tail_image);
     }
 
     saras_status build(const saras::GridLevels &G, const std::vector<std::vector<double>> &walls) {
         dim = G.dim;
         const int D = G.depth;
         lv.resize(D + 1);
+        ConstImage<T> img;
         hc2.assign(D + 1, {});
         hc1.assign(D + 1, {});
         hlo.assign(D + 1, {});
@@ -152,7 +159,8 @@ struct Hierarchy {
             for (int a = 0; a < 3; ++a) {
                 if (dim == 2 && a == 1) {
                     std::vector<double> z(1, 0.0);
-                    if (upload(&L.c2[a], z) || upload(&L.c1[a], z)) return SARAS_HIP_ERROR;
+                    img.add(&L.c2[a], z);
+                    img.add(&L.c1[a], z);
                     hc2[l][a] = z;
                     hc1[l][a] = z;
                     continue;
@@ -170,7 +178,8 @@ struct Hierarchy {
                     c1[i] = A.xixx[i + 1] * i2h;
                 }
                 for (int i = 1; i < A.n; ++i) L.uniform = L.uniform && c2[i] == c2[0] && c1[i] == c1[0];
-                if (upload(&L.c2[a], c2) || upload(&L.c1[a], c1)) return SARAS_HIP_ERROR;
+                img.add(&L.c2[a], c2);
+                img.add(&L.c1[a], c1);
                 hc2[l][a] = c2;
                 hc1[l][a] = c1;
                 if (a == 2 && L.hz) {
@@ -181,7 +190,8 @@ struct Hierarchy {
                             c2s[hh * half + mm] = c2[2 * mm + hh];
                             c1s[hh * half + mm] = c1[2 * mm + hh];
                         }
-                    if (upload(&L.c2zs, c2s) || upload(&L.c1zs, c1s)) return SARAS_HIP_ERROR;
+                    img.add(&L.c2zs, c2s);
+                    img.add(&L.c1zs, c1s);
                 }
                 if (l > 0) {
                     // restriction factors of coarse index I (poisson_d3.cc:494-502)
@@ -194,8 +204,9 @@ struct Hierarchy {
                         hi[I] = f1 - X;
                         wd[I] = f1 - f0;
                     }
-                    if (upload(&L.rlo[a], lo) || upload(&L.rhi[a], hi) || upload(&L.rwd[a], wd))
-                        return SARAS_HIP_ERROR;
+                    img.add(&L.rlo[a], lo);
+                    img.add(&L.rhi[a], hi);
+                    img.add(&L.rwd[a], wd);
                     hlo[l][a] = lo;
                     hhi[l][a] = hi;
                     hwd[l][a] = wd;
@@ -203,7 +214,9 @@ struct Hierarchy {
             }
         }
         for (int a = 0; a < 3; ++a)
-            if (!walls[a].empty() && upload(&wall[a], walls[a])) return SARAS_HIP_ERROR;
+            if (!walls[a].empty()) img.add(&wall[a], walls[a]);
+        saras_status st = img.send(&image);
+        if (st) return st;
         // coarsest-level workspace
         const DevLevel<T> &C = lv[D];
         const size_t padded = dim == 3 ? (size_t)(C.n[0] + 2) * (C.n[1] + 2) * (C.n[2] + 2)
@@ -445,8 +458,6 @@ saras_status pack_tail(const saras_mg *m, Hierarchy<T> &H) {
         set_error("internal error: tail coefficients do not match their layout");
         return SARAS_HIP_ERROR;
     }
-    saras_status st = upload(&H.tail_coef, flat);
-    if (st) return st;
     // the LDS image of the cell tables, then the tables of larger levels
     std::vector<unsigned> img((size_t)A.ncellw, 0u);
     size_t gn = 0;   // entries of the tables in global memory
@@ -478,16 +489,21 @@ saras_status pack_tail(const saras_mg *m, Hierarchy<T> &H) {
             w1[q] = t[q].czf;
         }
     }
-    HIP_TRY(hipMalloc((void **)&H.tail_cells, std::max<size_t>(4, img.size()) * sizeof(unsigned)));
-    HIP_TRY(hipMemcpy(H.tail_cells, img.data(), img.size() * sizeof(unsigned), hipMemcpyHostToDevice));
-    if (A.L[0].b < 0) {
-        HIP_TRY(hipMalloc((void **)&H.tail_b, 2 * (size_t)A.L[0].half * sizeof(T)));
-        A.bcol = H.tail_b;
-    }
-    A.coef = H.tail_coef;
-    A.cellimg = H.tail_cells;
-    A.cells4 = reinterpret_cast<const uint4 *>(H.tail_cells + nimg);
-    A.cells1 = H.tail_cells + nimg + 4 * gn;
+    // one allocation: the cell tables, the coefficients (each at a multiple of 256
+    // bytes) and the right-hand side by colour where LDS has no room for it
+    const size_t cells = (img.size() + 63) / 64 * 64, words = sizeof(T) / 4;
+    const std::vector<T> coef(flat.begin(), flat.end());
+    const size_t ncoef = (coef.size() * words + 63) / 64 * 64;
+    img.resize(cells + ncoef, 0u);
+    std::memcpy(img.data() + cells, coef.data(), coef.size() * sizeof(T));
+    const size_t nb = A.L[0].b < 0 ? 2 * (size_t)A.L[0].half * words : 0;
+    HIP_TRY(hipMalloc((void **)&H.tail_image, (img.size() + nb) * sizeof(unsigned)));
+    HIP_TRY(hipMemcpy(H.tail_image, img.data(), img.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+    A.coef = reinterpret_cast<const T *>(H.tail_image + cells);
+    if (nb) A.bcol = reinterpret_cast<T *>(H.tail_image + cells + ncoef);
+    A.cellimg = H.tail_image;
+    A.cells4 = reinterpret_cast<const uint4 *>(H.tail_image + nimg);
+    A.cells1 = H.tail_image + nimg + 4 * gn;
     return SARAS_OK;
 }
 
