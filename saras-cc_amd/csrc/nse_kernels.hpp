@@ -1053,16 +1053,24 @@ k_sgs_stress(Geom G, double nu, SgsMarch A) {
                     // the 13 offsets before (0, 0, 0) in (di, dj, dk) order
 #pragma unroll
                     for (int t = 0; t < 13; ++t) Qd += 2.0 * term(sx[t / 9], sy[(t / 3) % 3], sz[t % 3], std::true_type{});
-                } else {
-                    const int nt = mirror ? 13 : 27;
+                } else if (shorts) {
+                    // stretched axes: a plane of nine at a time (384^3 5.26 ms a call; one
+                    // offset at a time, with the forms chosen in the loop, 6.79)
 #pragma unroll 1
-                    for (int t = 0; t < nt; ++t) {
+                    for (int a = 0; a < 3; ++a) {
+                        const float dx = a == 0 ? sx[0] : a == 1 ? 0.0f : sx[2];
+#pragma unroll
+                        for (int t = 0; t < 9; ++t)
+                            if (a != 1 || t != 4) Qd += term(dx, sy[t / 3], sz[t % 3], std::true_type{});
+                    }
+                } else {
+#pragma unroll 1
+                    for (int t = 0; t < (mirror ? 13 : 27); ++t) {
                         const int a = t / 9, b = (t / 3) % 3, c = t % 3;
-                        if (t == 13) continue;
-                        const float dx = a == 0 ? sx[0] : a == 1 ? 0.0f : sx[2], dy = b == 0 ? sy[0] : b == 1 ? 0.0f : sy[2];
-                        const float dz = c == 0 ? sz[0] : c == 1 ? 0.0f : sz[2];
-                        const double v = shorts ? term(dx, dy, dz, std::true_type{}) : term(dx, dy, dz, std::false_type{});
-                        Qd += mirror ? 2.0 * v : v;
+                        if (t != 13)
+                            Qd += (mirror ? 2.0 : 1.0) * term(a == 0 ? sx[0] : a == 1 ? 0.0f : sx[2],
+                                                              b == 0 ? sy[0] : b == 1 ? 0.0f : sy[2],
+                                                              c == 0 ? sz[0] : c == 1 ? 0.0f : sz[2], std::false_type{});
                     }
                 }
             } else {

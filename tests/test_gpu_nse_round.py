@@ -95,14 +95,16 @@ def test_by6(lib):
     assert np.abs(out.view(np.int64) - (a / 6.0).view(np.int64)).max() <= 1
 
 
+@pytest.mark.parametrize("tanh", [False, True], ids=["uniform", "tanh"])
 @pytest.mark.parametrize("width", [2e-16, 1e-13, 1e-3], ids=["2e-16", "1e-13", "1e-3"])
-def test_stresses_of_narrow_cells(width):
-    """The velocities shrink with the cells, so that the strain rates stay."""
+def test_stresses_of_narrow_cells(width, tanh):
+    """The velocities shrink with the cells, so that the strain rates stay.  On
+    stretched axes all 26 neighbour offsets are evaluated."""
     n = (8, 6, 72)
     length = tuple(width * m for m in n)
     kw = dict(has_T=0, nu=1.0 / 1600 * width ** 2, dt=1e-3, cn_tol=1e-10, les=1)
     mg = mg_kw(vc_count=2, vc_tol=1e-10, pre=2, post=2)
-    geo = dict(periodic=(1, 1, 1), gtype=(0, 0, 0), length=length, pad=2)
+    geo = dict(periodic=(1, 1, 1), gtype=(2, 2, 2) if tanh else (0, 0, 0), beta=(0.8, 0.7, 0.9), length=length, pad=2)
     so = O.Nse(O.nse_desc(O.grid_desc(n, **geo), mg=O.mg_params(bc=O.BC_NEUMANN, **mg), **kw))
     ss = S.Nse(S.grid_desc(n, **geo), S.mg_params(bc=S.BC_NEUMANN, precision=S.PREC_FP64, **mg),
                S.nse_params(**kw, les_sf32=1))
