@@ -180,8 +180,8 @@ saras_status plume_flags(saras_nse *s);
 // The stresses and per-block diagnostics of every core cell (les_sf32: the
 // structure-function integral in single precision); the number of blocks.
 // At 384^3 a call took 5.65 ms cell by cell and takes 4.19 (single-precision
-// integral): 2150 instead of 3540 instructions a cell, 86 % of the cycles; its
-// stores alone are 2.7 GB, 0.6 ms at the copy rate.
+// integral): 2150 instead of 3540 instructions a cell, 89 % of the cycles; its
+// stores alone are 2.7 GB, 0.44 ms at the copy kernel's 6.2 TB/s.
 unsigned launch_sgs(saras_nse *s) {
     using namespace saras::nse;
     SgsMarch A{};
@@ -242,7 +242,7 @@ saras_status rhs_euler(saras_nse *s) {
 
 // The explicit part of every field in one marching pass.  Per stage, the kernels
 // per field / this: 256^3 with T 2.0 / 0.84 ms, 384^3 with the stresses 5.7 /
-// 3.1 ms (its bytes, 152 a cell, take 1.8 ms at the copy rate).
+// 3.1 ms (its bytes, 152 a cell, take 1.4 ms at 6.2 TB/s).
 void launch_rhs_march(saras_nse *s, const saras::nse::StageCoef &c, int les) {
     using namespace saras::nse;
     RhsMarch A{};
@@ -348,7 +348,7 @@ void launch_div(saras_nse *s, double sc, double *b, long bsx, long bsy, long bhz
 }
 
 // The pressure correction.  k_correct / k_correct_march: 64^3 10.2 / 9.2 us, 160^3
-// 84 / 79, 256^3 318 / 279, 384^3 1078 / 940 (850 at the copy rate).
+// 84 / 79, 256^3 318 / 279, 384^3 1078 / 940 (660 at 6.2 TB/s).
 void launch_correct(saras_nse *s, double pc) {
     using namespace saras::nse;
     const SplitField pp = s->pp();
@@ -367,7 +367,7 @@ void launch_correct(saras_nse *s, double pc) {
 // One Jacobi iteration of field f from `in` to `out`; with `res`, the partial
 // maxima of the input's residual in s->part.  Returns their number.  An iteration
 // with its maximum by k_jacobi / k_jacobi_march: 256^3 154 / 122 us, 384^3 486 /
-// 393 us (84 and 283 at the copy rate).
+// 393 us (65 and 219 at 6.2 TB/s).
 long launch_jacobi(saras_nse *s, int f, const double *in, double *out, double diff, double beta, bool res) {
     using namespace saras::nse;
     const double dt = s->p.dt;
@@ -881,8 +881,9 @@ saras_status saras_nse_create(const saras_grid_desc *grid, const saras_mg_params
         const char *env = std::getenv("SARAS_NO_NSE_MARCH");
         // dScheme 2 with Morinishi's term in boxes periodic in x and y, whose z
         // walls are none or plain Dirichlet / Neumann ones (no stored ghosts, no
-        // column flags, the z edge test at the last cell); every other form
-        // takes the kernels per field
+        // column flags) with ny == nz: elsewhere the edge test on z, which
+        // compares with ny, reads the second stored layer (top2) at the last
+        // cell.  Every other form takes the kernels per field
         bool ok = !planar && P.scheme == 0 && P.dscheme == 2 && P.nlscheme == 3 && g.periodic[0] && g.periodic[1] &&
                   s->elems * sizeof(double) <= 0xffffffffull && !(env && env[0] == '1');
         for (int q = 0; q < 5; ++q) {
